@@ -18,9 +18,8 @@ __host__ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
 __host__ __device__ __forceinline__ uint64_t stream_key(uint64_t seed, uint64_t stream) {
   return mix64(seed ^ mix64(stream));
 }
-__host__ __device__ __forceinline__ uint64_t rand_word(uint64_t key, uint64_t i) {
-  return mix64(key + i * 0xD1342543DE82EF95ull);
-}
+constexpr uint64_t kRandStep = 0xD1342543DE82EF95ull;
+__host__ __device__ __forceinline__ uint64_t rand_word(uint64_t key, uint64_t i) { return mix64(key + i * kRandStep); }
 
 constexpr uint64_t kStreamRmat = 0x524D4154ull;  // "RMAT"
 constexpr uint64_t kStreamEr = 0x45524E59ull;    // "ERNY"
