@@ -59,13 +59,37 @@ __global__ void k_vertex_gid(const uint32_t* __restrict__ labels, uint64_t n, co
   gid[v] = first + segment_of(voff, count, old);
 }
 
-// Edges of every graph: each oriented row adds its length to its graph.
-__global__ void k_graph_edges(const uint32_t* __restrict__ row_ptr, uint64_t n, const uint32_t* __restrict__ gid,
-                              unsigned long long* __restrict__ m) {
-  const uint64_t u = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (u >= n) return;
-  const uint32_t d = row_ptr[u + 1] - row_ptr[u];
-  if (d) atomicAdd(&m[gid[u]], (unsigned long long)d);
+// Edges of every graph: each oriented row adds its length to its graph. The
+// rows of a part are in degree order, so neighbouring rows belong to any of its
+// graphs and one atomic per row on the graphs' counters serialised on a few
+// hundred addresses (768 graphs, 36M rows: 15.6 ms; 96 graphs, 1.3M rows: 2.84
+// ms). Each block sums the part's graphs in LDS and adds its sums once (the 96
+// graphs: 0.014 ms); parts of more than kEdgeGraphs graphs spread over
+// so many addresses that the direct atomics stay.
+constexpr uint32_t kEdgeGraphs = 8192;  // 32-bit LDS counters (a part has fewer than 2^32 edges)
+constexpr unsigned kEdgeBlocks = 512;
+__global__ void __launch_bounds__(512) k_graph_edges(const uint32_t* __restrict__ row_ptr, uint64_t n,
+                                                     const uint32_t* __restrict__ gid, uint32_t first, uint32_t count,
+                                                     unsigned long long* __restrict__ m) {
+  extern __shared__ uint32_t s_m[];
+  const bool lds = count <= kEdgeGraphs;
+  if (lds) {
+    for (uint32_t i = threadIdx.x; i < count; i += blockDim.x) s_m[i] = 0u;
+    __syncthreads();
+  }
+  for (uint64_t u = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; u < n; u += (uint64_t)gridDim.x * blockDim.x) {
+    const uint32_t d = row_ptr[u + 1] - row_ptr[u];
+    if (!d) continue;
+    if (lds)
+      atomicAdd(&s_m[gid[u] - first], d);
+    else
+      atomicAdd(&m[gid[u]], (unsigned long long)d);
+  }
+  if (lds) {
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < count; i += blockDim.x)
+      if (s_m[i]) atomicAdd(&m[first + i], (unsigned long long)s_m[i]);
+  }
 }
 
 __global__ void k_zero_words(unsigned long long* p, uint64_t n) {
@@ -130,7 +154,8 @@ void build_part(tribit_ctx* ctx, tribit_batch* b, uint32_t first, uint32_t count
     k_vertex_gid<<<grid_for(n, 256), 256, 0, s>>>(part.g->labels, n, voff.p, count, first, gid.p);
     DevBuf<unsigned long long> m(ctx, b->ngraphs);
     k_zero_words<<<grid_for(b->ngraphs, 256), 256, 0, s>>>(m.p, b->ngraphs);
-    k_graph_edges<<<grid_for(n, 256), 256, 0, s>>>(part.g->row_ptr, n, gid.p, m.p);
+    k_graph_edges<<<std::min(kEdgeBlocks, grid_for(n, 512)), 512, count <= kEdgeGraphs ? 4 * count : 0, s>>>(
+        part.g->row_ptr, n, gid.p, first, count, m.p);
     std::vector<unsigned long long> mh(b->ngraphs);
     TB_HIP(hipMemcpyAsync(mh.data(), m.p, 8 * b->ngraphs, hipMemcpyDeviceToHost, s));
     ctx->sync();
