@@ -2123,17 +2123,6 @@ void make_schedule(tribit_ctx* ctx, tribit_graph* g, int layout, int flags, bool
     if ((flags & TRIBIT_COUNT_FORCE_TILES) && plan.kind[i] == kKindBlock) plan.kind[i] = kKindTile;
     if (((flags & TRIBIT_COUNT_NO_TILES) || S.blocks) && plan.kind[i] == kKindTile) plan.kind[i] = kKindBlock;
   }
-  bool any_tiles = false;
-  for (int i = 0; i < plan.nslots; ++i) any_tiles |= plan.kind[i] == kKindTile;
-  if (any_tiles && g->m) {
-    const int width = (flags & TRIBIT_COUNT_TILES32) ? 32 : 64;
-    build_tiles(ctx, g, layout, width);  // once per graph, width and layout
-    const tribit_graph::TileSet& T = g->tiles[width == 32 ? 0 : 1];
-    S.ts.blk = T.blk;
-    S.ts.mask = width == 64 ? reinterpret_cast<const unsigned long long*>(T.mask) : nullptr;
-    S.ts.mask32 = width == 32 ? reinterpret_cast<const uint32_t*>(T.mask) : nullptr;
-    S.ts.trng = T.trng[layout & 3];
-  }
   DevBuf<uint8_t> dtable_own;
   uint8_t* dtable = scratch_buf(ctx, arena, dtable_own, kBuckets);
   {
@@ -2177,6 +2166,21 @@ void make_schedule(tribit_ctx* ctx, tribit_graph* g, int layout, int flags, bool
     S.tasks = DevBuf<uint4>(ctx, S.ntask ? S.ntask : 1);
   if (nb) k_sched_fill<<<(unsigned)nb, kSchedBlock, 0, s>>>(sv, pd, n, off, S.base, S.tasks.p);
   TB_HIP(hipGetLastError());
+  // bit tiles only for a launch that streams them: the menu always has a tile
+  // slot, but the heuristic and most learned tables send it no task, and
+  // building the tiles for it cost more than the whole count (R-MAT scale 25:
+  // 49 ms of the first count's 98)
+  bool any_tiles = false;
+  for (int i = 0; i < plan.nslots; ++i) any_tiles |= plan.kind[i] == kKindTile && S.tot.v[i];
+  if (any_tiles) {
+    const int width = (flags & TRIBIT_COUNT_TILES32) ? 32 : 64;
+    build_tiles(ctx, g, layout, width);  // once per graph, width and layout
+    const tribit_graph::TileSet& T = g->tiles[width == 32 ? 0 : 1];
+    S.ts.blk = T.blk;
+    S.ts.mask = width == 64 ? reinterpret_cast<const unsigned long long*>(T.mask) : nullptr;
+    S.ts.mask32 = width == 32 ? reinterpret_cast<const uint32_t*>(T.mask) : nullptr;
+    S.ts.trng = T.trng[layout & 3];
+  }
   // every plan but the textbook one: a one-task wave-64 launch with thousands
   // of tasks per CU runs as multi-task waves (same tasks, eight per wave at
   // once); with fewer, the one-task kernel was faster (R-MAT s25: 1.40 -> 1.03
@@ -2809,7 +2813,7 @@ static double batch_capture(tribit_ctx* ctx, tribit_batch* b, int att, uint32_t*
     for (int k = 0; k < S.plan.nslots; ++k) {
       const bool blockish = S.kdef[k] == kKindBlock || S.kdef[k] == kKindTile;
       S.plan.kind[k] = (tw && blockish) ? kKindTile : S.kdef[k];
-      tiles |= S.plan.kind[k] == kKindTile;
+      tiles |= S.plan.kind[k] == kKindTile && S.tot.v[k];
     }
     if (tiles && p.g->m) {
       const int width = tw ? tw : (b->flags & TRIBIT_COUNT_TILES32) ? 32 : 64;

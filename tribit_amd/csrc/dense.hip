@@ -46,7 +46,8 @@ __global__ void k_core_zero(uint4* __restrict__ p, uint64_t n16) {
 // window is then written whole, so the matrix is stored once, coalesced, with
 // no zeroing pass (bound: the kp^2 / 8 bytes written). A thread per row, setting
 // its bits in memory one dependent read-modify-write at a time, took 1.84 ms for
-// the 24,576-id core of R-MAT scale 25; this takes 0.072 ms. Rows of up to 65,536 columns, the largest core the schedule picks, are one window.
+// the 24,576-id core of R-MAT scale 25; this takes 0.072 ms. Rows of up to
+// 65,536 columns, the largest core the schedule picks, are one window.
 constexpr uint32_t kCoreWin = 65536;  // columns per LDS window: 8 KiB a wave, 5 blocks of 4 waves per CU
 __global__ void __launch_bounds__(256) k_core_bits(const uint32_t* __restrict__ row_ptr,
                                                    const uint32_t* __restrict__ col, uint64_t n, uint64_t d0,
