@@ -159,9 +159,11 @@ typedef struct {
 } tribit_variant_work;
 
 /* ---- context ------------------------------------------------------------ */
-/* Selects `device`, creates a stream and sets the default memory pool to keep
- * freed memory (release threshold = max), as init_gpu_kernel5
- * (main5_multi.cu:578-587) and allocate_memory (tribit.cu:825-838) do. */
+/* Selects `device` and creates a stream and a device memory pool that keeps
+ * freed memory for later calls, as init_gpu_kernel5 (main5_multi.cu:578-587) and
+ * allocate_memory (tribit.cu:825-838) do. The pool is the context's own: at most
+ * a quarter of the device's memory stays in it unused, and tribit_shutdown gives
+ * all of it back, so free the context's graphs, batches and models first. */
 int tribit_init(int device, tribit_ctx** out);
 int tribit_shutdown(tribit_ctx* ctx);
 /* Test hook: fail device allocations beyond `bytes` in total (0 = no cap). */
@@ -176,7 +178,7 @@ int tribit_set_alloc_cap(tribit_ctx* ctx, uint64_t bytes);
                                 same either way. */
 #define TRIBIT_OPT_BATCH_PART_KEYS 2 /* input keys per batch part (default 2^30) */
 int tribit_set_option(tribit_ctx* ctx, int option, int64_t value);
-/* Peak bytes held from the memory pool since tribit_init. */
+/* Peak bytes in use from the context's memory pool since tribit_init. */
 int tribit_pool_peak(tribit_ctx* ctx, uint64_t* bytes);
 const char* tribit_status_str(int status);
 /* Build description: library version, rocPRIM and HIP versions, target. */

@@ -86,9 +86,7 @@ int tribit_init(int device, tribit_ctx** out) {
       snprintf(dname, sizeof(dname), "%s", prop.name);
     snprintf(ctx->name, sizeof(ctx->name), "%s (%s, %d CUs)", dname, prop.gcnArchName, prop.multiProcessorCount);
     TB_HIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
-    TB_HIP(hipDeviceGetDefaultMemPool(&ctx->pool, device));
-    uint64_t thr = UINT64_MAX;  // keep freed blocks in the pool (tribit.cu:829-830)
-    TB_HIP(hipMemPoolSetAttribute(ctx->pool, hipMemPoolAttrReleaseThreshold, &thr));
+    ctx->pool.init(ctx->stream, prop.totalGlobalMem / 4);  // freed memory stays with the context (tribit.cu:829-830)
     for (auto& e : ctx->ev) TB_HIP(hipEventCreate(&e));
     tb::noalloc_init(ctx);  // the device is current: its copy of the scratch array
   });
@@ -103,6 +101,8 @@ int tribit_init(int device, tribit_ctx** out) {
 int tribit_shutdown(tribit_ctx* ctx) {
   if (!ctx) return TRIBIT_ERR_ARG;
   (void)hipSetDevice(ctx->device);
+  (void)hipStreamSynchronize(ctx->stream);
+  ctx->pool.release();
   (void)hipStreamSynchronize(ctx->stream);
   for (auto& e : ctx->ev)
     if (e) (void)hipEventDestroy(e);

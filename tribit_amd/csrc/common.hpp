@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "../../include/tribit.h"
+#include "pool.hpp"
 
 namespace tb {
 
@@ -47,12 +48,12 @@ inline unsigned grid_for(uint64_t items, unsigned block) {
 
 }  // namespace tb
 
-// Per-device context: one stream, stream-ordered pool allocations with
-// byte accounting (cap for tests, peak for reporting), timing events.
+// Per-device context: one stream, its own device memory pool with byte
+// accounting (cap for tests, peak for reporting), timing events.
 struct tribit_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
-  hipMemPool_t pool = nullptr;
+  tb::DevicePool pool;
   int cus = 0;
   int lds_per_block = 0;
   char name[256] = {0};
@@ -85,12 +86,8 @@ struct tribit_ctx {
     if (bytes == 0) bytes = 8;
     bytes = (bytes + 255) & ~uint64_t(255);
     if (cap && held + bytes > cap) tb::fail(TRIBIT_ERR_NOMEM, "allocation exceeds the configured cap");
-    void* p = nullptr;
-    hipError_t e = hipMallocAsync(&p, bytes, stream);
-    if (e != hipSuccess || !p) {
-      (void)hipGetLastError();
-      tb::fail(TRIBIT_ERR_NOMEM, std::string("hipMallocAsync: ") + hipGetErrorString(e));
-    }
+    void* p = pool.alloc(bytes);
+    if (!p) tb::fail(TRIBIT_ERR_NOMEM, "no device memory for " + std::to_string(bytes) + " bytes");
     sizes[p] = bytes;
     held += bytes;
     if (held > peak) peak = held;
@@ -107,7 +104,7 @@ struct tribit_ctx {
       held -= it->second;
       sizes.erase(it);
     }
-    (void)hipFreeAsync(p, stream);
+    pool.free(p);
   }
   void sync() { TB_HIP(hipStreamSynchronize(stream)); }
 };
