@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 
 import tribit_amd
+from tests.test_gpu_parity import assert_same_structure
 
 pytestmark = pytest.mark.gpu
 
@@ -45,3 +46,46 @@ def test_batch_edge_counts(gpu_ctx, oracle_mod, graphs):
         assert [int(x) for x in m] == [len(set(k.tolist())) for k in keys]
         c, _ = b.count()
         assert [int(x) for x in c] == [oracle_mod.count_keys(k, int(v)) for k, v in zip(keys, ns)]
+
+
+# (vertices, keys): one bucket, the first two buckets, the widest single pass, the first two-pass partition with
+# 64-bit items, 32-bit items and items of exactly 32 bits
+@pytest.mark.parametrize("n,nk", [(5, 1), (5000, 2048), (5000, 2049), (70000, 1 << 20), (1 << 26, (1 << 20) + 1),
+                                  (100000, (1 << 20) + 1), (1 << 21, 1500001)])
+def test_distinct_keys_partition(gpu_ctx, oracle_mod, n, nk):
+    """Sentinels and repeated keys among the input; every structure equals the oracle's."""
+    note(f"partition of {nk} keys over {n} ids")
+    rng = np.random.default_rng(nk)
+    a, b = rng.integers(0, n, (2, nk))
+    k = ((np.minimum(a, b) << 32) | np.maximum(a, b)).astype(np.uint64)
+    k[a == b] = oracle_mod.SENTINEL
+    k[rng.integers(0, nk, nk // 5)] = k[rng.integers(0, nk, nk // 5)]
+    with gpu_ctx.graph_from_keys(k, n) as g:
+        assert_same_structure(g, k, n, oracle_mod)
+
+
+def test_distinct_keys_repeated(gpu_ctx, oracle_mod):
+    """Keys repeated thousands of times overflow their bucket: the sort takes over."""
+    note("500 keys, 2M times")
+    rng = np.random.default_rng(5)
+    keys = oracle_mod.gen_er(3000, 500, seed=2)
+    k = keys[rng.integers(0, keys.size, 2_000_000)]
+    with gpu_ctx.graph_from_keys(k, 3000) as g:
+        assert_same_structure(g, k, 3000, oracle_mod)
+
+
+@pytest.mark.parametrize("n,nk", [(65536, 300000), (65537, 300000), (3 * 65536 + 32769, 3000000),
+                                  ((1 << 27) + 70001, 300000)])
+def test_degrees_by_id_range(gpu_ctx, n, nk):
+    """Degrees around the ends of an id group and half group, of one group's counting tasks (a hub group), and past
+    the ids of one pass."""
+    note(f"degrees over {n} ids")
+    rng = np.random.default_rng(n)
+    a = rng.integers(0, n, nk)
+    b = np.where(rng.random(nk) < 0.7, rng.integers(0, min(n, 30000), nk), n - 1 - rng.integers(0, 7, nk))
+    k = np.unique(((np.minimum(a, b) << 32) | np.maximum(a, b))[a != b].astype(np.uint64))
+    want = np.bincount((k >> np.uint64(32)).astype(np.int64), minlength=n)
+    want += np.bincount((k & np.uint64(0xFFFFFFFF)).astype(np.int64), minlength=n)
+    with gpu_ctx.graph_from_keys(k, n) as g:
+        labels, _ = g.labels()
+        assert np.array_equal(g.download()[2], want[labels].astype(np.uint32))

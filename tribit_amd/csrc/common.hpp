@@ -289,6 +289,10 @@ void gen_rmat(tribit_ctx* ctx, uint32_t scale, uint32_t ef, double a, double b, 
               uint64_t* d_keys);
 void gen_er(tribit_ctx* ctx, uint64_t n, uint64_t nsamples, uint64_t seed, uint64_t* d_keys);
 void rmat_thresholds(double a, double b, double c, uint32_t t[3]);
+// partition.hip
+bool distinct_keys(tribit_ctx* ctx, const uint64_t* d_keys, uint64_t nk, uint64_t n, uint32_t kb, uint64_t* out,
+                   uint64_t* m, bool* bad, uint64_t band_ids, uint64_t* band);
+void count_degrees(tribit_ctx* ctx, const uint64_t* keys, uint64_t m, uint64_t n, uint32_t kb, uint32_t* deg);
 // gen.hip
 uint64_t chung_lu_samples(uint64_t n, double avg_deg);
 void chung_lu_cdf(uint64_t n, double gamma, uint64_t* cdf);

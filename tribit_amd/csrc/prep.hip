@@ -4,8 +4,8 @@
 // Replaces the reference's preprocessing chain, src/single_gpu/tribit.cu:
 // 664-763 (radix sort + unique of packed keys, L/U bit structures, singleton
 // purge, warp schedule). The product here is a degree-oriented CSR instead:
-//   keys (min<<32|max) --sort--> --unique--> m undirected edges
-//   deg[v] (wave-aggregated atomics)
+//   keys (min<<32|max) --partition, LDS hash sets--> m undirected edges
+//   deg[v] (endpoints by id range, counted in LDS)
 //   orient {a<b}: a->b iff deg(a) <= deg(b)       (rank = (deg, id))
 //   --sort--> row_ptr[n+1] (u32), col[m] (u32, ascending within a row)
 //   W+ = sum over v of indeg(v) * outdeg(v); wedge ranges (relabelled graphs)
@@ -141,31 +141,6 @@ __global__ void k_scatter_heads(const uint64_t* __restrict__ k, uint64_t nk, con
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nk) return;
   if (pos[i + 1] != pos[i]) out[pos[i]] = k[i];
-}
-
-// Degrees of the sorted unique keys. Consecutive keys repeat their smaller
-// endpoint, so a wave adds each run of it with one atomic; the larger
-// endpoints are written to `hi`, sorted, and added the same way by
-// k_add_runs (one atomic per key took 37 ms for the 523M keys of R-MAT
-// scale 25).
-__global__ void k_degree_lo(const uint64_t* __restrict__ keys, uint64_t m, uint32_t kb, uint32_t* __restrict__ deg,
-                            uint32_t* __restrict__ hi) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool valid = i < m;
-  const uint64_t k = valid ? keys[i] : 0;
-  const uint32_t a = valid ? (uint32_t)(k >> kb) : 0xFFFFFFFFu;
-  if (valid) hi[i] = (uint32_t)(k & ((1ull << kb) - 1));
-  const uint32_t run = wave_run_length(a, valid);
-  if (run) atomicAdd(&deg[a], run);
-}
-
-// deg[v] += the number of v in the sorted ids[0, m), one atomic per run per wave.
-__global__ void k_add_runs(const uint32_t* __restrict__ ids, uint64_t m, uint32_t* __restrict__ deg) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool valid = i < m;
-  const uint32_t a = valid ? ids[i] : 0xFFFFFFFFu;
-  const uint32_t run = wave_run_length(a, valid);
-  if (run) atomicAdd(&deg[a], run);
 }
 
 // Oriented arcs u -> v are sorted as packed keys (u << kb) | v with kb =
@@ -618,11 +593,10 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
 
   // keys checked and packed to (min << kb) | max for the sort
   const uint32_t kb = bits_for(n);
-  DevBuf<uint32_t> flag(ctx, 4);
-  k_fill_u32<<<1, 64, 0, s>>>(flag.p, 4, 0u);
-  if (nkeys) k_validate_pack<<<grid_for(nkeys, kBlock), kBlock, 0, s>>>(keys.p, nkeys, n, kb, flag.p);
 
-  // 1-2. sort + unique (tribit.cu:666-667). The sentinel sorts last.
+  // 1-2. distinct keys (tribit.cu:666-667): by partition, in any order; the
+  // sort, after which the sentinel comes last, is for keys repeated so often
+  // that a bucket of the partition overflows and for more than 2^32 - 2 keys.
   const uint32_t end_bit = 2 * kb;
   uint64_t m = 0;
   // id-band edges for the automatic choice of ids (TRIBIT_OPT_RELABEL 3)
@@ -631,7 +605,22 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
   DevBuf<unsigned long long> band;
   band.ctx = ctx;
   DevBuf<uint64_t> uniq(ctx, nkeys ? nkeys : 1);
-  if (nkeys) {
+  bool bad_key = false, distinct = false;
+  if (nkeys && nkeys <= 0xFFFFFFFEull) {
+    try {
+      distinct = distinct_keys(ctx, keys.p, nkeys, n, kb, uniq.p, &m, &bad_key, kBandIds,
+                               want_band ? &band_edges : nullptr);
+    } catch (const Error& e) {  // the partition's regions take more room than the sort's
+      if (e.status != TRIBIT_ERR_NOMEM) throw;
+    }
+  }
+  if (distinct) {
+    keys.reset();
+    if (bad_key) fail(TRIBIT_ERR_RANGE, "edge key is not (min < max < n)");
+  } else if (nkeys) {
+    DevBuf<uint32_t> flag(ctx, 4);
+    k_fill_u32<<<1, 64, 0, s>>>(flag.p, 4, 0u);
+    k_validate_pack<<<grid_for(nkeys, kBlock), kBlock, 0, s>>>(keys.p, nkeys, n, kb, flag.p);
     DevBuf<uint64_t> sorted(ctx, nkeys);
     sort_keys(ctx, keys.p, sorted.p, nkeys, end_bit);
     keys.reset();
@@ -693,15 +682,7 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
 
   // 3. degrees
   DevBuf<uint32_t> deg(ctx, n);
-  k_fill_u32<<<grid_for(n, kBlock), kBlock, 0, s>>>(deg.p, n, 0u);
-  if (m) {
-    DevBuf<uint32_t> hi(ctx, m), hi_sorted(ctx, m);
-    k_degree_lo<<<grid_for(m, kBlock), kBlock, 0, s>>>(uniq.p, m, kb, deg.p, hi.p);
-    with_temp(ctx, [&](void* t, size_t& b) {
-      return rocprim::radix_sort_keys<IdSortConfig>(t, b, hi.p, hi_sorted.p, (size_t)m, 0u, bits_for(n), s);
-    });
-    k_add_runs<<<grid_for(m, kBlock), kBlock, 0, s>>>(hi_sorted.p, m, deg.p);
-  }
+  count_degrees(ctx, uniq.p, m, n, kb, deg.p);
 
   // 3b. optional degree relabelling: internal id = rank of (deg, id) (mode 1)
   // or of (octave of deg, id) (mode 2; mode 3 picks 1 or 2 from the id-band
