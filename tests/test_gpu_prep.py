@@ -89,3 +89,30 @@ def test_degrees_by_id_range(gpu_ctx, n, nk):
     with gpu_ctx.graph_from_keys(k, n) as g:
         labels, _ = g.labels()
         assert np.array_equal(g.download()[2], want[labels].astype(np.uint32))
+
+
+def hub_graph(rng, n, hubs, leaves, extra):
+    """`hubs` top vertices joined to `leaves` random others each and to each other, plus `extra` random edges."""
+    a = [np.repeat(np.arange(hubs), leaves), rng.integers(0, n, extra), np.repeat(np.arange(hubs), hubs)]
+    b = [rng.integers(hubs, n, hubs * leaves), rng.integers(0, n, extra), np.tile(np.arange(hubs), hubs)]
+    a, b = np.concatenate(a), np.concatenate(b)
+    return np.unique(((np.minimum(a, b) << 32) | np.maximum(a, b))[a != b].astype(np.uint64))
+
+
+# a wave or less, hubs that own most ranges, hubs whose own ranges are the longest (two 64K-id windows among them)
+@pytest.mark.parametrize("n,hubs,leaves,extra", [(60, 1, 20, 100), (9000, 0, 0, 8192), (9000, 2, 4095, 30000),
+                                                 (30000, 3, 4097, 60000), (200000, 1, 150000, 20000),
+                                                 (100000, 4, 20000, 2000000), (100000, 40, 30000, 1000000),
+                                                 (400000, 3, 300000, 3500000)])
+def test_wedge_records(gpu_ctx, oracle_mod, n, hubs, leaves, extra):
+    """Wedge ranges grouped by head: counts over them with and without a core (whose cut relies on their order) and
+    from 16- and 32-bit ids (whose narrow records travel through the sort)."""
+    note(f"wedges: {n} ids, {hubs} hubs of {leaves}, {extra} others")
+    k = hub_graph(np.random.default_rng(n + hubs), n, hubs, leaves, extra)
+    want = oracle_mod.count_keys(k, n)
+    with gpu_ctx.graph_from_keys(k, n) as g:
+        assert_same_structure(g, k, n, oracle_mod)
+        for core in (0, 64, min(n, 5000)):
+            assert g.count("wedge", dense_core=core).triangles == want, core
+        assert g.count("wedge", flags=tribit_amd.WIDE_IDS).triangles == want
+        assert sum(g.variant_stats("wedge")["edges"]) <= k.size

@@ -82,4 +82,26 @@ __device__ __forceinline__ bool wave_segment_tail(uint32_t key, bool valid, uint
   return valid && (!(above & 1ull) || nk != key);
 }
 
+// As wave_segment_tail for values whose sum over a wave fits 32 bits: one
+// inclusive scan, from which a run's sum is the difference between its last lane
+// and its first (8 shuffles of 32 bits instead of 18).
+__device__ __forceinline__ bool wave_segment_tail_u32(uint32_t key, bool valid, uint32_t val, uint32_t* sum) {
+  const uint32_t lane = lane_id();
+  uint32_t inc = valid ? val : 0u;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t t = __shfl_up(inc, o);
+    if (lane >= (uint32_t)o) inc += t;
+  }
+  const uint32_t prev = __shfl_up(key, 1);
+  const uint64_t heads = __ballot(lane == 0 || prev != key), valids = __ballot(valid);
+  const uint64_t upto = heads & (~0ull >> (63 - lane));
+  const uint32_t first = 63u - (uint32_t)__clzll((long long)upto);
+  const uint32_t before = __shfl(inc - (valid ? val : 0u), (int)first);
+  *sum = inc - before;
+  const uint64_t after = lane == 63 ? 0ull : ~0ull << (lane + 1);
+  const bool next_same = ((valids & ~heads) >> ((lane + 1) & 63)) & 1ull;
+  return valid && (!(valids & after) || !next_same);
+}
+
 }  // namespace tb

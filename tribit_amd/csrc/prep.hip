@@ -10,6 +10,7 @@
 //   --sort--> row_ptr[n+1] (u32), col[m] (u32, ascending within a row)
 //   W+ = sum over v of indeg(v) * outdeg(v); wedge ranges (relabelled graphs)
 // Every launch is a 1-D grid of 256-thread blocks (4 waves).
+#include <cmath>
 #include <cstring>
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
@@ -351,8 +352,8 @@ __global__ void k_row_split(const uint32_t* __restrict__ row_ptr, const uint32_t
   split[u] = lo;
 }
 
-// Relabelled graphs, one pass over the arcs e = (u -> v) in CSR order (okeys
-// sorted, packed (u << kb) | v), every lane one arc, into arec[e]:
+// The record of arc e = (u -> v) of a relabelled graph, packed k = (u << kb) | v,
+// in CSR order:
 //   .x = row_ptr[u + 1] (the end of arc e's wedge range [e + 1, end), the part
 //        of N+(u) after v), with bits 31 / 30 of the narrow record;
 //   .y (with nar, m < 2^30) = the rest of that range's narrow record: bit 31
@@ -361,13 +362,9 @@ __global__ void k_row_split(const uint32_t* __restrict__ row_ptr, const uint32_t
 //        of the first id with H + 1 (from the row's split position); .y bits
 //        16..23 H - (v >> 16), 255 when larger. In CSR order the range's ids
 //        are the row's next ones, so the reads stay in cache.
-// One 8-byte record per arc, so the wedge-range fill gathers once per range.
-__global__ void k_arc_rec(const uint64_t* __restrict__ okeys, uint64_t m, uint32_t kb,
-                          const uint32_t* __restrict__ row_ptr, const uint32_t* __restrict__ col,
-                          const uint32_t* __restrict__ rsplit, bool nar, uint2* __restrict__ arec) {
-  const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= m) return;
-  const uint64_t k = okeys[e];
+__device__ __forceinline__ uint2 arc_record(uint64_t k, uint64_t e, uint32_t kb, const uint32_t* __restrict__ row_ptr,
+                                            const uint32_t* __restrict__ col, const uint32_t* __restrict__ rsplit,
+                                            bool nar) {
   const uint32_t u = (uint32_t)(k >> kb);
   const uint32_t v = (uint32_t)(k & ((1ull << kb) - 1));
   const uint32_t end = row_ptr[u + 1];
@@ -383,7 +380,50 @@ __global__ void k_arc_rec(const uint64_t* __restrict__ okeys, uint64_t m, uint32
       y = (d << 16) | (two ? rsplit[u] - b : 0u);
     }
   }
-  arec[e] = make_uint2(x, y);
+  return make_uint2(x, y);
+}
+
+// One 8-byte record per arc, so the wedge-range fill gathers once per range
+// (graphs whose records do not fit ArcPack).
+__global__ void k_arc_rec(const uint64_t* __restrict__ okeys, uint64_t m, uint32_t kb,
+                          const uint32_t* __restrict__ row_ptr, const uint32_t* __restrict__ col,
+                          const uint32_t* __restrict__ rsplit, bool nar, uint2* __restrict__ arec) {
+  const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < m) arec[e] = arc_record(okeys[e], e, kb, row_ptr, col, rsplit, nar);
+}
+
+// An arc and its record in the value of the sort by head and the bits of its
+// 32-bit key above the head: from bit 0, the arc (eb bits), its range's length
+// (lb bits: no outdegree has more) and, with narrow records, their two flags, dh
+// (8 bits) and the split offset (lb bits, below the length); the key takes what
+// passes 64 bits. The sort then delivers the records in place: sorting arc
+// numbers and gathering 8-byte records by them pulled a sector from HBM for each
+// (R-MAT scale 25: sort 11.2 + gather 11.9 ms; with the records in the values 13.3
+// + 5.3).
+struct ArcPack {
+  uint32_t kb, eb, lb;
+  bool nar;
+  __host__ __device__ uint32_t bits() const { return eb + lb + (nar ? 10 + lb : 0); }
+  __host__ __device__ bool fits() const { return bits() <= 64 + (32 - kb); }
+};
+
+__global__ void k_arc_pack(const uint64_t* __restrict__ okeys, uint64_t m, ArcPack p,
+                           const uint32_t* __restrict__ row_ptr, const uint32_t* __restrict__ col,
+                           const uint32_t* __restrict__ rsplit, uint32_t* __restrict__ key,
+                           uint64_t* __restrict__ val) {
+  const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= m) return;
+  const uint64_t k = okeys[e];
+  const uint2 r = arc_record(k, e, p.kb, row_ptr, col, rsplit, p.nar);
+  const uint32_t len = (p.nar ? r.x & 0x3FFFFFFFu : r.x) - (uint32_t)e - 1;
+  unsigned __int128 w = e | ((unsigned __int128)len << p.eb);
+  if (p.nar) {
+    const uint64_t n = (r.x >> 30) | ((uint64_t)(r.y >> 16) << 2) | ((uint64_t)(r.y & 0xFFFFu) << 10);
+    w |= (unsigned __int128)n << (p.eb + p.lb);
+  }
+  val[e] = (uint64_t)w;
+  const uint32_t hi = (uint32_t)(w >> 64);  // zero when p.kb == 32
+  key[e] = (uint32_t)(k & ((1ull << p.kb) - 1)) | (p.kb < 32 ? hi << p.kb : 0u);
 }
 
 // ------------------------------------------------------------ range lists
@@ -515,6 +555,32 @@ __global__ void k_sfx_fill(const uint32_t* __restrict__ head, const uint32_t* __
   }
   uint64_t sum = 0;
   if (wave_segment_tail(v, valid, len, &sum) && sum) atomicAdd(&w_sfx[v], (unsigned long long)sum);
+}
+
+// k_sfx_fill from packed records (ArcPack) sorted by head: everything streams.
+__global__ void k_sfx_unpack(const uint32_t* __restrict__ key, const uint64_t* __restrict__ val, uint64_t m, ArcPack p,
+                             uint2* __restrict__ rng, uint8_t* __restrict__ dh, uint16_t* __restrict__ split,
+                             unsigned long long* __restrict__ w_sfx) {
+  const uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const bool valid = j < m;
+  const uint32_t k = valid ? key[j] : 0u;
+  const uint32_t v = valid ? (uint32_t)(k & ((1ull << p.kb) - 1)) : 0xFFFFFFFFu;
+  uint32_t len = 0;
+  if (valid) {
+    const unsigned __int128 w = ((unsigned __int128)(p.kb < 32 ? k >> p.kb : 0u) << 64) | val[j];
+    const uint32_t b = (uint32_t)((uint64_t)w & ((1ull << p.eb) - 1)) + 1;
+    len = (uint32_t)((uint64_t)(w >> p.eb) & ((1ull << p.lb) - 1));
+    uint32_t x = b + len;
+    if (p.nar) {
+      const uint64_t n = (uint64_t)(w >> (p.eb + p.lb));
+      x |= (uint32_t)(n & 3) << 30;
+      dh[j] = (uint8_t)(n >> 2);
+      split[j] = (uint16_t)((n >> 10) & ((1ull << p.lb) - 1));
+    }
+    rng[j] = make_uint2(b, x);
+  }
+  uint32_t sum = 0;  // 64 lengths of at most 2^17
+  if (wave_segment_tail_u32(v, valid, len, &sum) && sum) atomicAdd(&w_sfx[v], (unsigned long long)sum);
 }
 
 // In-arcs per vertex: deg(v) - outdeg(v) (cnt[n] = 0 for the exclusive scan).
@@ -740,25 +806,17 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
     });
   }
 
-  // 7. totals (W+, active rows, largest outdeg) from the rows; relabelled
-  // graphs also get every arc's record (row end, narrow record of its wedge range)
+  // 7. totals (W+, active rows, largest outdeg) from the rows
   DevBuf<RowStats> st(ctx, 1);
   k_fill_u32<<<1, 64, 0, s>>>(reinterpret_cast<uint32_t*>(st.p), sizeof(RowStats) / 4, 0u);
   k_row_flags<<<totals_grid(n), kBlock, 0, s>>>(row_ptr.p, deg.p, n, st.p);
   const bool narrow = relabel && m && m < (1ull << 30);
-  DevBuf<uint2> arec;
-  arec.ctx = ctx;
-  if (relabel && m) {
-    arec = DevBuf<uint2>(ctx, m);
-    DevBuf<uint32_t> rsplit;
-    rsplit.ctx = ctx;
-    if (narrow) {
-      rsplit = DevBuf<uint32_t>(ctx, n);
-      k_row_split<<<grid_for(n, kBlock), kBlock, 0, s>>>(row_ptr.p, col.p, n, rsplit.p);
-    }
-    k_arc_rec<<<grid_for(m, kBlock), kBlock, 0, s>>>(uniq.p, m, kb, row_ptr.p, col.p, rsplit.p, narrow, arec.p);
+  DevBuf<uint32_t> rsplit;
+  rsplit.ctx = ctx;
+  if (narrow) {
+    rsplit = DevBuf<uint32_t>(ctx, n);
+    k_row_split<<<grid_for(n, kBlock), kBlock, 0, s>>>(row_ptr.p, col.p, n, rsplit.p);
   }
-  uniq.reset();
   RowStats hst;
   TB_HIP(hipMemcpyAsync(&hst, st.p, sizeof(hst), hipMemcpyDeviceToHost, s));
 
@@ -784,19 +842,44 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
     DevBuf<uint32_t> cnt(ctx, n + 1);
     k_in_count<<<grid_for(n + 1, kBlock), kBlock, 0, s>>>(row_ptr.p, deg.p, n, cnt.p);
     if (m) {
-      DevBuf<uint32_t> arcs(ctx, m), head(ctx, m), arc_sorted(ctx, m);
-      k_iota_u32<<<grid_for(m, kBlock), kBlock, 0, s>>>(arcs.p, m);
-      with_temp(ctx, [&](void* t, size_t& b) {
-        return rocprim::radix_sort_pairs<IdSortConfig>(t, b, col.p, head.p, arcs.p, arc_sorted.p, (size_t)m, 0u,
-                                                       bits_for(n), s);
-      });
-      arcs.reset();
-      k_sfx_fill<<<grid_for(m, kBlock), kBlock, 0, s>>>(head.p, arc_sorted.p, m, arec.p, rng_sfx.p, sfx_dh.p,
-                                                        sfx_split.p, reinterpret_cast<unsigned long long*>(w_sfx.p));
+      // no outdegree passes 2 sqrt(m): its vertices' degrees (octave ids: half of
+      // them) are all at least as large. The real largest is asked for only when
+      // that bound leaves the records too wide.
+      ArcPack pack{kb, bits_for(m), bits_for((uint64_t)(2.0 * std::sqrt((double)m)) + 2), narrow};
+      if (!pack.fits()) {
+        ctx->sync();
+        pack.lb = bits_for((uint64_t)hst.max_outdeg + 1);
+      }
+      if (pack.fits()) {
+        DevBuf<uint32_t> key(ctx, m), key_sorted(ctx, m);
+        DevBuf<uint64_t> val(ctx, m), val_sorted(ctx, m);
+        k_arc_pack<<<grid_for(m, kBlock), kBlock, 0, s>>>(uniq.p, m, pack, row_ptr.p, col.p, rsplit.p, key.p, val.p);
+        with_temp(ctx, [&](void* t, size_t& b) {
+          return rocprim::radix_sort_pairs<IdSortConfig>(t, b, key.p, key_sorted.p, val.p, val_sorted.p, (size_t)m,
+                                                         0u, kb, s);
+        });
+        k_sfx_unpack<<<grid_for(m, kBlock), kBlock, 0, s>>>(key_sorted.p, val_sorted.p, m, pack, rng_sfx.p, sfx_dh.p,
+                                                           sfx_split.p,
+                                                           reinterpret_cast<unsigned long long*>(w_sfx.p));
+      } else {
+        DevBuf<uint2> arec(ctx, m);
+        k_arc_rec<<<grid_for(m, kBlock), kBlock, 0, s>>>(uniq.p, m, kb, row_ptr.p, col.p, rsplit.p, narrow, arec.p);
+        DevBuf<uint32_t> arcs(ctx, m), head(ctx, m), arc_sorted(ctx, m);
+        k_iota_u32<<<grid_for(m, kBlock), kBlock, 0, s>>>(arcs.p, m);
+        with_temp(ctx, [&](void* t, size_t& b) {
+          return rocprim::radix_sort_pairs<IdSortConfig>(t, b, col.p, head.p, arcs.p, arc_sorted.p, (size_t)m, 0u,
+                                                         bits_for(n), s);
+        });
+        arcs.reset();
+        k_sfx_fill<<<grid_for(m, kBlock), kBlock, 0, s>>>(head.p, arc_sorted.p, m, arec.p, rng_sfx.p, sfx_dh.p,
+                                                          sfx_split.p,
+                                                          reinterpret_cast<unsigned long long*>(w_sfx.p));
+      }
     }
     with_temp(ctx, [&](void* t, size_t& b) {
       return rocprim::exclusive_scan(t, b, cnt.p, sfx_ptr.p, 0u, (size_t)(n + 1), rocprim::plus<uint32_t>(), s);
     });
+    uniq.reset();
     if (narrow) {
       const uint64_t words = (m + 1) / 2 + 1;
       col16 = DevBuf<uint32_t>(ctx, words);
@@ -804,7 +887,6 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
       k_col16<<<grid_for(m, kBlock), kBlock, 0, s>>>(col.p, m, reinterpret_cast<uint16_t*>(col16.p));
     }
   }
-  arec.reset();
 
   // the graph owns its buffers from here on (freed by tribit_graph_free, also on error)
   g->row_ptr = row_ptr.release();
