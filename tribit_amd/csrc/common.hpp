@@ -143,12 +143,17 @@ struct DevBuf {
 namespace tb {
 struct BucketCache;
 
-// Device counters of one count: u64 [0] triangles, [1] fallback tasks; from
-// u64 index kQueueOff, the task queues: per menu slot, kQueues sub-queues of
-// one u32 each, kQStride u32 apart so that no two share a cache line.
-constexpr uint32_t kQueues = 8;
-constexpr uint32_t kQStride = 64;
-constexpr size_t kQueueOff = 32;
+// Device counters of one count, none of them sharing a 128-byte line with
+// another: kResults slots of u64 {triangles, fallback tasks}, then from u64
+// index kQueueOff the task queues, per menu slot kQueues sub-queues of one u32.
+// Atomics on one address serialise at about 13 ns on MI355X, so a workgroup adds
+// its sums to slot blockIdx.x % kResults (the host adds the slots up) and claims
+// its tasks from sub-queue blockIdx.x % kQueues first.
+constexpr uint32_t kResults = 16;
+constexpr uint32_t kResultStride = 16;  // u64
+constexpr uint32_t kQueues = 64;        // eight per XCD
+constexpr uint32_t kQStride = 32;       // u32
+constexpr size_t kQueueOff = (size_t)kResults * kResultStride;
 constexpr size_t kCountScratch = kQueueOff + (size_t)TRIBIT_MENU_SLOTS * kQueues * kQStride / 2;
 }  // namespace tb
 

@@ -35,6 +35,10 @@ constexpr unsigned kBlock = 256;
 // tasks are the longest: taken first, they overlap with the many short
 // tasks instead of forming the launch's tail.
 constexpr uint32_t kWaveBatch = 16;      // most wave tasks taken per queue atomic
+// Tasks per wave of launches too small to fill the chip. A task is a serial chain
+// of dependent loads (about 3 us), so more waves shorten the launch: 80K-edge
+// R-MAT, 16 and 4 tasks a wave 51 + 21 us, two 28 + 17 (outdeg <= 32, <= 256).
+constexpr uint32_t kTasksPerWave = 2;
 constexpr uint32_t kClaimsPerWave = 8;   // queue claims per wave of a wave launch (when tasks allow)
 constexpr uint32_t kChunk = 2048;        // probe-set chunk of class-3 rows
 constexpr uint64_t kWaveCap = 1u << 15;  // target streamed elements per wave task
@@ -610,63 +614,108 @@ __device__ __forceinline__ uint32_t stream_tiles(const TileSrc& ts, const uint2*
 // consecutive tasks. The units are split over kQueues sub-queues (unit k goes
 // to sub-queue k % kQueues, in order: each sub-queue also starts with its
 // heaviest) and claimed `claim` units at a time; a block starts on sub-queue
-// blockIdx.x % kQueues and moves on to the next one when that one runs dry.
-// Claims on one address serialise (about 13 ns each on MI355X): with one
-// queue, a launch of ~100K tasks spent most of its time claiming. Every value
-// is wave-uniform.
+// blockIdx.x % kQueues. Claims on one address serialise (about 13 ns each on
+// MI355X): a full grid of 8,192 waves makes about 64K claims, 106 us of them on
+// each of eight sub-queues, 13 us on each of 64. When a wave's sub-queue runs
+// dry, its 64 lanes read all the counters at once (no atomics: 8,192 waves
+// finding eight dry queues one by one took another 106 us) and it moves to the
+// nearest that is not, those of its own XCD first. With both and one result
+// atomic per workgroup, a 1.1M-edge Chung-Lu graph's two wave launches take 0.14 +
+// 0.086 instead of 0.353 + 0.097 ms. Every value is wave-uniform.
 //
-// Contiguous mode (batches, whose tasks are grouped by graph): sub-queue q
-// holds the q-th eighth of the units instead. Workgroup b runs on XCD b % 8
-// and starts on sub-queue b % kQueues, so each XCD streams the rows of its own
-// graphs and its L2 is not filled with the rows the other seven stream.
+// Contiguous mode (batches, whose tasks are grouped by graph): XCD x's eight
+// sub-queues (x, x + 8, ...) share the x-th eighth of the units, dealt out to
+// them in runs of `claim`. So they advance together through the same graphs, and
+// a claim is a run of neighbouring owners, whose ranges overlap (768 Chung-Lu
+// graphs: an eighth of the eighth for each sub-queue 22.6 ms, single units dealt
+// out 18.6, runs 17.8). Workgroup b runs on XCD b % 8 and starts on sub-queue
+// b % kQueues, so each XCD streams the rows of its own graphs and its L2 is not
+// filled with the rows the other seven stream.
 struct TaskFeed {
+  static_assert(kQueues == 64, "one lane per sub-queue");
   uint32_t* queue;
   uint32_t ntasks, unit, claim;
-  bool contig;
-  uint32_t q, left;      // current sub-queue, sub-queues not yet found empty
-  uint32_t c, cend, nq;  // claimed units [c, cend) of sub-queue q, its unit count
-  uint32_t q0;           // contiguous mode: the first unit of sub-queue q
+  bool contig, open;  // open: sub-queue q may have units left
+  uint32_t home, q;   // the block's sub-queue, the current one
+  uint32_t c, cend;   // claimed units: numbers in the launch (contiguous mode) or in sub-queue q
+  uint64_t dry;       // sub-queues this wave's claims found empty: each is tried in vain once at most
 
   __device__ TaskFeed(uint32_t* qs, uint32_t nt, uint32_t unit_, uint32_t claim_, bool contig_ = false)
-      : queue(qs), ntasks(nt), unit(unit_), claim(claim_), contig(contig_), q(blockIdx.x % kQueues),
-        left(kQueues), c(0), cend(0), nq(units_of(blockIdx.x % kQueues)), q0(first_unit(blockIdx.x % kQueues)) {}
+      : queue(qs), ntasks(nt), unit(unit_), claim(claim_), contig(contig_), open(true), home(blockIdx.x % kQueues),
+        q(home), c(0), cend(0), dry(0) {}
 
-  __device__ uint32_t first_unit(uint32_t sq) const {
-    const uint64_t nu = (ntasks + unit - 1) / unit;
-    return contig ? (uint32_t)(nu * sq / kQueues) : 0u;
-  }
+  __device__ uint32_t eighth(uint32_t x) const { return (uint32_t)((uint64_t)((ntasks + unit - 1) / unit) * x / 8); }
 
-  __device__ uint32_t units_of(uint32_t sq) const {
-    const uint32_t nu = (ntasks + unit - 1) / unit;
-    if (contig) return first_unit(sq + 1) - first_unit(sq);
-    return nu > sq ? (nu - sq + kQueues - 1) / kQueues : 0u;
+  // What sub-queue sq counts up to: its units, or its runs of `claim` units.
+  __device__ uint32_t size_of(uint32_t sq) const {
+    const uint32_t step = contig ? 8 : kQueues, at = contig ? sq >> 3 : sq;
+    const uint32_t all = contig ? (eighth((sq & 7) + 1) - eighth(sq & 7) + claim - 1) / claim
+                                : (ntasks + unit - 1) / unit;
+    return all > at ? (all - at + step - 1) / step : 0u;
   }
 
   // The next unit [tb, tend) of this wave; false when the launch has none left.
   __device__ bool get(uint32_t lane, uint32_t& tb, uint32_t& tend) {
     for (;;) {
       if (c < cend) {
-        tb = (contig ? q0 + c : c * kQueues + q) * unit;
+        tb = (contig ? c : c * kQueues + q) * unit;
         tend = min(tb + unit, ntasks);
         ++c;
         return true;
       }
-      if (!left) return false;
+      if (!open) {
+        // lane p: the p-th sub-queue to try, the eight of the block's XCD first
+        const uint32_t sq = ((home + (lane >> 3)) & 7) + 8 * (((home >> 3) + lane) & 7);
+        const uint32_t v = __hip_atomic_load(queue + sq * kQStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint64_t left = __ballot(v < size_of(sq) && !((dry >> sq) & 1ull));
+        if (!left) return false;  // counters only grow: an empty sub-queue stays empty
+        q = __builtin_amdgcn_readlane(sq, __ffsll((long long)left) - 1);
+      }
+      const uint32_t nq = size_of(q), by = contig ? 1u : claim;
       uint32_t v = 0;
-      if (lane == 0) v = atomicAdd(queue + q * kQStride, claim);
-      v = __shfl(v, 0);
-      if (v < nq) {
+      if (lane == 0) v = atomicAdd(queue + q * kQStride, by);
+      v = __builtin_amdgcn_readfirstlane(v);  // every member stays in scalar registers
+      open = v < nq;
+      if (!open) {
+        dry |= 1ull << q;
+      } else if (contig) {
+        const uint32_t f = eighth(q & 7);
+        c = f + (8 * v + (q >> 3)) * claim;
+        cend = min(c + claim, eighth((q & 7) + 1));
+      } else {
         c = v;
         cend = min(v + claim, nq);
-      } else {
-        --left;
-        q = (q + 1) % kQueues;
-        nq = units_of(q);
-        q0 = first_unit(q);
       }
     }
   }
 };
+
+// A workgroup's counts, summed over its WAVES waves, to its result slot: one
+// atomic instead of one per wave on a single address (8,192 of them: 106 us).
+// Called by every thread; acc per lane, fallbacks per wave.
+template <int WAVES>
+__device__ __forceinline__ void add_result(unsigned long long* result, uint64_t acc, uint32_t fallbacks,
+                                           uint32_t lane) {
+  __shared__ unsigned long long s_acc[WAVES];
+  __shared__ uint32_t s_fall[WAVES];
+  acc = wave_sum_u64(acc);
+  if (lane == 0) {
+    s_acc[threadIdx.x >> 6] = acc;
+    s_fall[threadIdx.x >> 6] = fallbacks;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long a = 0;
+    uint32_t f = 0;
+    for (int i = 0; i < WAVES; ++i) {
+      a += s_acc[i];
+      f += s_fall[i];
+    }
+    unsigned long long* r = result + (blockIdx.x % kResults) * kResultStride;
+    if (a) atomicAdd(r, a);
+    if (f) atomicAdd(r + 1, (unsigned long long)f);
+  }
+}
 
 // A wave's per-graph counts (batches), summed while consecutive tasks belong
 // to one graph and added to that graph's counter when the graph changes: one
@@ -748,9 +797,7 @@ __global__ __launch_bounds__(256) void k_count_wave(const uint32_t* __restrict__
     }
   }
   if (gcount) gsum.flush(gcount, lane);
-  acc = wave_sum_u64(acc);
-  if (lane == 0 && acc) atomicAdd(result, (unsigned long long)acc);
-  if (lane == 0 && fallbacks) atomicAdd(result + 1, (unsigned long long)fallbacks);
+  add_result<4>(result, acc, fallbacks, lane);
 }
 
 // Multi-task waves for owners with tiny sets: a wave takes MT tasks at once,
@@ -889,9 +936,7 @@ __global__ __launch_bounds__(256) void k_count_wave_multi(const uint32_t* __rest
     }
   }
   if (gcount) gsum.flush(gcount, lane);
-  acc = wave_sum_u64(acc);
-  if (lane == 0 && acc) atomicAdd(result, (unsigned long long)acc);
-  if (lane == 0 && fallbacks) atomicAdd(result + 1, (unsigned long long)fallbacks);
+  add_result<4>(result, acc, fallbacks, lane);
 }
 
 // ----------------------------------------------------- block-level tasks
@@ -1110,9 +1155,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_count_block(const uint32_t* _
     }
     if (tdur && threadIdx.x == 0) tdur[ntasks - 1 - t] = (uint32_t)(wall_clock64() - t0);
   }
-  acc = wave_sum_u64(acc);
-  if (lane == 0 && acc) atomicAdd(result, (unsigned long long)acc);
-  if (threadIdx.x == 0 && fallbacks) atomicAdd(result + 1, (unsigned long long)fallbacks);
+  add_result<kBlockThreads / 64>(result, acc, threadIdx.x == 0 ? fallbacks : 0u, lane);
 }
 
 // Kernel variants: LDS set size (LOGS), staged ranges per batch (KMAX), lane
@@ -1859,7 +1902,7 @@ static void learned_table(tribit_ctx* ctx, const BucketStats& st, int layout, in
 // whole count can be captured into a hipGraph).
 struct LaunchArgs {
   int att = 0;                           // mode word (attempts | flags)
-  unsigned long long* result = nullptr;  // [0] triangles, [1] fallback tasks
+  unsigned long long* result = nullptr;  // kResults slots of {triangles, fallback tasks}
   uint32_t* queue = nullptr;             // per slot kQueues task counters, kQStride apart
   uint32_t* tdur = nullptr;              // per-task durations, indexed like the schedule's tasks, or null
   const uint4* task0 = nullptr;          // the schedule's first task (tdur's origin)
@@ -1887,11 +1930,7 @@ static void launch_wave_t(const LaunchArgs& a, int slot, uint32_t ntasks, int cu
   TB_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_count_wave<LOGS, KMAX, G, U, BUF>, kBlock, 0));
   if (a.waves[slot] > 0 && per_cu > a.waves[slot]) per_cu = a.waves[slot];
   if (per_cu < 1) per_cu = 1;
-  // waves for about kWaveBatch tasks each (4 for the 512-slot sets, whose
-  // short launches on small graphs gained from more waves; the 64-slot
-  // kernel's did not)
-  const uint64_t tpw = LOGS >= kC1Logs ? 4 : kWaveBatch;
-  const uint64_t want = (ntasks + 4 * tpw - 1) / (4 * tpw);
+  const uint64_t want = (ntasks + 4 * kTasksPerWave - 1) / (4 * kTasksPerWave);
   const unsigned grid = (unsigned)std::min<uint64_t>(want, (uint64_t)cus * per_cu);
   const uint32_t wb = claim_size(ntasks, 4ull * grid, 1);
   k_count_wave<LOGS, KMAX, G, U, BUF><<<grid, kBlock, 0, s>>>(g->row_ptr, g->col, g->m, rng, tasks, ntasks,
@@ -2271,10 +2310,14 @@ static uint64_t count_once(tribit_ctx* ctx, tribit_graph* g, int sched, int flag
       if (S.tot.v[v])
         k_tdur_reduce<<<(unsigned)std::min<uint64_t>((S.tot.v[v] + 255) / 256, 1024), 256, 0, s>>>(
             S.tasks.p + S.base.v[v], tdur.p + S.base.v[v], S.tot.v[v], tlog + (size_t)v * kBuckets);
-  unsigned long long res[2] = {0, 0};
-  TB_HIP(hipMemcpyAsync(res, a.result, sizeof(res), hipMemcpyDeviceToHost, s));
+  unsigned long long slots[kQueueOff], res[2] = {0, 0};
+  TB_HIP(hipMemcpyAsync(slots, a.result, sizeof(slots), hipMemcpyDeviceToHost, s));
   TB_HIP(hipEventSynchronize(last));
   ctx->sync();
+  for (uint32_t i = 0; i < kResults; ++i) {
+    res[0] += slots[i * kResultStride];
+    res[1] += slots[i * kResultStride + 1];
+  }
   *ms_sched = elapsed(ctx->ev[2], ctx->ev[3]);
   *ms_kernel = elapsed(ctx->ev[3], last);
   *ms_total = elapsed(ctx->ev[2], last);
