@@ -12,9 +12,13 @@
 // Every launch is a 1-D grid of 256-thread blocks (4 waves).
 #include <cmath>
 #include <cstring>
+#include <rocprim/block/block_radix_sort.hpp>
+#include <rocprim/block/block_scan.hpp>
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 #include <rocprim/device/device_select.hpp>
+#include <rocprim/iterator/counting_iterator.hpp>
+#include <rocprim/iterator/transform_iterator.hpp>
 
 #include "common.hpp"
 #include "device.hpp"
@@ -22,6 +26,9 @@
 namespace tb {
 
 constexpr unsigned kBlock = 256;
+
+// Ids in col16: m rounded up to whole dwords, and one more dword.
+__host__ __device__ inline uint64_t col16_ids(uint64_t m) { return ((m + 1) / 2 + 1) * 2; }
 
 // ---------------------------------------------------------------- generators
 
@@ -151,23 +158,7 @@ __device__ __forceinline__ uint64_t arc_key(uint32_t u, uint32_t v, uint32_t kb)
   return ((uint64_t)u << kb) | (uint64_t)v;
 }
 
-// Degree orientation: {a<b} becomes a->b iff deg(a) <= deg(b).
-__global__ void k_orient(const uint64_t* __restrict__ keys, uint64_t m, const uint32_t* __restrict__ deg,
-                         uint32_t kb, uint64_t* __restrict__ okeys) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  const uint64_t k = keys[i];
-  const uint32_t a = (uint32_t)(k >> kb), b = (uint32_t)(k & ((1ull << kb) - 1));
-  okeys[i] = (deg[a] <= deg[b]) ? arc_key(a, b, kb) : arc_key(b, a, kb);
-}
-
-// col[i] = dst, odeg[src] += 1 (sorted by src: aggregated per run).
 // Degree relabelling: new id = rank of (deg, old id); lab[old] = new.
-__global__ void k_iota_u32(uint32_t* __restrict__ p, uint64_t n) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = (uint32_t)i;
-}
-
 // cls[v] = floor(log2(deg[v])) + 1 (0 for an isolated vertex): octave classes.
 __global__ void k_octave(const uint32_t* __restrict__ deg, uint64_t n, uint32_t* __restrict__ cls) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -186,23 +177,55 @@ __global__ void k_scatter_labels(const uint32_t* __restrict__ old_of_new, uint64
   if (i < n) lab[old_of_new[i]] = (uint32_t)i;
 }
 
+// Zeroed on the way by a kernel whose grid covers them: one launch fewer each.
+struct ZeroSpans {
+  uint32_t* p[3];
+  uint64_t n[3];
+  __device__ __forceinline__ void clear(uint64_t i) const {
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      if (i < n[k]) p[k][i] = 0u;
+  }
+  uint64_t most() const { return std::max(n[0], std::max(n[1], n[2])); }
+};
+
+// Degree orientation: {a<b} becomes a->b iff deg(a) <= deg(b).
+__global__ void k_orient(const uint64_t* __restrict__ keys, uint64_t m, const uint32_t* __restrict__ deg,
+                         uint32_t kb, uint64_t* __restrict__ okeys, ZeroSpans z) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  z.clear(i);
+  if (i >= m) return;
+  const uint64_t k = keys[i];
+  const uint32_t a = (uint32_t)(k >> kb), b = (uint32_t)(k & ((1ull << kb) - 1));
+  okeys[i] = (deg[a] <= deg[b]) ? arc_key(a, b, kb) : arc_key(b, a, kb);
+}
+
 // With relabelled ids the degree order is the id order: a -> b iff a < b.
 __global__ void k_orient_relabel(const uint64_t* __restrict__ keys, uint64_t m, const uint32_t* __restrict__ lab,
-                                 uint32_t kb, uint64_t* __restrict__ okeys) {
+                                 uint32_t kb, uint64_t* __restrict__ okeys, ZeroSpans z) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  z.clear(i);
   if (i >= m) return;
   const uint64_t k = keys[i];
   const uint32_t a = lab[(uint32_t)(k >> kb)], b = lab[(uint32_t)(k & ((1ull << kb) - 1))];
   okeys[i] = a < b ? arc_key(a, b, kb) : arc_key(b, a, kb);
 }
 
+// col[i] = dst (and its low 16 bits in col16, when given: narrow wedge ranges
+// are streamed from these), odeg[src] += 1 (sorted by src: aggregated per run).
 __global__ void k_csr_split(const uint64_t* __restrict__ okeys, uint64_t m, uint32_t kb, uint32_t* __restrict__ col,
-                            uint32_t* __restrict__ odeg) {
+                            uint16_t* __restrict__ col16, uint32_t* __restrict__ odeg) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const bool valid = i < m;
   const uint64_t k = valid ? okeys[i] : 0;
   const uint32_t s = valid ? (uint32_t)(k >> kb) : 0xFFFFFFFFu;
-  if (valid) col[i] = (uint32_t)(k & ((1ull << kb) - 1));
+  if (valid) {
+    const uint32_t v = (uint32_t)(k & ((1ull << kb) - 1));
+    col[i] = v;
+    if (col16) col16[i] = (uint16_t)v;
+  } else if (col16 && i < col16_ids(m)) {
+    col16[i] = 0;  // the padding to whole dwords plus one
+  }
   const uint32_t run = wave_run_length(s, valid);
   if (run) atomicAdd(&odeg[s], run);
 }
@@ -217,7 +240,7 @@ struct RowStats {
 // Totals over a bounded grid (grid-stride loops, one atomic per block and
 // field): one atomic per wave on a single address serialises at about 13 ns
 // each, 7 ms for 2^25 rows and 100 ms for 2^29 arcs.
-constexpr unsigned kTotalsBlocks = 1024;
+constexpr unsigned kTotalsBlocks = 2048;
 inline unsigned totals_grid(uint64_t n) {
   return (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(kTotalsBlocks, (n + kBlock - 1) / kBlock));
 }
@@ -294,19 +317,36 @@ int auto_relabel(uint64_t n, uint64_t band_edges) {
 
 // Rows with outdeg >= 2, the largest outdeg and, with deg (undirected
 // degrees), W+ = sum over v of indeg(v) * outdeg(v): every arc u -> v streams
-// N+(v) once, and v has deg(v) - outdeg(v) in-arcs.
-__global__ void __launch_bounds__(kBlock) k_row_flags(const uint32_t* __restrict__ row_ptr,
-                                                      const uint32_t* __restrict__ deg, uint64_t n,
-                                                      RowStats* __restrict__ st) {
+// N+(v) once, and v has deg(v) - outdeg(v) in-arcs. With split (relabelled
+// graphs), also per row the position where its last 64K-id window begins (the
+// first id whose high 16 bits equal the last id's), for the narrow records of its
+// wedge ranges: one lower-bound search per row.
+__global__ void __launch_bounds__(kBlock) k_rows(const uint32_t* __restrict__ row_ptr,
+                                                 const uint32_t* __restrict__ deg, const uint32_t* __restrict__ col,
+                                                 uint64_t n, RowStats* __restrict__ st, uint32_t* __restrict__ split) {
   __shared__ unsigned long long s_act[kBlock / 64], s_w[kBlock / 64];
   __shared__ uint32_t s_max[kBlock / 64];
   uint64_t act = 0, w = 0;
   uint32_t dm = 0;
   for (uint64_t u = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; u < n; u += (uint64_t)gridDim.x * blockDim.x) {
-    const uint32_t d = row_ptr[u + 1] - row_ptr[u];
+    const uint32_t b = row_ptr[u], e = row_ptr[u + 1], d = e - b;
     act += d >= 2;
     dm = d > dm ? d : dm;
     if (deg) w += (uint64_t)(deg[u] - d) * d;
+    if (!split) continue;
+    uint32_t lo = b;
+    if (b < e) {
+      const uint32_t l = col[e - 1] >> 16;
+      uint32_t hi = e - 1;  // col[hi] is in window l
+      while (lo < hi) {
+        const uint32_t mid = lo + ((hi - lo) >> 1);
+        if ((col[mid] >> 16) >= l)
+          hi = mid;
+        else
+          lo = mid + 1;
+      }
+    }
+    split[u] = lo;
   }
   act = wave_sum_u64(act);
   w = wave_sum_u64(w);
@@ -327,29 +367,6 @@ __global__ void __launch_bounds__(kBlock) k_row_flags(const uint32_t* __restrict
     if (w) atomicAdd(&st->wplus, (unsigned long long)w);
     if (dm) atomicMax(&st->max_outdeg, dm);
   }
-}
-
-// Per row u of a relabelled graph: the position where the row's last 64K-id
-// window begins (the first id whose high 16 bits equal the last id's), for
-// the narrow records of its wedge ranges. One lower-bound search per row.
-__global__ void k_row_split(const uint32_t* __restrict__ row_ptr, const uint32_t* __restrict__ col, uint64_t n,
-                            uint32_t* __restrict__ split) {
-  const uint64_t u = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (u >= n) return;
-  const uint32_t b = row_ptr[u], e = row_ptr[u + 1];
-  uint32_t lo = b;
-  if (b < e) {
-    const uint32_t l = col[e - 1] >> 16;
-    uint32_t hi = e - 1;  // col[hi] is in window l
-    while (lo < hi) {
-      const uint32_t mid = lo + ((hi - lo) >> 1);
-      if ((col[mid] >> 16) >= l)
-        hi = mid;
-      else
-        lo = mid + 1;
-    }
-  }
-  split[u] = lo;
 }
 
 // The record of arc e = (u -> v) of a relabelled graph, packed k = (u << kb) | v,
@@ -583,14 +600,6 @@ __global__ void k_sfx_unpack(const uint32_t* __restrict__ key, const uint64_t* _
   if (wave_segment_tail_u32(v, valid, len, &sum) && sum) atomicAdd(&w_sfx[v], (unsigned long long)sum);
 }
 
-// In-arcs per vertex: deg(v) - outdeg(v) (cnt[n] = 0 for the exclusive scan).
-__global__ void k_in_count(const uint32_t* __restrict__ row_ptr, const uint32_t* __restrict__ deg, uint64_t n,
-                           uint32_t* __restrict__ cnt) {
-  const uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (v < n) cnt[v] = deg[v] - (row_ptr[v + 1] - row_ptr[v]);
-  if (v == n) cnt[v] = 0;
-}
-
 // W+(u) = sum of outdeg(v) over v in N+(u), per row (the PLAIN layout's work).
 __global__ void k_row_wplus(const uint32_t* __restrict__ row_ptr, const uint32_t* __restrict__ col, uint64_t n,
                             uint64_t* __restrict__ wrow) {
@@ -602,12 +611,6 @@ __global__ void k_row_wplus(const uint32_t* __restrict__ row_ptr, const uint32_t
     w += row_ptr[v + 1] - row_ptr[v];
   }
   wrow[u] = w;
-}
-
-// Low 16 bits of every id (narrow wedge ranges are streamed from these).
-__global__ void k_col16(const uint32_t* __restrict__ col, uint64_t m, uint16_t* __restrict__ col16) {
-  const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < m) col16[e] = (uint16_t)(col[e] & 0xFFFFu);
 }
 
 __global__ void k_fill_u64(unsigned long long* __restrict__ p, uint64_t n) {
@@ -638,7 +641,133 @@ using IdSortConfig = rocprim::radix_sort_config<
     rocprim::radix_sort_onesweep_config<rocprim::kernel_config<1024, 16>, rocprim::kernel_config<1024, 16>, 9,
                                         rocprim::block_radix_rank_algorithm::match>>;
 
+// Sorts and scans of at most kSmallSort items: one workgroup, one launch. The
+// device-wide ones are seven or eight launches at these sizes (a block sort and
+// its merge steps), about 7 us each, and most of what a small graph's
+// preprocessing took: 1,000 vertices and 8,000 keys 0.35 -> 0.2 ms a call, with
+// the passes over n and m that now share a launch.
+constexpr uint32_t kSmallSort = 8192;
+constexpr uint32_t kSmallThreads = 1024;
+constexpr uint32_t kSmallItems = kSmallSort / kSmallThreads;
+
+// Missing items get the largest key of `bits` bits and, the sort being stable, stay last.
+template <typename K, typename V>
+__global__ void __launch_bounds__(kSmallThreads) k_sort_small(const K* __restrict__ in, K* __restrict__ out,
+                                                              const V* __restrict__ vin, V* __restrict__ vout,
+                                                              uint32_t n, uint32_t bits) {
+  using Sort = rocprim::block_radix_sort<K, kSmallThreads, kSmallItems, V>;
+  __shared__ typename Sort::storage_type tmp;
+  K k[kSmallItems];
+  V v[kSmallItems];
+#pragma unroll
+  for (uint32_t j = 0; j < kSmallItems; ++j) {
+    const uint32_t i = threadIdx.x * kSmallItems + j;
+    k[j] = i < n ? in[i] : (K)~(K)0;
+    v[j] = i < n ? (vin ? vin[i] : (V)i) : (V)0;
+  }
+  Sort().sort_to_striped(k, v, tmp, 0, bits);
+#pragma unroll
+  for (uint32_t j = 0; j < kSmallItems; ++j) {
+    const uint32_t i = threadIdx.x + j * kSmallThreads;
+    if (i < n) {
+      out[i] = k[j];
+      vout[i] = v[j];
+    }
+  }
+}
+
+__global__ void __launch_bounds__(kSmallThreads) k_sort_small_keys(const uint64_t* __restrict__ in,
+                                                                   uint64_t* __restrict__ out, uint32_t n,
+                                                                   uint32_t bits) {
+  using Sort = rocprim::block_radix_sort<uint64_t, kSmallThreads, kSmallItems>;
+  __shared__ typename Sort::storage_type tmp;
+  uint64_t k[kSmallItems];
+#pragma unroll
+  for (uint32_t j = 0; j < kSmallItems; ++j) {
+    const uint32_t i = threadIdx.x * kSmallItems + j;
+    k[j] = i < n ? in[i] : ~0ull;
+  }
+  Sort().sort_to_striped(k, tmp, 0, bits);
+#pragma unroll
+  for (uint32_t j = 0; j < kSmallItems; ++j) {
+    const uint32_t i = threadIdx.x + j * kSmallThreads;
+    if (i < n) out[i] = k[j];
+  }
+}
+
+// values null: the items' numbers
+template <typename Config, typename V>
+static void sort_pairs(tribit_ctx* ctx, const uint32_t* in, uint32_t* out, const V* vin, V* vout, uint64_t n,
+                       uint32_t bits) {
+  if (n <= kSmallSort) {
+    k_sort_small<uint32_t, V><<<1, kSmallThreads, 0, ctx->stream>>>(in, out, vin, vout, (uint32_t)n, bits);
+    return;
+  }
+  with_temp(ctx, [&](void* t, size_t& b) {
+    if (vin) return rocprim::radix_sort_pairs<Config>(t, b, in, out, vin, vout, (size_t)n, 0u, bits, ctx->stream);
+    return rocprim::radix_sort_pairs<Config>(t, b, in, out, rocprim::counting_iterator<V>(0), vout, (size_t)n, 0u,
+                                             bits, ctx->stream);
+  });
+}
+
+// row_ptr[n + 1], the exclusive scan of odeg[0, n], and, with sfx_ptr, that of the
+// in-degrees deg - odeg. Small n: a workgroup each in one launch.
+constexpr uint64_t kSmallScan = 32768;
+__global__ void __launch_bounds__(kSmallThreads) k_scan_small(const uint32_t* __restrict__ odeg,
+                                                              const uint32_t* __restrict__ deg, uint32_t n,
+                                                              uint32_t* __restrict__ row_ptr,
+                                                              uint32_t* __restrict__ sfx_ptr) {
+  using Scan = rocprim::block_scan<uint32_t, kSmallThreads>;
+  __shared__ typename Scan::storage_type tmp;
+  const bool in = blockIdx.x == 1;
+  uint32_t* out = in ? sfx_ptr : row_ptr;
+  uint32_t carry = 0;
+  for (uint32_t i0 = 0; i0 <= n; i0 += kSmallThreads * kSmallItems) {
+    uint32_t v[kSmallItems], total;
+#pragma unroll
+    for (uint32_t j = 0; j < kSmallItems; ++j) {
+      const uint32_t i = i0 + threadIdx.x * kSmallItems + j;
+      v[j] = i < n ? (in ? deg[i] - odeg[i] : odeg[i]) : 0u;
+    }
+    Scan().exclusive_scan(v, v, carry, total, tmp, rocprim::plus<uint32_t>());
+#pragma unroll
+    for (uint32_t j = 0; j < kSmallItems; ++j) {
+      const uint32_t i = i0 + threadIdx.x * kSmallItems + j;
+      if (i <= n) out[i] = v[j];
+    }
+    carry += total;
+    __syncthreads();
+  }
+}
+
+struct InDegree {
+  const uint32_t *deg, *odeg;
+  uint64_t n;
+  __host__ __device__ uint32_t operator()(uint64_t v) const { return v < n ? deg[v] - odeg[v] : 0u; }
+};
+
+static void scan_rows(tribit_ctx* ctx, const uint32_t* odeg, const uint32_t* deg, uint64_t n, uint32_t* row_ptr,
+                      uint32_t* sfx_ptr) {
+  hipStream_t s = ctx->stream;
+  if (n <= kSmallScan) {
+    k_scan_small<<<sfx_ptr ? 2 : 1, kSmallThreads, 0, s>>>(odeg, deg, (uint32_t)n, row_ptr, sfx_ptr);
+    return;
+  }
+  with_temp(ctx, [&](void* t, size_t& b) {
+    return rocprim::exclusive_scan(t, b, odeg, row_ptr, 0u, (size_t)(n + 1), rocprim::plus<uint32_t>(), s);
+  });
+  if (!sfx_ptr) return;
+  const auto indeg = rocprim::make_transform_iterator(rocprim::counting_iterator<uint64_t>(0), InDegree{deg, odeg, n});
+  with_temp(ctx, [&](void* t, size_t& b) {
+    return rocprim::exclusive_scan(t, b, indeg, sfx_ptr, 0u, (size_t)(n + 1), rocprim::plus<uint32_t>(), s);
+  });
+}
+
 static void sort_keys(tribit_ctx* ctx, const uint64_t* in, uint64_t* out, uint64_t nk, uint32_t end_bit) {
+  if (nk <= kSmallSort) {
+    if (nk) k_sort_small_keys<<<1, kSmallThreads, 0, ctx->stream>>>(in, out, (uint32_t)nk, end_bit);
+    return;
+  }
   with_temp(ctx, [&](void* t, size_t& b) {
     return rocprim::radix_sort_keys(t, b, in, out, (size_t)nk, 0u, end_bit, ctx->stream);
   });
@@ -760,93 +889,78 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
   labels.ctx = ctx;
   DevBuf<uint64_t> okeys;  // oriented arcs, packed (u << kb) | v
   okeys.ctx = ctx;
+  DevBuf<uint32_t> odeg(ctx, n + 1);
+  DevBuf<RowStats> st(ctx, 1);
+  DevBuf<uint64_t> w_sfx;
+  w_sfx.ctx = ctx;
+  if (relabel) w_sfx = DevBuf<uint64_t>(ctx, n);
+  const ZeroSpans zero{{odeg.p, reinterpret_cast<uint32_t*>(st.p), reinterpret_cast<uint32_t*>(w_sfx.p)},
+                       {n + 1, sizeof(RowStats) / 4, relabel ? 2 * n : 0}};
+  const unsigned orient_grid = grid_for(std::max(m, zero.most()), kBlock);
+  if (m) okeys = DevBuf<uint64_t>(ctx, m);
   if (relabel) {
-    DevBuf<uint32_t> ids(ctx, n), deg_sorted(ctx, n), lab(ctx, n);
+    DevBuf<uint32_t> deg_sorted(ctx, n), lab(ctx, n);
     labels = DevBuf<uint32_t>(ctx, n);
-    k_iota_u32<<<grid_for(n, kBlock), kBlock, 0, s>>>(ids.p, n);
     if (relabel == 2) {
       // octave classes: rank of (floor(log2(deg)), id); runs of consecutive
       // input ids with similar degrees (a block of a block model) stay runs
       DevBuf<uint32_t> cls(ctx, n);
       k_octave<<<grid_for(n, kBlock), kBlock, 0, s>>>(deg.p, n, cls.p);
-      with_temp(ctx, [&](void* t, size_t& b) {
-        return rocprim::radix_sort_pairs(t, b, cls.p, deg_sorted.p, ids.p, labels.p, (size_t)n, 0u, 6u, s);
-      });
+      sort_pairs<rocprim::default_config, uint32_t>(ctx, cls.p, deg_sorted.p, nullptr, labels.p, n, 6u);
       k_gather_u32<<<grid_for(n, kBlock), kBlock, 0, s>>>(deg.p, labels.p, n, deg_sorted.p);
     } else {
-      with_temp(ctx, [&](void* t, size_t& b) {
-        return rocprim::radix_sort_pairs<IdSortConfig>(t, b, deg.p, deg_sorted.p, ids.p, labels.p, (size_t)n, 0u,
-                                         bits_for(n), s);
-      });
+      sort_pairs<IdSortConfig, uint32_t>(ctx, deg.p, deg_sorted.p, nullptr, labels.p, n, bits_for(n));
     }
     std::swap(deg.p, deg_sorted.p);  // deg now indexed by internal id
     k_scatter_labels<<<grid_for(n, kBlock), kBlock, 0, s>>>(labels.p, n, lab.p);
-    if (m) {
-      okeys = DevBuf<uint64_t>(ctx, m);
-      k_orient_relabel<<<grid_for(m, kBlock), kBlock, 0, s>>>(uniq.p, m, lab.p, kb, okeys.p);
-    }
-  } else if (m) {
-    okeys = DevBuf<uint64_t>(ctx, m);
-    k_orient<<<grid_for(m, kBlock), kBlock, 0, s>>>(uniq.p, m, deg.p, kb, okeys.p);
+    k_orient_relabel<<<orient_grid, kBlock, 0, s>>>(uniq.p, m, lab.p, kb, okeys.p, zero);
+  } else {
+    k_orient<<<orient_grid, kBlock, 0, s>>>(uniq.p, m, deg.p, kb, okeys.p, zero);
   }
 
   // 4-6. sort the arcs by (u, v) into the CSR
+  const bool narrow = relabel && m && m < (1ull << 30);
   DevBuf<uint32_t> col(ctx, m ? m : 1);
   DevBuf<uint32_t> row_ptr(ctx, n + 1);
-  {
-    DevBuf<uint32_t> odeg(ctx, n + 1);
-    k_fill_u32<<<grid_for(n + 1, kBlock), kBlock, 0, s>>>(odeg.p, n + 1, 0u);
-    if (m) {
-      sort_keys(ctx, okeys.p, uniq.p, m, 2 * kb);
-      okeys.reset();
-      k_csr_split<<<grid_for(m, kBlock), kBlock, 0, s>>>(uniq.p, m, kb, col.p, odeg.p);
-    }
-    with_temp(ctx, [&](void* t, size_t& b) {
-      return rocprim::exclusive_scan(t, b, odeg.p, row_ptr.p, 0u, (size_t)(n + 1), rocprim::plus<uint32_t>(), s);
-    });
+  DevBuf<uint32_t> sfx_ptr;
+  DevBuf<uint32_t> col16;
+  sfx_ptr.ctx = ctx;
+  if (relabel) sfx_ptr = DevBuf<uint32_t>(ctx, n + 1);
+  if (narrow) col16 = DevBuf<uint32_t>(ctx, col16_ids(m) / 2);
+  if (m) {
+    sort_keys(ctx, okeys.p, uniq.p, m, 2 * kb);
+    okeys.reset();
+    k_csr_split<<<grid_for(m + 4, kBlock), kBlock, 0, s>>>(uniq.p, m, kb, col.p, reinterpret_cast<uint16_t*>(col16.p),
+                                                          odeg.p);
   }
+  scan_rows(ctx, odeg.p, deg.p, n, row_ptr.p, sfx_ptr.p);
 
-  // 7. totals (W+, active rows, largest outdeg) from the rows
-  DevBuf<RowStats> st(ctx, 1);
-  k_fill_u32<<<1, 64, 0, s>>>(reinterpret_cast<uint32_t*>(st.p), sizeof(RowStats) / 4, 0u);
-  k_row_flags<<<totals_grid(n), kBlock, 0, s>>>(row_ptr.p, deg.p, n, st.p);
-  const bool narrow = relabel && m && m < (1ull << 30);
+  // 7. totals (W+, active rows, largest outdeg) from the rows, and the rows' split positions
   DevBuf<uint32_t> rsplit;
   rsplit.ctx = ctx;
-  if (narrow) {
-    rsplit = DevBuf<uint32_t>(ctx, n);
-    k_row_split<<<grid_for(n, kBlock), kBlock, 0, s>>>(row_ptr.p, col.p, n, rsplit.p);
-  }
+  if (narrow) rsplit = DevBuf<uint32_t>(ctx, n);
+  k_rows<<<totals_grid(n), kBlock, 0, s>>>(row_ptr.p, deg.p, col.p, n, st.p, rsplit.p);
   RowStats hst;
-  TB_HIP(hipMemcpyAsync(&hst, st.p, sizeof(hst), hipMemcpyDeviceToHost, s));
 
   // 8. wedge ranges (relabelled graphs): in-arcs of every v, each with its
-  // suffix range; narrow ranges flagged, and col16 (the low 16 bits of every
-  // id, padded to whole dwords plus one) built for streaming them
+  // suffix range; narrow ranges flagged (streamed from col16)
   DevBuf<uint2> rng_sfx;
-  DevBuf<uint32_t> sfx_ptr;
-  DevBuf<uint64_t> w_sfx;
-  DevBuf<uint32_t> col16;
   DevBuf<uint8_t> sfx_dh;
   DevBuf<uint16_t> sfx_split;
-  rng_sfx.ctx = sfx_ptr.ctx = w_sfx.ctx = ctx;
+  rng_sfx.ctx = ctx;
   if (relabel) {
     rng_sfx = DevBuf<uint2>(ctx, m ? m : 1);
-    sfx_ptr = DevBuf<uint32_t>(ctx, n + 1);
-    w_sfx = DevBuf<uint64_t>(ctx, n);
     if (narrow) {
       sfx_dh = DevBuf<uint8_t>(ctx, m);
       sfx_split = DevBuf<uint16_t>(ctx, m);
     }
-    k_fill_u64<<<grid_for(n, kBlock), kBlock, 0, s>>>(reinterpret_cast<unsigned long long*>(w_sfx.p), n);
-    DevBuf<uint32_t> cnt(ctx, n + 1);
-    k_in_count<<<grid_for(n + 1, kBlock), kBlock, 0, s>>>(row_ptr.p, deg.p, n, cnt.p);
     if (m) {
       // no outdegree passes 2 sqrt(m): its vertices' degrees (octave ids: half of
       // them) are all at least as large. The real largest is asked for only when
       // that bound leaves the records too wide.
       ArcPack pack{kb, bits_for(m), bits_for((uint64_t)(2.0 * std::sqrt((double)m)) + 2), narrow};
       if (!pack.fits()) {
+        TB_HIP(hipMemcpyAsync(&hst, st.p, sizeof(hst), hipMemcpyDeviceToHost, s));
         ctx->sync();
         pack.lb = bits_for((uint64_t)hst.max_outdeg + 1);
       }
@@ -854,39 +968,23 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
         DevBuf<uint32_t> key(ctx, m), key_sorted(ctx, m);
         DevBuf<uint64_t> val(ctx, m), val_sorted(ctx, m);
         k_arc_pack<<<grid_for(m, kBlock), kBlock, 0, s>>>(uniq.p, m, pack, row_ptr.p, col.p, rsplit.p, key.p, val.p);
-        with_temp(ctx, [&](void* t, size_t& b) {
-          return rocprim::radix_sort_pairs<IdSortConfig>(t, b, key.p, key_sorted.p, val.p, val_sorted.p, (size_t)m,
-                                                         0u, kb, s);
-        });
+        sort_pairs<IdSortConfig, uint64_t>(ctx, key.p, key_sorted.p, val.p, val_sorted.p, m, kb);
         k_sfx_unpack<<<grid_for(m, kBlock), kBlock, 0, s>>>(key_sorted.p, val_sorted.p, m, pack, rng_sfx.p, sfx_dh.p,
                                                            sfx_split.p,
                                                            reinterpret_cast<unsigned long long*>(w_sfx.p));
       } else {
         DevBuf<uint2> arec(ctx, m);
         k_arc_rec<<<grid_for(m, kBlock), kBlock, 0, s>>>(uniq.p, m, kb, row_ptr.p, col.p, rsplit.p, narrow, arec.p);
-        DevBuf<uint32_t> arcs(ctx, m), head(ctx, m), arc_sorted(ctx, m);
-        k_iota_u32<<<grid_for(m, kBlock), kBlock, 0, s>>>(arcs.p, m);
-        with_temp(ctx, [&](void* t, size_t& b) {
-          return rocprim::radix_sort_pairs<IdSortConfig>(t, b, col.p, head.p, arcs.p, arc_sorted.p, (size_t)m, 0u,
-                                                         bits_for(n), s);
-        });
-        arcs.reset();
+        DevBuf<uint32_t> head(ctx, m), arc_sorted(ctx, m);
+        sort_pairs<IdSortConfig, uint32_t>(ctx, col.p, head.p, nullptr, arc_sorted.p, m, kb);
         k_sfx_fill<<<grid_for(m, kBlock), kBlock, 0, s>>>(head.p, arc_sorted.p, m, arec.p, rng_sfx.p, sfx_dh.p,
                                                           sfx_split.p,
                                                           reinterpret_cast<unsigned long long*>(w_sfx.p));
       }
     }
-    with_temp(ctx, [&](void* t, size_t& b) {
-      return rocprim::exclusive_scan(t, b, cnt.p, sfx_ptr.p, 0u, (size_t)(n + 1), rocprim::plus<uint32_t>(), s);
-    });
-    uniq.reset();
-    if (narrow) {
-      const uint64_t words = (m + 1) / 2 + 1;
-      col16 = DevBuf<uint32_t>(ctx, words);
-      k_fill_u32<<<1, 64, 0, s>>>(col16.p + words - 2, 2, 0u);
-      k_col16<<<grid_for(m, kBlock), kBlock, 0, s>>>(col.p, m, reinterpret_cast<uint16_t*>(col16.p));
-    }
   }
+  uniq.reset();
+  TB_HIP(hipMemcpyAsync(&hst, st.p, sizeof(hst), hipMemcpyDeviceToHost, s));
 
   // the graph owns its buffers from here on (freed by tribit_graph_free, also on error)
   g->row_ptr = row_ptr.release();
@@ -1095,7 +1193,7 @@ void build_offdiag(tribit_ctx* ctx, const uint64_t* d_cols, uint64_t ncols, cons
   {
     DevBuf<uint32_t> odeg(ctx, n + 1);
     k_fill_u32<<<grid_for(n + 1, kBlock), kBlock, 0, s>>>(odeg.p, n + 1, 0u);
-    if (mh) k_csr_split<<<grid_for(mh, kBlock), kBlock, 0, s>>>(hk.p, mh, 32, col.p, odeg.p);
+    if (mh) k_csr_split<<<grid_for(mh, kBlock), kBlock, 0, s>>>(hk.p, mh, 32, col.p, nullptr, odeg.p);
     with_temp(ctx, [&](void* t, size_t& b) {
       return rocprim::exclusive_scan(t, b, odeg.p, row_ptr.p, 0u, (size_t)(n + 1), rocprim::plus<uint32_t>(), s);
     });
@@ -1153,7 +1251,7 @@ void build_offdiag(tribit_ctx* ctx, const uint64_t* d_cols, uint64_t ncols, cons
   k_fill_u32<<<1, 64, 0, s>>>(reinterpret_cast<uint32_t*>(st.p), sizeof(RowStats) / 4, 0u);
   k_sum_u64<<<totals_grid(n), kBlock, 0, s>>>(reinterpret_cast<const unsigned long long*>(w_rv.p), n,
                                               &st.p->wplus);
-  k_row_flags<<<totals_grid(n), kBlock, 0, s>>>(row_ptr.p, nullptr, n, st.p);
+  k_rows<<<totals_grid(n), kBlock, 0, s>>>(row_ptr.p, nullptr, nullptr, n, st.p, nullptr);
   RowStats hst;
   TB_HIP(hipMemcpyAsync(&hst, st.p, sizeof(hst), hipMemcpyDeviceToHost, s));
   ctx->sync();
