@@ -88,6 +88,7 @@ int tribit_init(int device, tribit_ctx** out) {
     TB_HIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
     ctx->pool.init(ctx->stream, prop.totalGlobalMem / 4);  // freed memory stays with the context (tribit.cu:829-830)
     for (auto& e : ctx->ev) TB_HIP(hipEventCreate(&e));
+    TB_HIP(hipHostMalloc(&ctx->readback, tribit_ctx::kReadback, hipHostMallocDefault));
     tb::noalloc_init(ctx);  // the device is current: its copy of the scratch array
   });
   if (st != TRIBIT_OK) {
@@ -106,6 +107,7 @@ int tribit_shutdown(tribit_ctx* ctx) {
   (void)hipStreamSynchronize(ctx->stream);
   for (auto& e : ctx->ev)
     if (e) (void)hipEventDestroy(e);
+  if (ctx->readback) (void)hipHostFree(ctx->readback);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
   return TRIBIT_OK;

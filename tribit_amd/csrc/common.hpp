@@ -80,6 +80,10 @@ struct tribit_ctx {
   // device address of the no-allocation count's scratch array on this
   // context's device (count.hip; looked up once at tribit_init)
   void* noalloc_scratch = nullptr;
+  // pinned host memory for the small read-backs of a count (kReadback bytes):
+  // copies into pageable memory go through a staging buffer and wait
+  void* readback = nullptr;
+  static constexpr size_t kReadback = 4096;
   std::string last_error;
 
   void* alloc(uint64_t bytes) {
@@ -200,6 +204,8 @@ struct tribit_graph {
   uint32_t* core_bits = nullptr;  // kp rows of kp / 32 words
   uint64_t core_c = 0, core_kp = 0;
   uint32_t core_e0 = 0;    // row_ptr[n - core_c]: first arc of the core's rows
+  // sum of outdeg (outdeg - 1) / 2 over the k-th kCoreStep ids from the top (relabelled graphs)
+  uint64_t core_wedges[16] = {};
   int64_t core_pick = -1;  // the learned schedule's core size from core_choose (-1: not chosen yet)
   // dense diagonal blocks (dense.hip): id ranges [s, e) whose induced subgraph
   // is dense, counted on the matrix cores; found on first use
@@ -279,6 +285,7 @@ struct tribit_batch {
 };
 
 namespace tb {
+constexpr uint64_t kCoreStep = 4096;  // core sizes are multiples of this, up to 16 of them
 // prep.hip
 // relabel: a TRIBIT_OPT_RELABEL mode, or -1 for the context's option.
 void preprocess(tribit_ctx* ctx, uint64_t* d_keys, uint64_t nkeys, uint64_t n, tribit_graph* g, int relabel = -1);
@@ -354,7 +361,7 @@ void mlp_infer_dev(tribit_mlp* m, const float* dX, uint64_t n, float* dout);
 void core_prepare(tribit_ctx* ctx, tribit_graph* g, uint64_t c);
 void core_release(tribit_graph* g);
 void core_launch(tribit_ctx* ctx, const tribit_graph* g, unsigned long long* result);
-uint64_t core_choose(tribit_ctx* ctx, const tribit_graph* g);
+uint64_t core_choose(const tribit_graph* g);
 double core_macs(uint64_t kp, uint64_t tile);
 bool blocks_prepare(tribit_ctx* ctx, tribit_graph* g);  // false: no dense block found
 void blocks_release(tribit_graph* g);

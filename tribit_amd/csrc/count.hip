@@ -1262,10 +1262,17 @@ struct SchedView {
   uint32_t core_cut;       // entries sorted by source: kept iff rng.x < core_cut
 };
 
+// A plan as a kernel argument, its bucket -> slot table copied into LDS by the
+// kernels that look buckets up.
 struct PlanDev {
   int kind[kSlots];
-  const uint8_t* table;  // bucket -> slot
+  uint8_t table[kBuckets];
 };
+static_assert(kBuckets % 4 == 0, "the table is copied as words");
+__device__ __forceinline__ void load_table(const PlanDev& pd, uint8_t* s_table) {
+  for (uint32_t i = threadIdx.x; i < kBuckets / 4; i += blockDim.x)
+    reinterpret_cast<uint32_t*>(s_table)[i] = reinterpret_cast<const uint32_t*>(pd.table)[i];
+}
 
 struct Cnt8 {
   uint32_t v[kSlots];
@@ -1343,7 +1350,8 @@ __device__ __forceinline__ uint32_t list_chunks(int kind, uint32_t d, bool curso
 
 // Per owner: tasks per slot.
 // Tasks of owner x per slot.
-__device__ __forceinline__ Cnt8 owner_counts(const SchedView& sv, const PlanDev& pd, uint64_t x) {
+__device__ __forceinline__ Cnt8 owner_counts(const SchedView& sv, const PlanDev& pd, const uint8_t* table,
+                                             uint64_t x) {
   Cnt8 c;
   for (int i = 0; i < kSlots; ++i) c.v[i] = 0;
   const uint32_t d = sv.row_ptr[x + 1] - sv.row_ptr[x];
@@ -1352,7 +1360,7 @@ __device__ __forceinline__ Cnt8 owner_counts(const SchedView& sv, const PlanDev&
     uint64_t w;
     owner_list(sv, x, l, &b, &k, &w);
     if (!list_useful(sv, l, d, k)) continue;
-    const int s = pd.table[bucket_of(d, w, k)];
+    const int s = table[bucket_of(d, w, k)];
     const int kind = pd.kind[s];
     const bool cur = cursor_list(kind, d, sv.layout);
     c.v[s] += list_splits(kind, k, w, cur) * list_chunks(kind, d, cur);
@@ -1367,14 +1375,19 @@ __device__ __forceinline__ Cnt8 owner_counts(const SchedView& sv, const PlanDev&
 // per-block sums go through HBM.
 constexpr unsigned kSchedBlock = 256;
 
+// Also zeroes the count's counters (nzero words), when given.
 __global__ __launch_bounds__(kSchedBlock) void k_sched_count(SchedView sv, PlanDev pd, uint64_t n,
-                                                             Cnt8* __restrict__ blocksum) {
+                                                             Cnt8* __restrict__ blocksum,
+                                                             unsigned long long* __restrict__ zero, uint32_t nzero) {
   __shared__ uint32_t sc[kSlots];
+  __shared__ __attribute__((aligned(4))) uint8_t s_table[kBuckets];
+  load_table(pd, s_table);
   if (threadIdx.x < kSlots) sc[threadIdx.x] = 0;
   __syncthreads();
   const uint64_t x = (uint64_t)blockIdx.x * kSchedBlock + threadIdx.x;
+  for (uint64_t i = x; i < nzero; i += (uint64_t)gridDim.x * kSchedBlock) zero[i] = 0ull;
   if (x < n) {
-    const Cnt8 c = owner_counts(sv, pd, x);
+    const Cnt8 c = owner_counts(sv, pd, s_table, x);
     for (int i = 0; i < kSlots; ++i)
       if (c.v[i]) atomicAdd(&sc[i], c.v[i]);
   }
@@ -1388,6 +1401,8 @@ __global__ __launch_bounds__(kSchedBlock) void k_sched_fill(SchedView sv, PlanDe
                                                             const Cnt8* __restrict__ blockoff, Cnt8 base,
                                                             uint4* __restrict__ tasks) {
   __shared__ uint32_t sc[kSlots];
+  __shared__ __attribute__((aligned(4))) uint8_t s_table[kBuckets];
+  load_table(pd, s_table);
   if (threadIdx.x < kSlots) sc[threadIdx.x] = 0;
   __syncthreads();
   const uint64_t x = (uint64_t)blockIdx.x * kSchedBlock + threadIdx.x;
@@ -1399,7 +1414,7 @@ __global__ __launch_bounds__(kSchedBlock) void k_sched_fill(SchedView sv, PlanDe
     owner_list(sv, x, l, &b, &k, &w);
     if (!list_useful(sv, l, d, k)) continue;
     const uint32_t bucket = (uint32_t)bucket_of(d, w, k);
-    const int s = pd.table[bucket];
+    const int s = s_table[bucket];
     const int kind = pd.kind[s];
     const bool cur = cursor_list(kind, d, sv.layout);
     const uint32_t sp = list_splits(kind, k, w, cur), nch = list_chunks(kind, d, cur);
@@ -1412,6 +1427,52 @@ __global__ __launch_bounds__(kSchedBlock) void k_sched_fill(SchedView sv, PlanDe
         out[j++] = make_uint4((uint32_t)x, b + k0, q + (i < r ? 1u : 0u),
                               (cur ? kAllChunks : c) | (bucket << kBucketShift));
       }
+  }
+}
+
+// Exclusive scan of the per-block counts cnt[0, nb] (entry nb is zero) by one
+// workgroup, the totals also into pinned host memory: one launch and no copy
+// where a device-wide scan and a read-back of the last entry took three. From
+// kScanBlocks blocks (524K owners, two trips of this loop) the device-wide scan.
+constexpr uint64_t kScanBlocks = 2048;
+constexpr uint32_t kScanThreads = 1024;
+__global__ __launch_bounds__(kScanThreads) void k_sched_scan(const Cnt8* __restrict__ cnt, Cnt8* __restrict__ off,
+                                                             uint32_t nb, Cnt8* __restrict__ host_tot) {
+  __shared__ uint32_t s_w[kScanThreads / 64][kSlots];
+  const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  uint32_t carry[kSlots] = {};
+  for (uint32_t i0 = 0; i0 <= nb; i0 += kScanThreads) {
+    const uint32_t i = i0 + threadIdx.x;
+    Cnt8 c, inc;
+    for (int k = 0; k < kSlots; ++k) c.v[k] = 0u;
+    if (i < nb) c = cnt[i];
+    inc = c;
+#pragma unroll
+    for (int k = 0; k < kSlots; ++k) {
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t t = __shfl_up(inc.v[k], o);
+        if (lane >= (uint32_t)o) inc.v[k] += t;
+      }
+      if (lane == 63) s_w[wv][k] = inc.v[k];
+    }
+    __syncthreads();
+    Cnt8 e;
+#pragma unroll
+    for (int k = 0; k < kSlots; ++k) {
+      uint32_t before = carry[k], total = 0;
+#pragma unroll
+      for (uint32_t q = 0; q < kScanThreads / 64; ++q) {
+        const uint32_t t = s_w[q][k];
+        before += q < wv ? t : 0u;
+        total += t;
+      }
+      e.v[k] = before + inc.v[k] - c.v[k];
+      carry[k] += total;
+    }
+    if (i <= nb) off[i] = e;
+    if (i == nb) *host_tot = e;
+    __syncthreads();
   }
 }
 
@@ -1561,14 +1622,6 @@ __global__ __launch_bounds__(256) void k_tdur_reduce(const uint4* __restrict__ t
 __global__ void k_zero_u64(unsigned long long* p, uint32_t n) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0ull;
-}
-
-// A plan's bucket -> slot table, passed by value as a kernel argument.
-struct PlanTable {
-  uint8_t t[kBuckets];
-};
-__global__ void k_put_table(PlanTable pt, uint8_t* out) {
-  for (uint32_t i = threadIdx.x; i < (uint32_t)kBuckets; i += blockDim.x) out[i] = pt.t[i];
 }
 
 // With `blocks` (wedge layout, dense diagonal blocks on the matrix cores) the
@@ -2120,9 +2173,9 @@ static T* scratch_buf(tribit_ctx* ctx, Arena* arena, DevBuf<T>& own, uint64_t co
 // Resolves the plan (learned table, tile opt-in/out) and builds the task
 // lists (one host sync for the per-slot totals). With `arena`, every device
 // buffer comes from it (the caller rules out what would allocate: learned
-// tables, tiles, a dense core).
+// tables, tiles, a dense core). zero: words the first launch clears.
 void make_schedule(tribit_ctx* ctx, tribit_graph* g, int layout, int flags, bool learned, Schedule& S,
-                   uint64_t core_c, Arena* arena = nullptr) {
+                   uint64_t core_c, Arena* arena = nullptr, unsigned long long* zero = nullptr, uint32_t nzero = 0) {
   hipStream_t s = ctx->stream;
   const uint64_t n = g->n;
   Plan& plan = S.plan;
@@ -2162,16 +2215,9 @@ void make_schedule(tribit_ctx* ctx, tribit_graph* g, int layout, int flags, bool
     if ((flags & TRIBIT_COUNT_FORCE_TILES) && plan.kind[i] == kKindBlock) plan.kind[i] = kKindTile;
     if (((flags & TRIBIT_COUNT_NO_TILES) || S.blocks) && plan.kind[i] == kKindTile) plan.kind[i] = kKindBlock;
   }
-  DevBuf<uint8_t> dtable_own;
-  uint8_t* dtable = scratch_buf(ctx, arena, dtable_own, kBuckets);
-  {
-    PlanTable pt;
-    memcpy(pt.t, plan.table, kBuckets);
-    k_put_table<<<1, kBlock, 0, s>>>(pt, dtable);  // a kernel argument: no host staging
-  }
   PlanDev pd;
   for (int i = 0; i < kSlots; ++i) pd.kind[i] = i < plan.nslots ? plan.kind[i] : kKindBlock;
-  pd.table = dtable;
+  memcpy(pd.table, plan.table, kBuckets);
 
   // per-block task counts (block nb covers no owner: its sum is zero), scanned
   const uint64_t nb = (n + kSchedBlock - 1) / kSchedBlock;
@@ -2180,19 +2226,22 @@ void make_schedule(tribit_ctx* ctx, tribit_graph* g, int layout, int flags, bool
   Cnt8* off = scratch_buf(ctx, arena, off_own, nb + 1);
   const SchedView sv = sched_view(g, layout, core_d0, core_cut, S.blocks);
   S.rng = sched_ranges(g, layout, S.blocks);
-  k_sched_count<<<(unsigned)(nb + 1), kSchedBlock, 0, s>>>(sv, pd, n, cnt);
-  {
-    Cnt8 zero;
-    for (int i = 0; i < kSlots; ++i) zero.v[i] = 0;
+  k_sched_count<<<(unsigned)(nb + 1), kSchedBlock, 0, s>>>(sv, pd, n, cnt, zero, nzero);
+  Cnt8* tot = static_cast<Cnt8*>(ctx->readback);
+  if (nb < kScanBlocks) {
+    k_sched_scan<<<1, kScanThreads, 0, s>>>(cnt, off, (uint32_t)nb, tot);
+  } else {
+    Cnt8 none;
+    for (int i = 0; i < kSlots; ++i) none.v[i] = 0;
     size_t bytes = 0;
-    TB_HIP(rocprim::exclusive_scan(nullptr, bytes, cnt, off, zero, (size_t)(nb + 1), Cnt8Plus(), s));
+    TB_HIP(rocprim::exclusive_scan(nullptr, bytes, cnt, off, none, (size_t)(nb + 1), Cnt8Plus(), s));
     DevBuf<uint8_t> tmp_own;
     uint8_t* tmp = scratch_buf(ctx, arena, tmp_own, bytes ? bytes : 8);
-    TB_HIP(rocprim::exclusive_scan(tmp, bytes, cnt, off, zero, (size_t)(nb + 1), Cnt8Plus(), s));
+    TB_HIP(rocprim::exclusive_scan(tmp, bytes, cnt, off, none, (size_t)(nb + 1), Cnt8Plus(), s));
+    TB_HIP(hipMemcpyAsync(tot, off + nb, sizeof(Cnt8), hipMemcpyDeviceToHost, s));  // the totals
   }
-  // off[nb] = totals
-  TB_HIP(hipMemcpyAsync(&S.tot, off + nb, sizeof(Cnt8), hipMemcpyDeviceToHost, s));
   ctx->sync();
+  S.tot = *tot;
   S.ntask = 0;
   for (int i = 0; i < kSlots; ++i) {
     S.base.v[i] = (uint32_t)S.ntask;
@@ -2241,7 +2290,8 @@ void make_schedule(tribit_ctx* ctx, tribit_graph* g, int layout, int flags, bool
 
 // The counting launches of a schedule (capturable: no allocation, no sync).
 // The caller zeroes a.result and a.queue. With `ev`, an event is recorded
-// after each slot's launch (ev[i] for slot i).
+// after each slot's launch (ev[i] for slot i; none for a slot without tasks: a
+// recorded event delays the next launch by 3 to 4 us).
 void launch_schedule(tribit_ctx* ctx, tribit_graph* g, const Schedule& S, const LaunchArgs& a, hipEvent_t* ev,
                      uint64_t* blocks) {
   hipStream_t s = ctx->stream;
@@ -2250,6 +2300,7 @@ void launch_schedule(tribit_ctx* ctx, tribit_graph* g, const Schedule& S, const 
   for (int i = 0; i < plan.nslots; ++i) {
     const uint4* tk = S.tasks.p + S.base.v[i];
     const uint32_t nt = S.tot.v[i];
+    if (!nt) continue;
     if (plan.kind[i] == kKindWave64)
       launch_wave<kC0Logs, kC0K>(a, i, plan.g[i], nt, cus, s, g, S.rng, tk, blocks);
     else if (plan.kind[i] == kKindWaveMulti)
@@ -2288,9 +2339,8 @@ static uint64_t count_once(tribit_ctx* ctx, tribit_graph* g, int sched, int flag
   DevBuf<unsigned long long> counters_own;
   // counters first: an arena that is too small for the tasks fails before any launch
   unsigned long long* counters = scratch_buf(ctx, arena, counters_own, kCountScratch);
-  make_schedule(ctx, g, sched, flags, learned, S, core_c, arena);
+  make_schedule(ctx, g, sched, flags, learned, S, core_c, arena, counters, kCountScratch);
   plan = S.plan;
-  k_zero_u64<<<grid_for(kCountScratch, kBlock), kBlock, 0, s>>>(counters, kCountScratch);
   LaunchArgs a;
   a.att = mode_word(flags);
   a.result = counters;
@@ -2304,25 +2354,32 @@ static uint64_t count_once(tribit_ctx* ctx, tribit_graph* g, int sched, int flag
   TB_HIP(hipEventRecord(ctx->ev[3], s));
   uint64_t blocks = 0;
   launch_schedule(ctx, g, S, a, ctx->ev + 4, &blocks);
-  hipEvent_t last = ctx->ev[3 + plan.nslots + (S.core_c ? 1 : 0) + (S.blocks ? 1 : 0)];
+  // the event after each slot (the one before it for a slot without tasks), the core and the blocks
+  hipEvent_t after[kSlots + 1];
+  hipEvent_t last = ctx->ev[3];
+  for (int v = 0; v < plan.nslots; ++v) after[v] = last = S.tot.v[v] ? ctx->ev[4 + v] : last;
+  const hipEvent_t sparse = last;
+  if (S.core_c || S.blocks) last = ctx->ev[3 + plan.nslots + (S.core_c ? 1 : 0) + (S.blocks ? 1 : 0)];
   if (tlog)
     for (int v = 0; v < plan.nslots; ++v)
       if (S.tot.v[v])
         k_tdur_reduce<<<(unsigned)std::min<uint64_t>((S.tot.v[v] + 255) / 256, 1024), 256, 0, s>>>(
             S.tasks.p + S.base.v[v], tdur.p + S.base.v[v], S.tot.v[v], tlog + (size_t)v * kBuckets);
-  unsigned long long slots[kQueueOff], res[2] = {0, 0};
-  TB_HIP(hipMemcpyAsync(slots, a.result, sizeof(slots), hipMemcpyDeviceToHost, s));
-  TB_HIP(hipEventSynchronize(last));
+  static_assert(kQueueOff * 8 <= tribit_ctx::kReadback, "result slots");
+  const unsigned long long* slots = static_cast<const unsigned long long*>(ctx->readback);
+  unsigned long long res[2] = {0, 0};
+  TB_HIP(hipMemcpyAsync(ctx->readback, a.result, kQueueOff * 8, hipMemcpyDeviceToHost, s));
   ctx->sync();
   for (uint32_t i = 0; i < kResults; ++i) {
     res[0] += slots[i * kResultStride];
     res[1] += slots[i * kResultStride + 1];
   }
   *ms_sched = elapsed(ctx->ev[2], ctx->ev[3]);
-  *ms_kernel = elapsed(ctx->ev[3], last);
+  *ms_kernel = last == ctx->ev[3] ? 0.0 : elapsed(ctx->ev[3], last);
   *ms_total = elapsed(ctx->ev[2], last);
-  for (int v = 0; v < plan.nslots; ++v) ms_var[v] = elapsed(ctx->ev[3 + v], ctx->ev[4 + v]);
-  if (ms_core) *ms_core = (S.core_c || S.blocks) ? elapsed(ctx->ev[3 + plan.nslots], last) : 0.0;
+  for (int v = 0; v < plan.nslots; ++v)
+    ms_var[v] = S.tot.v[v] ? elapsed(v ? after[v - 1] : ctx->ev[3], after[v]) : 0.0;
+  if (ms_core) *ms_core = (S.core_c || S.blocks) ? elapsed(sparse, last) : 0.0;
   if (info) {
     info->launch_blocks = blocks;
     info->tasks = S.ntask;
@@ -2386,7 +2443,7 @@ static bool candidate(tribit_ctx* ctx, tribit_graph* g, const tribit_count_opts&
   if (opts.dense_core > 0)
     core = std::min<uint64_t>((uint64_t)opts.dense_core, g->n);
   else if (opts.dense_core == 0 && g->relabeled) {
-    if (g->core_pick < 0) g->core_pick = (int64_t)core_choose(ctx, g);  // the graph does not change
+    if (g->core_pick < 0) g->core_pick = (int64_t)core_choose(g);  // the graph does not change
     core = (uint64_t)g->core_pick;
   }
   int dummy = 0;

@@ -376,20 +376,14 @@ static double kCoreMacPerMs = 1.3e12;
 // measured figures on MI355X (streaming kernels ~2e12 wedge checks/s, the
 // core kernel ~1.3e15 int8 MAC/s including its staging: 7.7e11 MACs in
 // 0.57 ms for 16,384 ids).
-uint64_t core_choose(tribit_ctx* ctx, const tribit_graph* g) {
+uint64_t core_choose(const tribit_graph* g) {
   if (!g->relabeled || g->n < 4096 || !g->m) return 0;
-  const uint64_t top = std::min<uint64_t>(g->n, 65536);
-  std::vector<uint32_t> rp(top + 1);
-  TB_HIP(hipMemcpyAsync(rp.data(), g->row_ptr + (g->n - top), 4 * (top + 1), hipMemcpyDeviceToHost, ctx->stream));
-  ctx->sync();
+  const uint64_t top = std::min<uint64_t>(g->n, 16 * kCoreStep);
   uint64_t best = 0;
   double best_gain = 0.5;
-  double wedges = 0.0;  // of the top c ids, grown 4,096 ids at a time
-  for (uint64_t c = 4096; c <= top; c += 4096) {
-    for (uint64_t i = top - c; i < top - c + 4096; ++i) {
-      const double d = (double)(rp[i + 1] - rp[i]);
-      wedges += d * (d - 1.0) * 0.5;
-    }
+  double wedges = 0.0;  // of the top c ids
+  for (uint64_t c = kCoreStep; c <= top; c += kCoreStep) {
+    wedges += (double)g->core_wedges[c / kCoreStep - 1];
     const uint64_t kp = (c + kCoreTile2 - 1) / kCoreTile2 * kCoreTile2;
     const double sparse_ms = wedges / 2.0e9;
     const double dense_ms = core_macs(kp, kCoreTile2) / kCoreMacPerMs;

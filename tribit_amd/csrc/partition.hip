@@ -407,6 +407,25 @@ __global__ void k_deg_direct(const uint64_t* __restrict__ keys, uint64_t m, uint
   atomicAdd(&deg[(uint32_t)(k & ((1ull << kb) - 1))], 1u);
 }
 
+// Few edges over ids that fit LDS: every block counts its share there and adds
+// it once (80K edges of an R-MAT graph, whose hubs' atomics queue up: 45 us with
+// an atomic per endpoint).
+__global__ void __launch_bounds__(kEndThreads) k_deg_lds(const uint64_t* __restrict__ keys, uint32_t m, uint32_t kb,
+                                                         uint32_t n, uint32_t* __restrict__ deg) {
+  __shared__ uint32_t s_c[kEndCounters];
+  for (uint32_t i = threadIdx.x; i < n; i += kEndThreads) s_c[i] = 0u;
+  __syncthreads();
+  const uint64_t lo = (1ull << kb) - 1;
+  for (uint32_t i = blockIdx.x * kEndThreads + threadIdx.x; i < m; i += gridDim.x * kEndThreads) {
+    const uint64_t k = keys[i];
+    atomicAdd(&s_c[(uint32_t)(k >> kb)], 1u);
+    atomicAdd(&s_c[(uint32_t)(k & lo)], 1u);
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < n; i += kEndThreads)
+    if (s_c[i]) atomicAdd(&deg[i], s_c[i]);
+}
+
 __global__ void __launch_bounds__(kPartThreads) k_ends_hist(const uint64_t* __restrict__ keys, uint64_t m, uint32_t kb,
                                                             uint32_t g0, uint32_t groups,
                                                             uint32_t* __restrict__ hist) {
@@ -561,6 +580,11 @@ void count_degrees(tribit_ctx* ctx, const uint64_t* keys, uint64_t m, uint64_t n
   hipStream_t s = ctx->stream;
   k_part_zero<<<grid_for(n, kBlock), kBlock, 0, s>>>(deg, n);
   if (!m) return;
+  if (m <= kDirectEdges && n <= kEndCounters) {
+    k_deg_lds<<<std::min<uint32_t>(64, grid_for(m, 4 * kEndThreads)), kEndThreads, 0, s>>>(keys, (uint32_t)m, kb,
+                                                                                          (uint32_t)n, deg);
+    return;
+  }
   if (m <= kDirectEdges || m > 0x7FFFFFFFull) {  // 32-bit cursors over 2 m endpoints
     k_deg_direct<<<grid_for(m, kBlock), kBlock, 0, s>>>(keys, m, kb, deg);
     return;

@@ -235,6 +235,7 @@ struct RowStats {
   unsigned long long rows_active;
   unsigned int max_outdeg;
   unsigned int pad;
+  unsigned long long core_wedges[16];  // tribit_graph.core_wedges
 };
 
 // Totals over a bounded grid (grid-stride loops, one atomic per block and
@@ -320,16 +321,30 @@ int auto_relabel(uint64_t n, uint64_t band_edges) {
 // N+(v) once, and v has deg(v) - outdeg(v) in-arcs. With split (relabelled
 // graphs), also per row the position where its last 64K-id window begins (the
 // first id whose high 16 bits equal the last id's), for the narrow records of its
-// wedge ranges: one lower-bound search per row.
+// wedge ranges: one lower-bound search per row. With wedges, the top ids' wedges
+// by steps of kCoreStep ids, from which the core size is chosen.
 __global__ void __launch_bounds__(kBlock) k_rows(const uint32_t* __restrict__ row_ptr,
                                                  const uint32_t* __restrict__ deg, const uint32_t* __restrict__ col,
-                                                 uint64_t n, RowStats* __restrict__ st, uint32_t* __restrict__ split) {
+                                                 uint64_t n, RowStats* __restrict__ st, uint32_t* __restrict__ split,
+                                                 bool wedges) {
   __shared__ unsigned long long s_act[kBlock / 64], s_w[kBlock / 64];
   __shared__ uint32_t s_max[kBlock / 64];
   uint64_t act = 0, w = 0;
   uint32_t dm = 0;
   for (uint64_t u = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; u < n; u += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t b = row_ptr[u], e = row_ptr[u + 1], d = e - b;
+    // wedges of the top ids: a wave's rows are neighbours, of one step or two
+    if (wedges && n - u <= 16 * kCoreStep) {
+      const uint32_t k = (uint32_t)((n - 1 - u) / kCoreStep);
+      const uint64_t c = (uint64_t)d * (d ? d - 1 : 0) / 2, live = __ballot(true);
+      const uint32_t k0 = __builtin_amdgcn_readfirstlane(k);
+      if (__ballot(k == k0) == live && live == ~0ull) {
+        const uint64_t sum = wave_sum_u64(c);
+        if (lane_id() == 0 && sum) atomicAdd(&st->core_wedges[k], (unsigned long long)sum);
+      } else if (c) {
+        atomicAdd(&st->core_wedges[k], (unsigned long long)c);
+      }
+    }
     act += d >= 2;
     dm = d > dm ? d : dm;
     if (deg) w += (uint64_t)(deg[u] - d) * d;
@@ -939,7 +954,7 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
   DevBuf<uint32_t> rsplit;
   rsplit.ctx = ctx;
   if (narrow) rsplit = DevBuf<uint32_t>(ctx, n);
-  k_rows<<<totals_grid(n), kBlock, 0, s>>>(row_ptr.p, deg.p, col.p, n, st.p, rsplit.p);
+  k_rows<<<totals_grid(n), kBlock, 0, s>>>(row_ptr.p, deg.p, col.p, n, st.p, rsplit.p, relabel != 0);
   RowStats hst;
 
   // 8. wedge ranges (relabelled graphs): in-arcs of every v, each with its
@@ -1011,6 +1026,7 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
   g->wplus = hst.wplus;
   g->rows_active = hst.rows_active;
   g->max_outdeg = hst.max_outdeg;
+  for (int k = 0; k < 16; ++k) g->core_wedges[k] = hst.core_wedges[k];
 }
 
 // ------------------------------------------------------------ range layouts
@@ -1251,7 +1267,7 @@ void build_offdiag(tribit_ctx* ctx, const uint64_t* d_cols, uint64_t ncols, cons
   k_fill_u32<<<1, 64, 0, s>>>(reinterpret_cast<uint32_t*>(st.p), sizeof(RowStats) / 4, 0u);
   k_sum_u64<<<totals_grid(n), kBlock, 0, s>>>(reinterpret_cast<const unsigned long long*>(w_rv.p), n,
                                               &st.p->wplus);
-  k_rows<<<totals_grid(n), kBlock, 0, s>>>(row_ptr.p, nullptr, nullptr, n, st.p, nullptr);
+  k_rows<<<totals_grid(n), kBlock, 0, s>>>(row_ptr.p, nullptr, nullptr, n, st.p, nullptr, false);
   RowStats hst;
   TB_HIP(hipMemcpyAsync(&hst, st.p, sizeof(hst), hipMemcpyDeviceToHost, s));
   ctx->sync();
