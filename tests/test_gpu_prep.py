@@ -116,3 +116,38 @@ def test_wedge_records(gpu_ctx, oracle_mod, n, hubs, leaves, extra):
             assert g.count("wedge", dense_core=core).triangles == want, core
         assert g.count("wedge", flags=tribit_amd.WIDE_IDS).triangles == want
         assert sum(g.variant_stats("wedge")["edges"]) <= k.size
+
+
+# m edges around the smallest graph whose rows are partitioned and around the second pass (2 m = 512 quanta of rows),
+# and a clique: full slots (rows below 4096 arcs) and rows longer than a slot
+@pytest.mark.parametrize("n,m,clique", [(300, 8192, 0), (300, 8193, 0), (70000, 8193, 0), (5000, (1 << 20) - 1, 0),
+                                        (3000000, 1 << 20, 0), (200000, 1 << 21, 0), (9000, 20000, 1500),
+                                        (20000, 30000, 4000), (5000, 50000, 4096), (30000, 30000, 4300)])
+@pytest.mark.parametrize("relabel", [1, 2])
+def test_rows_by_partition(gpu_ctx, relabel, n, m, clique):
+    """The arcs of both relabelled id orders, each row's ids ascending, as a sort of the relabelled edges gives them."""
+    note(f"rows: {n} ids, {m} edges, clique of {clique}, id order {relabel}")
+    rng = np.random.default_rng(n + m + clique)
+    k = np.zeros(0, np.uint64)
+    while k.size < m:
+        a, b = rng.integers(0, n, (2, m))
+        x = ((np.minimum(a, b) << 32) | np.maximum(a, b))[a != b].astype(np.uint64)
+        k = np.unique(np.concatenate([k, x]))
+    k = rng.permutation(k)[:m]
+    ids = rng.choice(n, clique, replace=False)
+    i, j = np.triu_indices(clique, 1)
+    k = np.unique(np.concatenate([k, ((np.minimum(ids[i], ids[j]) << 32) | np.maximum(ids[i], ids[j])).astype(np.uint64)]))
+    gpu_ctx.set_relabel(relabel)
+    try:
+        with gpu_ctx.graph_from_keys(k, n) as g:
+            order, _ = g.labels()
+            row_ptr, col, deg = g.download()
+    finally:
+        gpu_ctx.set_relabel("auto")
+    new = np.empty(n, np.int64)
+    new[order] = np.arange(n)
+    a, b = new[(k >> np.uint64(32)).astype(np.int64)], new[(k & np.uint64(0xFFFFFFFF)).astype(np.int64)]
+    arcs = np.sort((np.minimum(a, b) << 32) | np.maximum(a, b))
+    assert np.array_equal(row_ptr, np.searchsorted(arcs, np.arange(n + 1) << 32).astype(np.uint32))
+    assert np.array_equal(col, (arcs & 0xFFFFFFFF).astype(np.uint32))
+    assert np.array_equal(deg, np.bincount(np.concatenate([a, b]), minlength=n).astype(np.uint32))

@@ -305,6 +305,10 @@ void rmat_thresholds(double a, double b, double c, uint32_t t[3]);
 bool distinct_keys(tribit_ctx* ctx, const uint64_t* d_keys, uint64_t nk, uint64_t n, uint32_t kb, uint64_t* out,
                    uint64_t* m, bool* bad, uint64_t band_ids, uint64_t* band);
 void count_degrees(tribit_ctx* ctx, const uint64_t* keys, uint64_t m, uint64_t n, uint32_t kb, uint32_t* deg);
+// rows.hip
+constexpr uint64_t kRowsMaxEdges = 1ull << 29;  // build_rows takes fewer edges than this
+void build_rows(tribit_ctx* ctx, const uint64_t* edges, uint64_t m, const uint32_t* lab, const uint32_t* deg, uint64_t n,
+                uint32_t kb, uint64_t* arcs, uint32_t* col, uint16_t* col16, uint32_t* odeg, uint32_t* flag);
 // gen.hip
 uint64_t chung_lu_samples(uint64_t n, double avg_deg);
 void chung_lu_cdf(uint64_t n, double gamma, uint64_t* cdf);

@@ -13,7 +13,6 @@
 #include <cmath>
 #include <cstring>
 #include <rocprim/block/block_radix_sort.hpp>
-#include <rocprim/block/block_scan.hpp>
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 #include <rocprim/device/device_select.hpp>
@@ -22,13 +21,11 @@
 
 #include "common.hpp"
 #include "device.hpp"
+#include "zero.hpp"
 
 namespace tb {
 
 constexpr unsigned kBlock = 256;
-
-// Ids in col16: m rounded up to whole dwords, and one more dword.
-__host__ __device__ inline uint64_t col16_ids(uint64_t m) { return ((m + 1) / 2 + 1) * 2; }
 
 // ---------------------------------------------------------------- generators
 
@@ -172,22 +169,12 @@ __global__ void k_gather_u32(const uint32_t* __restrict__ src, const uint32_t* _
   if (i < n) out[i] = src[idx[i]];
 }
 
-__global__ void k_scatter_labels(const uint32_t* __restrict__ old_of_new, uint64_t n, uint32_t* __restrict__ lab) {
+__global__ void k_scatter_labels(const uint32_t* __restrict__ old_of_new, uint64_t n, uint32_t* __restrict__ lab,
+                                 ZeroSpans z) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  z.clear(i);
   if (i < n) lab[old_of_new[i]] = (uint32_t)i;
 }
-
-// Zeroed on the way by a kernel whose grid covers them: one launch fewer each.
-struct ZeroSpans {
-  uint32_t* p[3];
-  uint64_t n[3];
-  __device__ __forceinline__ void clear(uint64_t i) const {
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-      if (i < n[k]) p[k][i] = 0u;
-  }
-  uint64_t most() const { return std::max(n[0], std::max(n[1], n[2])); }
-};
 
 // Degree orientation: {a<b} becomes a->b iff deg(a) <= deg(b).
 __global__ void k_orient(const uint64_t* __restrict__ keys, uint64_t m, const uint32_t* __restrict__ deg,
@@ -234,7 +221,7 @@ struct RowStats {
   unsigned long long wplus;
   unsigned long long rows_active;
   unsigned int max_outdeg;
-  unsigned int pad;
+  unsigned int row_overflow;           // build_rows' flag
   unsigned long long core_wedges[16];  // tribit_graph.core_wedges
 };
 
@@ -725,47 +712,35 @@ static void sort_pairs(tribit_ctx* ctx, const uint32_t* in, uint32_t* out, const
   });
 }
 
-// row_ptr[n + 1], the exclusive scan of odeg[0, n], and, with sfx_ptr, that of the
-// in-degrees deg - odeg. Small n: a workgroup each in one launch.
-constexpr uint64_t kSmallScan = 32768;
-__global__ void __launch_bounds__(kSmallThreads) k_scan_small(const uint32_t* __restrict__ odeg,
-                                                              const uint32_t* __restrict__ deg, uint32_t n,
-                                                              uint32_t* __restrict__ row_ptr,
-                                                              uint32_t* __restrict__ sfx_ptr) {
-  using Scan = rocprim::block_scan<uint32_t, kSmallThreads>;
-  __shared__ typename Scan::storage_type tmp;
-  const bool in = blockIdx.x == 1;
-  uint32_t* out = in ? sfx_ptr : row_ptr;
-  uint32_t carry = 0;
-  for (uint32_t i0 = 0; i0 <= n; i0 += kSmallThreads * kSmallItems) {
-    uint32_t v[kSmallItems], total;
-#pragma unroll
-    for (uint32_t j = 0; j < kSmallItems; ++j) {
-      const uint32_t i = i0 + threadIdx.x * kSmallItems + j;
-      v[j] = i < n ? (in ? deg[i] - odeg[i] : odeg[i]) : 0u;
-    }
-    Scan().exclusive_scan(v, v, carry, total, tmp, rocprim::plus<uint32_t>());
-#pragma unroll
-    for (uint32_t j = 0; j < kSmallItems; ++j) {
-      const uint32_t i = i0 + threadIdx.x * kSmallItems + j;
-      if (i <= n) out[i] = v[j];
-    }
-    carry += total;
-    __syncthreads();
-  }
-}
-
 struct InDegree {
   const uint32_t *deg, *odeg;
   uint64_t n;
   __host__ __device__ uint32_t operator()(uint64_t v) const { return v < n ? deg[v] - odeg[v] : 0u; }
 };
 
+struct OutDegree {
+  const uint32_t* odeg;
+  __device__ uint32_t operator()(uint64_t v) const { return odeg[v]; }
+};
+
+// Both scans of scan_rows for small n: a workgroup each in one launch.
+__global__ void __launch_bounds__(kScanBlockThreads) k_scan_small(OutDegree f, InDegree g, uint32_t n,
+                                                                  uint32_t* __restrict__ row_ptr,
+                                                                  uint32_t* __restrict__ sfx_ptr) {
+  if (blockIdx.x == 0)
+    scan_block(f, n, row_ptr);
+  else
+    scan_block(g, n, sfx_ptr);
+}
+
+// row_ptr[n + 1], the exclusive scan of odeg[0, n], and, with sfx_ptr, that of the
+// in-degrees deg - odeg.
 static void scan_rows(tribit_ctx* ctx, const uint32_t* odeg, const uint32_t* deg, uint64_t n, uint32_t* row_ptr,
                       uint32_t* sfx_ptr) {
   hipStream_t s = ctx->stream;
   if (n <= kSmallScan) {
-    k_scan_small<<<sfx_ptr ? 2 : 1, kSmallThreads, 0, s>>>(odeg, deg, (uint32_t)n, row_ptr, sfx_ptr);
+    k_scan_small<<<sfx_ptr ? 2 : 1, kScanBlockThreads, 0, s>>>(OutDegree{odeg}, InDegree{deg, odeg, n}, (uint32_t)n,
+                                                              row_ptr, sfx_ptr);
     return;
   }
   with_temp(ctx, [&](void* t, size_t& b) {
@@ -911,8 +886,18 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
   if (relabel) w_sfx = DevBuf<uint64_t>(ctx, n);
   const ZeroSpans zero{{odeg.p, reinterpret_cast<uint32_t*>(st.p), reinterpret_cast<uint32_t*>(w_sfx.p)},
                        {n + 1, sizeof(RowStats) / 4, relabel ? 2 * n : 0}};
-  const unsigned orient_grid = grid_for(std::max(m, zero.most()), kBlock);
-  if (m) okeys = DevBuf<uint64_t>(ctx, m);
+  const ZeroSpans none{};
+  // 4-6. the arcs sorted by (u, v) into the CSR
+  const bool narrow = relabel && m && m < (1ull << 30);
+  DevBuf<uint32_t> col(ctx, m ? m : 1);
+  DevBuf<uint32_t> row_ptr(ctx, n + 1);
+  DevBuf<uint32_t> sfx_ptr;
+  DevBuf<uint32_t> col16;
+  sfx_ptr.ctx = ctx;
+  if (relabel) sfx_ptr = DevBuf<uint32_t>(ctx, n + 1);
+  if (narrow) col16 = DevBuf<uint32_t>(ctx, col16_ids(m) / 2);
+  uint16_t* ids16 = reinterpret_cast<uint16_t*>(col16.p);
+  bool sorted = false;
   if (relabel) {
     DevBuf<uint32_t> deg_sorted(ctx, n), lab(ctx, n);
     labels = DevBuf<uint32_t>(ctx, n);
@@ -927,26 +912,29 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
       sort_pairs<IdSortConfig, uint32_t>(ctx, deg.p, deg_sorted.p, nullptr, labels.p, n, bits_for(n));
     }
     std::swap(deg.p, deg_sorted.p);  // deg now indexed by internal id
-    k_scatter_labels<<<grid_for(n, kBlock), kBlock, 0, s>>>(labels.p, n, lab.p);
-    k_orient_relabel<<<orient_grid, kBlock, 0, s>>>(uniq.p, m, lab.p, kb, okeys.p, zero);
+    k_scatter_labels<<<grid_for(std::max(n, zero.most()), kBlock), kBlock, 0, s>>>(labels.p, n, lab.p, zero);
+    // rows by partition, but a sort by one workgroup where that suffices (two
+    // launches of 35 us against five of 31) and for more edges than the slots cover
+    if (m > kSmallSort && m < kRowsMaxEdges) {
+      try {
+        build_rows(ctx, uniq.p, m, lab.p, deg.p, n, kb, uniq.p, col.p, ids16, odeg.p, &st.p->row_overflow);
+        sorted = true;
+      } catch (const Error& e) {  // the slots take more room than the sort
+        if (e.status != TRIBIT_ERR_NOMEM) throw;
+      }
+    }
+    if (m && !sorted) {
+      okeys = DevBuf<uint64_t>(ctx, m);
+      k_orient_relabel<<<grid_for(m, kBlock), kBlock, 0, s>>>(uniq.p, m, lab.p, kb, okeys.p, none);
+    }
   } else {
-    k_orient<<<orient_grid, kBlock, 0, s>>>(uniq.p, m, deg.p, kb, okeys.p, zero);
+    if (m) okeys = DevBuf<uint64_t>(ctx, m);
+    k_orient<<<grid_for(std::max(m, zero.most()), kBlock), kBlock, 0, s>>>(uniq.p, m, deg.p, kb, okeys.p, zero);
   }
-
-  // 4-6. sort the arcs by (u, v) into the CSR
-  const bool narrow = relabel && m && m < (1ull << 30);
-  DevBuf<uint32_t> col(ctx, m ? m : 1);
-  DevBuf<uint32_t> row_ptr(ctx, n + 1);
-  DevBuf<uint32_t> sfx_ptr;
-  DevBuf<uint32_t> col16;
-  sfx_ptr.ctx = ctx;
-  if (relabel) sfx_ptr = DevBuf<uint32_t>(ctx, n + 1);
-  if (narrow) col16 = DevBuf<uint32_t>(ctx, col16_ids(m) / 2);
-  if (m) {
+  if (m && !sorted) {
     sort_keys(ctx, okeys.p, uniq.p, m, 2 * kb);
     okeys.reset();
-    k_csr_split<<<grid_for(m + 4, kBlock), kBlock, 0, s>>>(uniq.p, m, kb, col.p, reinterpret_cast<uint16_t*>(col16.p),
-                                                          odeg.p);
+    k_csr_split<<<grid_for(m + 4, kBlock), kBlock, 0, s>>>(uniq.p, m, kb, col.p, ids16, odeg.p);
   }
   scan_rows(ctx, odeg.p, deg.p, n, row_ptr.p, sfx_ptr.p);
 
@@ -1023,6 +1011,7 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
   float ms = 0.f;
   TB_HIP(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]));
   g->ms_prep = ms;
+  if (hst.row_overflow) fail(TRIBIT_ERR_HIP, "a row passed its degree bound");
   g->wplus = hst.wplus;
   g->rows_active = hst.rows_active;
   g->max_outdeg = hst.max_outdeg;
