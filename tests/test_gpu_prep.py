@@ -151,3 +151,36 @@ def test_rows_by_partition(gpu_ctx, relabel, n, m, clique):
     assert np.array_equal(row_ptr, np.searchsorted(arcs, np.arange(n + 1) << 32).astype(np.uint32))
     assert np.array_equal(col, (arcs & 0xFFFFFFFF).astype(np.uint32))
     assert np.array_equal(deg, np.bincount(np.concatenate([a, b]), minlength=n).astype(np.uint32))
+
+
+# ids and arcs where their sorts change method: 2^16 items (keys of 16 bits), 2^18 (more bits), past 2^20
+@pytest.mark.parametrize("n,m", [(30000, 65535), (30000, 65536), (1 << 16, 65536), (1 << 16, 262143),
+                                 (262143, 262144), (262144, 262143), (70000, 1 << 20), (1 << 20, 300000),
+                                 ((1 << 20) + 1, (1 << 20) + 1)])
+def test_sort_sizes(gpu_ctx, oracle_mod, n, m):
+    """Graphs of exactly m edges: structure, and the wedge ranges through a count, against the oracle."""
+    note(f"sorts: {n} ids, {m} edges")
+    rng = np.random.default_rng(n + m)
+    k = np.zeros(0, np.uint64)
+    while k.size < m:
+        a, b = (rng.random((2, m)) ** 2 * n).astype(np.int64)
+        x = ((np.minimum(a, b) << 32) | np.maximum(a, b))[a != b].astype(np.uint64)
+        k = np.unique(np.concatenate([k, x]))
+    k = np.sort(rng.permutation(k)[:m])
+    with gpu_ctx.graph_from_keys(k, n) as g:
+        assert_same_structure(g, k, n, oracle_mod)
+        assert g.count("wedge").triangles == oracle_mod.count_keys(k, n)
+
+
+# totals of small scans (2^15 ids), of the counts in LDS (2^15 ids, 2^18 edges) and of one schedule scan (2^19 ids)
+@pytest.mark.parametrize("n,nk", [(32768, 100000), (32769, 100000), (32768, 262144), (32768, 270000), (8192, 60000),
+                                  (524288, 600000), (524289, 600000), (600001, 400000)])
+def test_scan_and_count_sizes(gpu_ctx, oracle_mod, n, nk):
+    """Ids around the ends of the one-launch scans and of the degree count in LDS, counted under every schedule."""
+    note(f"scans: {n} ids, {nk} keys")
+    k = oracle_mod.gen_er(n, nk, seed=n % 97)
+    want = oracle_mod.count_keys(k, n)
+    with gpu_ctx.graph_from_keys(k, n) as g:
+        assert_same_structure(g, k, n, oracle_mod)
+        for sched in ("plain", "learned", "wedge"):
+            assert g.count(sched).triangles == want, sched

@@ -642,6 +642,19 @@ using IdSortConfig = rocprim::radix_sort_config<
     rocprim::default_config, rocprim::default_config,
     rocprim::radix_sort_onesweep_config<rocprim::kernel_config<1024, 16>, rocprim::kernel_config<1024, 16>, 9,
                                         rocprim::block_radix_rank_algorithm::match>>;
+// rocPRIM merges blocks instead of sweeping digits up to 2^20 items: a launch per
+// doubling, each over all items. Digits of 8 bits in small tiles (two or three
+// passes of 7 to 14 us) are faster from kFewSort16 and kFewSort items on; whole builds with
+// digits / with merges, us: 40K ids 65K edges 222 / 226, 100K 228 / 241, 300K 326 /
+// 399, 1M 425 / 533; 1M ids 65K edges 291 / 344, 1M 546 / 703. Keys of more than 16
+// bits take a third pass: 250K ids 40K edges 282 / 268, 160K 327 / 329. Beyond 2^20
+// items the larger tiles of IdSortConfig win: 150K ids 4M edges 863 / 774.
+constexpr uint64_t kFewSort16 = 1ull << 16, kFewSort = 1ull << 18, kFewSortEnd = 1ull << 20;
+using FewSortConfig = rocprim::radix_sort_config<
+    rocprim::default_config, rocprim::default_config,
+    rocprim::radix_sort_onesweep_config<rocprim::kernel_config<512, 8>, rocprim::kernel_config<512, 8>, 8,
+                                        rocprim::block_radix_rank_algorithm::match>,
+    0>;
 
 // Sorts and scans of at most kSmallSort items: one workgroup, one launch. The
 // device-wide ones are seven or eight launches at these sizes (a block sort and
@@ -705,11 +718,18 @@ static void sort_pairs(tribit_ctx* ctx, const uint32_t* in, uint32_t* out, const
     k_sort_small<uint32_t, V><<<1, kSmallThreads, 0, ctx->stream>>>(in, out, vin, vout, (uint32_t)n, bits);
     return;
   }
-  with_temp(ctx, [&](void* t, size_t& b) {
-    if (vin) return rocprim::radix_sort_pairs<Config>(t, b, in, out, vin, vout, (size_t)n, 0u, bits, ctx->stream);
-    return rocprim::radix_sort_pairs<Config>(t, b, in, out, rocprim::counting_iterator<V>(0), vout, (size_t)n, 0u,
-                                             bits, ctx->stream);
-  });
+  const auto sort = [&](auto config) {
+    using C = decltype(config);
+    with_temp(ctx, [&](void* t, size_t& b) {
+      if (vin) return rocprim::radix_sort_pairs<C>(t, b, in, out, vin, vout, (size_t)n, 0u, bits, ctx->stream);
+      return rocprim::radix_sort_pairs<C>(t, b, in, out, rocprim::counting_iterator<V>(0), vout, (size_t)n, 0u, bits,
+                                          ctx->stream);
+    });
+  };
+  if (n <= kFewSortEnd && n >= (bits <= 16 ? kFewSort16 : kFewSort))
+    sort(FewSortConfig{});
+  else
+    sort(Config{});
 }
 
 struct InDegree {
