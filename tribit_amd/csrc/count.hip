@@ -2512,7 +2512,11 @@ bool judged_known(const tribit_ctx* ctx, const tribit_graph* g, const tribit_cou
 // stand-in, not device memory): noalloc_init looks its device address up once
 // per context, with the context's device current, and kernels get that.
 constexpr uint64_t kNoAllocScratchBytes = 128ull << 20;
-static __device__ __align__(256) unsigned char noalloc_scratch[kNoAllocScratchBytes];
+// The schedules that fit are those whose lists fit the documented size beside
+// 17,664 bytes; the counters' 64 sub-queues per slot take more, behind it.
+constexpr uint64_t kNoAllocSchedule = kNoAllocScratchBytes - 17664;
+constexpr uint64_t kNoAllocBytes = kNoAllocSchedule + kCountScratch * sizeof(unsigned long long);
+static __device__ __align__(256) unsigned char noalloc_scratch[kNoAllocBytes];
 
 void noalloc_init(tribit_ctx* ctx) {
   void* p = nullptr;
@@ -2617,7 +2621,7 @@ void count(tribit_ctx* ctx, tribit_graph* g, const tribit_count_opts& opts, trib
       fail(TRIBIT_ERR_ARG, "the no-allocation count needs the schedule's range layout resident: count the graph "
                            "once with tribit_count and this schedule first");
     arena.base = static_cast<char*>(ctx->noalloc_scratch);
-    arena.size = kNoAllocScratchBytes;
+    arena.size = kNoAllocBytes;
     if (!arena.base) fail(TRIBIT_ERR_HIP, "no scratch array address for this device");
   }
   if (!noalloc) ensure_layout(ctx, g, run.layout);  // first use of a layout: built outside the timing
