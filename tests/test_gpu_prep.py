@@ -184,3 +184,20 @@ def test_scan_and_count_sizes(gpu_ctx, oracle_mod, n, nk):
         assert_same_structure(g, k, n, oracle_mod)
         for sched in ("plain", "learned", "wedge"):
             assert g.count(sched).triangles == want, sched
+
+
+# arcs around a wave's share (256) and its steps (64), and hubs whose ranges fill several waves
+@pytest.mark.parametrize("n,hubs,leaves,extra", [(300, 0, 0, 30), (40, 0, 0, 62), (4000, 0, 0, 256), (4000, 0, 0, 257),
+                                                 (60, 0, 0, 700), (3000, 3, 900, 100), (3000, 40, 2000, 9000),
+                                                 (50000, 1, 40000, 300000)])
+def test_wedge_work(gpu_ctx, n, hubs, leaves, extra):
+    """The elements that the wedge ranges of all owners stream, summed per head while the records are unpacked."""
+    note(f"wedge work: {n} ids, {hubs} hubs of {leaves}, {extra} others")
+    k = hub_graph(np.random.default_rng(n + extra), n, hubs, leaves, extra)
+    with gpu_ctx.graph_from_keys(k, n) as g:
+        row_ptr, col, _ = g.download()
+        got = sum(g.variant_stats("wedge")["wplus"])
+    row_ptr = row_ptr.astype(np.int64)
+    d = np.diff(row_ptr)
+    after = np.repeat(row_ptr[1:], d) - np.arange(col.size) - 1
+    assert got == int(after[d[col] > 0].sum())

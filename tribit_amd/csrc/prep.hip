@@ -418,7 +418,7 @@ __global__ void k_arc_rec(const uint64_t* __restrict__ okeys, uint64_t m, uint32
 // passes 64 bits. The sort then delivers the records in place: sorting arc
 // numbers and gathering 8-byte records by them pulled a sector from HBM for each
 // (R-MAT scale 25: sort 11.2 + gather 11.9 ms; with the records in the values 13.3
-// + 5.3).
+// + 2.7).
 struct ArcPack {
   uint32_t kb, eb, lb;
   bool nar;
@@ -576,30 +576,72 @@ __global__ void k_sfx_fill(const uint32_t* __restrict__ head, const uint32_t* __
   if (wave_segment_tail(v, valid, len, &sum) && sum) atomicAdd(&w_sfx[v], (unsigned long long)sum);
 }
 
-// k_sfx_fill from packed records (ArcPack) sorted by head: everything streams.
-__global__ void k_sfx_unpack(const uint32_t* __restrict__ key, const uint64_t* __restrict__ val, uint64_t m, ArcPack p,
-                             uint2* __restrict__ rng, uint8_t* __restrict__ dh, uint16_t* __restrict__ split,
-                             unsigned long long* __restrict__ w_sfx) {
-  const uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool valid = j < m;
-  const uint32_t k = valid ? key[j] : 0u;
-  const uint32_t v = valid ? (uint32_t)(k & ((1ull << p.kb) - 1)) : 0xFFFFFFFFu;
-  uint32_t len = 0;
-  if (valid) {
-    const unsigned __int128 w = ((unsigned __int128)(p.kb < 32 ? k >> p.kb : 0u) << 64) | val[j];
-    const uint32_t b = (uint32_t)((uint64_t)w & ((1ull << p.eb) - 1)) + 1;
-    len = (uint32_t)((uint64_t)(w >> p.eb) & ((1ull << p.lb) - 1));
-    uint32_t x = b + len;
-    if (p.nar) {
-      const uint64_t n = (uint64_t)(w >> (p.eb + p.lb));
-      x |= (uint32_t)(n & 3) << 30;
-      dh[j] = (uint8_t)(n >> 2);
-      split[j] = (uint16_t)((n >> 10) & ((1ull << p.lb) - 1));
-    }
-    rng[j] = make_uint2(b, x);
+// k_sfx_fill from packed records (ArcPack) sorted by head: everything streams. A
+// wave takes kUnpackSteps x 64 consecutive arcs and stores the sum of a head whose
+// arcs it holds all of; only runs that may go on in another wave are added with
+// atomics, which bound this pass with 64 arcs per wave: 523M arcs 5.2 ms, now 2.7
+// (12 GB, 4.4 TB/s, the rate of a copy).
+constexpr uint32_t kUnpackSteps = 4;
+__global__ void __launch_bounds__(kBlock) k_sfx_unpack(const uint32_t* __restrict__ key,
+                                                       const uint64_t* __restrict__ val, uint64_t m, ArcPack p,
+                                                       uint2* __restrict__ rng, uint8_t* __restrict__ dh,
+                                                       uint16_t* __restrict__ split,
+                                                       unsigned long long* __restrict__ w_sfx) {
+  const uint32_t lane = lane_id();
+  const uint64_t j0 = ((uint64_t)blockIdx.x * kBlock + (threadIdx.x & ~63u)) * kUnpackSteps + lane;
+  uint32_t k[kUnpackSteps];
+  uint64_t lo[kUnpackSteps];
+#pragma unroll
+  for (uint32_t t = 0; t < kUnpackSteps; ++t) {
+    const uint64_t j = j0 + 64 * t;
+    k[t] = j < m ? key[j] : 0u;
+    lo[t] = j < m ? val[j] : 0ull;
   }
-  uint32_t sum = 0;  // 64 lengths of at most 2^17
-  if (wave_segment_tail_u32(v, valid, len, &sum) && sum) atomicAdd(&w_sfx[v], (unsigned long long)sum);
+  bool carried = false, open = true;  // a run of the last step goes on; it reaches back to the wave's first arc
+  uint32_t ck = 0, cs = 0;            // its head and sum
+#pragma unroll
+  for (uint32_t t = 0; t < kUnpackSteps; ++t) {
+    const uint64_t j = j0 + 64 * t;
+    const bool valid = j < m;
+    const uint32_t v = valid ? (uint32_t)(k[t] & ((1ull << p.kb) - 1)) : 0xFFFFFFFFu;
+    uint32_t len = 0;
+    if (valid) {
+      const unsigned __int128 w = ((unsigned __int128)(p.kb < 32 ? k[t] >> p.kb : 0u) << 64) | lo[t];
+      const uint32_t b = (uint32_t)((uint64_t)w & ((1ull << p.eb) - 1)) + 1;
+      len = (uint32_t)((uint64_t)(w >> p.eb) & ((1ull << p.lb) - 1));
+      uint32_t x = b + len;
+      if (p.nar) {
+        const uint64_t n = (uint64_t)(w >> (p.eb + p.lb));
+        x |= (uint32_t)(n & 3) << 30;
+        dh[j] = (uint8_t)(n >> 2);
+        split[j] = (uint16_t)((n >> 10) & ((1ull << p.lb) - 1));
+      }
+      rng[j] = make_uint2(b, x);
+    }
+    uint32_t sum = 0;  // 64 kUnpackSteps lengths of at most 2^17
+    const bool tail = wave_segment_tail_u32(v, valid, len, &sum);
+    const uint32_t v0 = __shfl(v, 0), v63 = __shfl(v, 63);
+    const bool full = __shfl((int)valid, 63), joins = carried && ck == v0;
+    if (carried && !joins && lane == 0 && cs) {  // the run ended with the last step
+      if (open)
+        atomicAdd(&w_sfx[ck], (unsigned long long)cs);
+      else
+        w_sfx[ck] = cs;
+    }
+    const bool reaches = t == 0 || (joins && open);  // this step's first run: back to the wave's first arc
+    if (joins && v == v0) sum += cs;
+    const bool last = full && v == v63;
+    if (tail && sum && !(last && t + 1 < kUnpackSteps)) {
+      if (last || (reaches && v == v0))
+        atomicAdd(&w_sfx[v], (unsigned long long)sum);
+      else
+        w_sfx[v] = sum;
+    }
+    carried = full;
+    open = reaches && v63 == v0;
+    ck = v63;
+    cs = __shfl(sum, 63);
+  }
 }
 
 // W+(u) = sum of outdeg(v) over v in N+(u), per row (the PLAIN layout's work).
@@ -992,7 +1034,7 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
         DevBuf<uint64_t> val(ctx, m), val_sorted(ctx, m);
         k_arc_pack<<<grid_for(m, kBlock), kBlock, 0, s>>>(uniq.p, m, pack, row_ptr.p, col.p, rsplit.p, key.p, val.p);
         sort_pairs<IdSortConfig, uint64_t>(ctx, key.p, key_sorted.p, val.p, val_sorted.p, m, kb);
-        k_sfx_unpack<<<grid_for(m, kBlock), kBlock, 0, s>>>(key_sorted.p, val_sorted.p, m, pack, rng_sfx.p, sfx_dh.p,
+        k_sfx_unpack<<<grid_for(m, kBlock * kUnpackSteps), kBlock, 0, s>>>(key_sorted.p, val_sorted.p, m, pack, rng_sfx.p, sfx_dh.p,
                                                            sfx_split.p,
                                                            reinterpret_cast<unsigned long long*>(w_sfx.p));
       } else {
