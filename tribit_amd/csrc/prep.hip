@@ -7,7 +7,8 @@
 //   keys (min<<32|max) --partition, LDS hash sets--> m undirected edges
 //   deg[v] (endpoints by id range, counted in LDS)
 //   orient {a<b}: a->b iff deg(a) <= deg(b)       (rank = (deg, id))
-//   --sort--> row_ptr[n+1] (u32), col[m] (u32, ascending within a row)
+//   --rows by partition, else a sort--> row_ptr[n+1] (u32), col[m] (u32, ascending
+//   within a row)
 //   W+ = sum over v of indeg(v) * outdeg(v); wedge ranges (relabelled graphs)
 // Every launch is a 1-D grid of 256-thread blocks (4 waves).
 #include <cmath>
