@@ -14,6 +14,7 @@
 
 #include "common.hpp"
 #include "device.hpp"
+#include "ends.hpp"
 
 namespace tb {
 
@@ -392,12 +393,6 @@ constexpr uint32_t kEndKeys = 16;         // keys per thread and tile: 32 KiB of
 constexpr uint32_t kEndTile = kPartThreads * kEndKeys;
 constexpr uint32_t kEndCounters = 32768;  // 128 KiB of LDS
 constexpr uint32_t kEndThreads = 1024;
-// Endpoints per counting task: about two tasks per CU, between 2^17 (smaller
-// ones spend their time adding 32K counters to memory: 1.1M edges over 200K ids
-// 0.17 ms with 2^21) and 2^21.
-static uint32_t end_chunk(uint64_t m, uint32_t cus) {
-  return (uint32_t)std::min<uint64_t>(1u << 21, std::max<uint64_t>(1u << 17, 2 * m / cus));
-}
 
 __global__ void k_deg_direct(const uint64_t* __restrict__ keys, uint64_t m, uint32_t kb, uint32_t* __restrict__ deg) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -456,7 +451,7 @@ __global__ void __launch_bounds__(kPartThreads) k_ends_base(const uint32_t* __re
   uint32_t t = 0;
   for (uint32_t i = i0; i < min(i0 + per, groups); ++i) {
     b += hist[i];
-    t += 2 * ((hist[i] + chunk - 1) / chunk);
+    t += 2 * end_chunks(hist[i], chunk);
   }
   s_b[threadIdx.x] = b;
   s_t[threadIdx.x] = t;
@@ -471,7 +466,7 @@ __global__ void __launch_bounds__(kPartThreads) k_ends_base(const uint32_t* __re
     base[i] = pb;
     task[i] = pt;
     pb += hist[i];
-    pt += 2 * ((hist[i] + chunk - 1) / chunk);
+    pt += 2 * end_chunks(hist[i], chunk);
   }
   if (i0 < groups && i0 + per >= groups) {
     base[groups] = pb;
