@@ -201,3 +201,38 @@ def test_wedge_work(gpu_ctx, n, hubs, leaves, extra):
     d = np.diff(row_ptr)
     after = np.repeat(row_ptr[1:], d) - np.arange(col.size) - 1
     assert got == int(after[d[col] > 0].sum())
+
+
+# longest rows of exactly the arcs that one sort takes (4608) and one more, of a row with gaps among its ids (a random
+# graph of average degree 6300: rows to about 6300 arcs), and of many slots
+@pytest.mark.parametrize("n,m,clique,p", [(5200, 9000, 4609, 1.0), (5200, 9000, 4610, 1.0), (40000, 30000, 6000, 1.0),
+                                          (9000, 0, 9000, 0.7)])
+@pytest.mark.parametrize("relabel", [1, 2])
+def test_rows_longer_than_a_sort(gpu_ctx, relabel, n, m, clique, p):
+    """Rows past the largest sort of a slot, listed through a bitmap: the arcs as a sort of the relabelled edges gives
+    them, row by row."""
+    note(f"long rows: {n} ids, {m} edges, {clique} ids joined with {p}, id order {relabel}")
+    rng = np.random.default_rng(n + m + clique)
+    a, b = rng.integers(0, n, (2, m))
+    ids = rng.choice(n, clique, replace=False)
+    i, j = np.triu_indices(clique, 1)
+    if p < 1:
+        keep = rng.random(i.size) < p
+        i, j = i[keep], j[keep]
+    a, b = np.concatenate([a, ids[i]]), np.concatenate([b, ids[j]])
+    k = np.unique(((np.minimum(a, b) << 32) | np.maximum(a, b))[a != b].astype(np.uint64))
+    gpu_ctx.set_relabel(relabel)
+    try:
+        with gpu_ctx.graph_from_keys(rng.permutation(k), n) as g:
+            order, _ = g.labels()
+            row_ptr, col, deg = g.download()
+    finally:
+        gpu_ctx.set_relabel("auto")
+    new = np.empty(n, np.int64)
+    new[order] = np.arange(n)
+    a, b = new[(k >> np.uint64(32)).astype(np.int64)], new[(k & np.uint64(0xFFFFFFFF)).astype(np.int64)]
+    arcs = np.sort((np.minimum(a, b) << 32) | np.maximum(a, b))
+    assert np.diff(row_ptr.astype(np.int64)).max() >= (4608 if clique == 4609 else 4609)
+    assert np.array_equal(row_ptr, np.searchsorted(arcs, np.arange(n + 1) << 32).astype(np.uint32))
+    assert np.array_equal(col, (arcs & 0xFFFFFFFF).astype(np.uint32))
+    assert np.array_equal(deg, np.bincount(np.concatenate([a, b]), minlength=n).astype(np.uint32))

@@ -249,6 +249,7 @@ struct RowOut {
   uint32_t* col;
   uint16_t* col16;   // low 16 bits of v, or null
   uint32_t* odeg;
+  uint32_t* flag;    // set when a row breaks the rules its place relies on
 };
 
 // A slot's c arcs sorted by (u, v) with IPT items a thread: keys (u - u0, v - u0)
@@ -343,7 +344,7 @@ __global__ void __launch_bounds__(kRowThreads, 8) k_row_sort(const uint64_t* __r
   }
   // One long row: its ids are distinct, so a bitmap of the ids after u0 lists them
   // in order. All of those have degree 2^kRowQBits or more, so they are fewer than
-  // 2 kRowsMaxEdges / 2^kRowQBits.
+  // 2 kRowsMaxEdges / 2^kRowQBits; an id order that breaks this sets the flag.
   const uint64_t low = (1ull << kb) - 1, w0 = (uint64_t)u0 + 1;
   const uint32_t lane = lane_id();
   constexpr uint32_t kWords = kRowWindow / 32, kPer = kWords / kRowThreads;
@@ -351,7 +352,10 @@ __global__ void __launch_bounds__(kRowThreads, 8) k_row_sort(const uint64_t* __r
   __syncthreads();
   for (uint32_t i = threadIdx.x; i < c; i += kRowThreads) {
     const uint64_t x = (in[i] & low) - w0;
-    if (x < kRowWindow) atomicOr(&s.bits[x >> 5], 1u << (x & 31));
+    if (x < kRowWindow)
+      atomicOr(&s.bits[x >> 5], 1u << (x & 31));
+    else
+      atomicOr(o.flag, 1u);
   }
   __syncthreads();
   uint32_t sum = 0;
@@ -440,7 +444,7 @@ void build_rows(tribit_ctx* ctx, const uint64_t* edges, uint64_t m, const uint32
     split(std::integral_constant<uint32_t, kRowItems>{});
   scan_to(ctx, Count{cnt.p, nslots}, nslots, cbase.p);
   k_row_sort<<<nslots, kRowThreads, 0, s>>>(two ? b2.p : b1.p, kb, n, first.p, P.p, cnt.p, cbase.p, m,
-                                            RowOut{arcs, col, col16, odeg});
+                                            RowOut{arcs, col, col16, odeg, flag});
   TB_HIP(hipGetLastError());
 }
 
