@@ -236,3 +236,36 @@ def test_rows_longer_than_a_sort(gpu_ctx, relabel, n, m, clique, p):
     assert np.array_equal(row_ptr, np.searchsorted(arcs, np.arange(n + 1) << 32).astype(np.uint32))
     assert np.array_equal(col, (arcs & 0xFFFFFFFF).astype(np.uint32))
     assert np.array_equal(deg, np.bincount(np.concatenate([a, b]), minlength=n).astype(np.uint32))
+
+
+# one partition pass, the first of two, ids without edges, keys mostly repeated, and one of a workgroup's sorts
+# (KiB: the least cap under which a build by sorts alone ran, by bisection; it differs by id order with the most ids)
+@pytest.mark.parametrize("n,nk,kib", [(50000, 300000, (13967, 13967)), (1 << 18, (1 << 20) + 1, (51205, 51205)),
+                                      (1 << 16, 2500000, (106986, 106986)), (1 << 20, 50000, (30775, 33164)),
+                                      (1500, 3000000, (94168, 94168)), (900, 7000, (317, 317))])
+@pytest.mark.parametrize("relabel", [1, 2])
+def test_build_in_the_memory_of_the_sorts(gpu_ctx, oracle_mod, relabel, n, nk, kib):
+    """A build under an allocation cap that holds what sorts need: each partition and the packed records give way to
+    a sort, with the same graph and counts."""
+    note(f"capped build: {nk} keys over {n} ids, id order {relabel}")
+    rng = np.random.default_rng(n)
+    a, b = (rng.random((2, nk)) ** 1.5 * n).astype(np.int64)
+    k = ((np.minimum(a, b) << 32) | np.maximum(a, b))[a != b].astype(np.uint64)
+    cap = kib[relabel - 1] << 10
+    with tribit_amd.Context(0) as ctx:
+        ctx.set_relabel(relabel)
+        ctx.set_alloc_cap(cap)
+        with ctx.graph_from_keys(k, n) as g:
+            ctx.set_alloc_cap(0)
+            assert ctx.pool_peak() <= cap
+            row_ptr, col, deg = g.download()
+            order, _ = g.labels()
+            got = g.count("wedge").triangles
+            work = sum(g.variant_stats("wedge")["wplus"])
+        ctx.set_alloc_cap(0)
+        with ctx.graph_from_keys(k, n) as g:  # with room for the partitions
+            for x, y in zip((row_ptr, col, deg), g.download()):
+                assert np.array_equal(x, y)
+            assert np.array_equal(order, g.labels()[0])
+            assert got == g.count("wedge").triangles == oracle_mod.count_keys(k, n)
+            assert work == sum(g.variant_stats("wedge")["wplus"])

@@ -826,6 +826,14 @@ static void sort_keys(tribit_ctx* ctx, const uint64_t* in, uint64_t* out, uint64
   });
 }
 
+// Where the labels of kSkewIds ids or more begin in their buffer (in ids): an
+// R-MAT graph's frequent endpoints are ids with few set bits, and the label
+// gathers of k_row_split met in few memory channels when the array began at a
+// multiple of 2 MiB (scale 25: 13.6 ms; 11.8 from 1 MiB past one; 11.0 from an
+// offset of many set bits). Smaller label arrays stay in L2.
+constexpr uint64_t kSkewIds = 1ull << 20;
+constexpr uint64_t kLabelSkew = 0x16A200 / 4;
+
 void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n, tribit_graph* g, int relabel_opt) {
   if (relabel_opt < 0) relabel_opt = ctx->relabel;
   DevBuf<uint64_t> keys;
@@ -942,45 +950,57 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
   labels.ctx = ctx;
   DevBuf<uint64_t> okeys;  // oriented arcs, packed (u << kb) | v
   okeys.ctx = ctx;
-  DevBuf<uint32_t> odeg(ctx, n + 1);
+  // Buffers are taken where they are first used and given back after their last
+  // use: with the fall-backs to sorts on NOMEM, a build needs no more than the
+  // sorts do, max(32 nkeys, 43 m + 28 n) bytes (degree-rank ids).
+  DevBuf<uint32_t> odeg;
   DevBuf<RowStats> st(ctx, 1);
   DevBuf<uint64_t> w_sfx;
-  w_sfx.ctx = ctx;
-  if (relabel) w_sfx = DevBuf<uint64_t>(ctx, n);
-  const ZeroSpans zero{{odeg.p, reinterpret_cast<uint32_t*>(st.p), reinterpret_cast<uint32_t*>(w_sfx.p)},
-                       {n + 1, sizeof(RowStats) / 4, relabel ? 2 * n : 0}};
-  const ZeroSpans none{};
+  odeg.ctx = w_sfx.ctx = ctx;
+  ZeroSpans zero{};
+  const auto take_zeroed = [&] {  // odeg, st and w_sfx, cleared by the next launch
+    odeg = DevBuf<uint32_t>(ctx, n + 1);
+    if (relabel) w_sfx = DevBuf<uint64_t>(ctx, n);
+    zero = {{odeg.p, reinterpret_cast<uint32_t*>(st.p), reinterpret_cast<uint32_t*>(w_sfx.p)},
+            {n + 1, sizeof(RowStats) / 4, relabel ? 2 * n : 0}};
+  };
   // 4-6. the arcs sorted by (u, v) into the CSR
   const bool narrow = relabel && m && m < (1ull << 30);
-  DevBuf<uint32_t> col(ctx, m ? m : 1);
-  DevBuf<uint32_t> row_ptr(ctx, n + 1);
-  DevBuf<uint32_t> sfx_ptr;
-  DevBuf<uint32_t> col16;
-  sfx_ptr.ctx = ctx;
-  if (relabel) sfx_ptr = DevBuf<uint32_t>(ctx, n + 1);
-  if (narrow) col16 = DevBuf<uint32_t>(ctx, col16_ids(m) / 2);
-  uint16_t* ids16 = reinterpret_cast<uint16_t*>(col16.p);
+  DevBuf<uint32_t> col, col16;
+  col.ctx = col16.ctx = ctx;
+  const auto take_columns = [&] {
+    col = DevBuf<uint32_t>(ctx, m ? m : 1);
+    if (narrow) col16 = DevBuf<uint32_t>(ctx, col16_ids(m) / 2);
+  };
+  const auto ids16 = [&] { return reinterpret_cast<uint16_t*>(col16.p); };
   bool sorted = false;
   if (relabel) {
-    DevBuf<uint32_t> deg_sorted(ctx, n), lab(ctx, n);
     labels = DevBuf<uint32_t>(ctx, n);
-    if (relabel == 2) {
-      // octave classes: rank of (floor(log2(deg)), id); runs of consecutive
-      // input ids with similar degrees (a block of a block model) stay runs
-      DevBuf<uint32_t> cls(ctx, n);
-      k_octave<<<grid_for(n, kBlock), kBlock, 0, s>>>(deg.p, n, cls.p);
-      sort_pairs<rocprim::default_config, uint32_t>(ctx, cls.p, deg_sorted.p, nullptr, labels.p, n, 6u);
-      k_gather_u32<<<grid_for(n, kBlock), kBlock, 0, s>>>(deg.p, labels.p, n, deg_sorted.p);
-    } else {
-      sort_pairs<IdSortConfig, uint32_t>(ctx, deg.p, deg_sorted.p, nullptr, labels.p, n, bits_for(n));
+    {
+      DevBuf<uint32_t> deg_sorted(ctx, n);
+      if (relabel == 2) {
+        // octave classes: rank of (floor(log2(deg)), id); runs of consecutive
+        // input ids with similar degrees (a block of a block model) stay runs
+        DevBuf<uint32_t> cls(ctx, n);
+        k_octave<<<grid_for(n, kBlock), kBlock, 0, s>>>(deg.p, n, cls.p);
+        sort_pairs<rocprim::default_config, uint32_t>(ctx, cls.p, deg_sorted.p, nullptr, labels.p, n, 6u);
+        k_gather_u32<<<grid_for(n, kBlock), kBlock, 0, s>>>(deg.p, labels.p, n, deg_sorted.p);
+      } else {
+        sort_pairs<IdSortConfig, uint32_t>(ctx, deg.p, deg_sorted.p, nullptr, labels.p, n, bits_for(n));
+      }
+      std::swap(deg.p, deg_sorted.p);  // deg now indexed by internal id
     }
-    std::swap(deg.p, deg_sorted.p);  // deg now indexed by internal id
-    k_scatter_labels<<<grid_for(std::max(n, zero.most()), kBlock), kBlock, 0, s>>>(labels.p, n, lab.p, zero);
+    const uint64_t skew = n >= kSkewIds ? kLabelSkew : 0;
+    DevBuf<uint32_t> lab_buf(ctx, n + skew);
+    uint32_t* lab = lab_buf.p + skew;
+    take_zeroed();
+    k_scatter_labels<<<grid_for(std::max(n, zero.most()), kBlock), kBlock, 0, s>>>(labels.p, n, lab, zero);
+    take_columns();
     // rows by partition, but a sort by one workgroup where that suffices (two
     // launches of 35 us against five of 31) and for more edges than the slots cover
     if (m > kSmallSort && m < kRowsMaxEdges) {
       try {
-        build_rows(ctx, uniq.p, m, lab.p, deg.p, n, kb, uniq.p, col.p, ids16, odeg.p, &st.p->row_overflow);
+        build_rows(ctx, uniq.p, m, lab, deg.p, n, kb, uniq.p, col.p, ids16(), odeg.p, &st.p->row_overflow);
         sorted = true;
       } catch (const Error& e) {  // the slots take more room than the sort
         if (e.status != TRIBIT_ERR_NOMEM) throw;
@@ -988,18 +1008,25 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
     }
     if (m && !sorted) {
       okeys = DevBuf<uint64_t>(ctx, m);
-      k_orient_relabel<<<grid_for(m, kBlock), kBlock, 0, s>>>(uniq.p, m, lab.p, kb, okeys.p, none);
+      k_orient_relabel<<<grid_for(m, kBlock), kBlock, 0, s>>>(uniq.p, m, lab, kb, okeys.p, ZeroSpans{});
     }
   } else {
     if (m) okeys = DevBuf<uint64_t>(ctx, m);
+    take_zeroed();
     k_orient<<<grid_for(std::max(m, zero.most()), kBlock), kBlock, 0, s>>>(uniq.p, m, deg.p, kb, okeys.p, zero);
+    take_columns();
   }
   if (m && !sorted) {
     sort_keys(ctx, okeys.p, uniq.p, m, 2 * kb);
     okeys.reset();
-    k_csr_split<<<grid_for(m + 4, kBlock), kBlock, 0, s>>>(uniq.p, m, kb, col.p, ids16, odeg.p);
+    k_csr_split<<<grid_for(m + 4, kBlock), kBlock, 0, s>>>(uniq.p, m, kb, col.p, ids16(), odeg.p);
   }
+  DevBuf<uint32_t> row_ptr(ctx, n + 1);
+  DevBuf<uint32_t> sfx_ptr;
+  sfx_ptr.ctx = ctx;
+  if (relabel) sfx_ptr = DevBuf<uint32_t>(ctx, n + 1);
   scan_rows(ctx, odeg.p, deg.p, n, row_ptr.p, sfx_ptr.p);
+  odeg.reset();
 
   // 7. totals (W+, active rows, largest outdeg) from the rows, and the rows' split positions
   DevBuf<uint32_t> rsplit;
@@ -1030,25 +1057,34 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
         ctx->sync();
         pack.lb = bits_for((uint64_t)hst.max_outdeg + 1);
       }
+      unsigned long long* w = reinterpret_cast<unsigned long long*>(w_sfx.p);
+      bool filled = false;
       if (pack.fits()) {
-        DevBuf<uint32_t> key(ctx, m), key_sorted(ctx, m);
-        DevBuf<uint64_t> val(ctx, m), val_sorted(ctx, m);
-        k_arc_pack<<<grid_for(m, kBlock), kBlock, 0, s>>>(uniq.p, m, pack, row_ptr.p, col.p, rsplit.p, key.p, val.p);
-        sort_pairs<IdSortConfig, uint64_t>(ctx, key.p, key_sorted.p, val.p, val_sorted.p, m, kb);
-        k_sfx_unpack<<<grid_for(m, kBlock * kUnpackSteps), kBlock, 0, s>>>(key_sorted.p, val_sorted.p, m, pack, rng_sfx.p, sfx_dh.p,
-                                                           sfx_split.p,
-                                                           reinterpret_cast<unsigned long long*>(w_sfx.p));
-      } else {
+        try {
+          DevBuf<uint32_t> key(ctx, m), key_sorted(ctx, m);
+          DevBuf<uint64_t> val(ctx, m), val_sorted(ctx, m);
+          k_arc_pack<<<grid_for(m, kBlock), kBlock, 0, s>>>(uniq.p, m, pack, row_ptr.p, col.p, rsplit.p, key.p, val.p);
+          sort_pairs<IdSortConfig, uint64_t>(ctx, key.p, key_sorted.p, val.p, val_sorted.p, m, kb);
+          k_sfx_unpack<<<grid_for(m, kBlock * kUnpackSteps), kBlock, 0, s>>>(
+              key_sorted.p, val_sorted.p, m, pack, rng_sfx.p, sfx_dh.p, sfx_split.p, w);
+          filled = true;
+        } catch (const Error& e) {  // 36 bytes an arc beside the keys; arc numbers and records take 24 without them
+          if (e.status != TRIBIT_ERR_NOMEM) throw;
+        }
+      }
+      if (!filled) {
         DevBuf<uint2> arec(ctx, m);
         k_arc_rec<<<grid_for(m, kBlock), kBlock, 0, s>>>(uniq.p, m, kb, row_ptr.p, col.p, rsplit.p, narrow, arec.p);
+        uniq.reset();
+        rsplit.reset();
         DevBuf<uint32_t> head(ctx, m), arc_sorted(ctx, m);
         sort_pairs<IdSortConfig, uint32_t>(ctx, col.p, head.p, nullptr, arc_sorted.p, m, kb);
         k_sfx_fill<<<grid_for(m, kBlock), kBlock, 0, s>>>(head.p, arc_sorted.p, m, arec.p, rng_sfx.p, sfx_dh.p,
-                                                          sfx_split.p,
-                                                          reinterpret_cast<unsigned long long*>(w_sfx.p));
+                                                          sfx_split.p, w);
       }
     }
   }
+  rsplit.reset();
   uniq.reset();
   TB_HIP(hipMemcpyAsync(&hst, st.p, sizeof(hst), hipMemcpyDeviceToHost, s));
 
