@@ -269,3 +269,42 @@ def test_build_in_the_memory_of_the_sorts(gpu_ctx, oracle_mod, relabel, n, nk, k
             assert np.array_equal(order, g.labels()[0])
             assert got == g.count("wedge").triangles == oracle_mod.count_keys(k, n)
             assert work == sum(g.variant_stats("wedge")["wplus"])
+
+
+# edges around a block's share (2048) and the most of this way, over ids that just pass LDS and many; stars and few hubs
+@pytest.mark.parametrize("n,m,hubs", [(32769, 1, 0), (40000, 2048, 0), (40000, 2049, 3), (300000, 1 << 18, 0),
+                                      (300000, 1 << 18, 1), (300000, 1 << 18, 8), (1 << 24, 262143, 1)])
+def test_degrees_of_few_edges(gpu_ctx, n, m, hubs):
+    note(f"degrees: {m} edges over {n} ids, {hubs} hubs")
+    rng = np.random.default_rng(n + m + hubs)
+    k = np.zeros(0, np.uint64)
+    while k.size < m:
+        a = rng.integers(0, n, 2 * m) if hubs == 0 else n - 1 - rng.integers(0, hubs, 2 * m)
+        b = rng.integers(0, n, 2 * m)
+        x = ((np.minimum(a, b) << 32) | np.maximum(a, b))[a != b].astype(np.uint64)
+        k = np.unique(np.concatenate([k, x]))
+    k = rng.permutation(k)[:m]
+    want = np.bincount((k >> np.uint64(32)).astype(np.int64), minlength=n)
+    want += np.bincount((k & np.uint64(0xFFFFFFFF)).astype(np.int64), minlength=n)
+    with gpu_ctx.graph_from_keys(k, n) as g:
+        labels, _ = g.labels()
+        assert np.array_equal(g.download()[2], want[labels].astype(np.uint32))
+
+
+def test_star_builds_like_other_graphs(gpu_ctx):
+    """Device time of a star of 2^18 edges against a random graph's: a queue of atomics on its hub made it ten times."""
+    note("star and random graph of 2^18 edges")
+    n, m = 300000, 1 << 18
+    rng = np.random.default_rng(1)
+    leaf = np.arange(1, m + 1, dtype=np.uint64)
+    a, b = rng.integers(0, n, (2, m))
+    other = ((np.minimum(a, b) << 32) | np.maximum(a, b))[a != b].astype(np.uint64)
+
+    def ms(keys):
+        t = []
+        for _ in range(6):
+            with gpu_ctx.graph_from_keys(keys, n) as g:
+                t.append(g.info()["ms_preprocess"])
+        return min(t)
+
+    assert ms(leaf) < 4 * ms(other)
