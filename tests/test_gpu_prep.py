@@ -308,3 +308,12 @@ def test_star_builds_like_other_graphs(gpu_ctx):
         return min(t)
 
     assert ms(leaf) < 4 * ms(other)
+
+
+def test_degrees_of_more_than_2_31_edges(gpu_ctx):
+    """Two spans of keys: W+ (which every degree enters) and the triangles are those that a build by sorts gave."""
+    note("er of 2.3G keys over 2^24 ids")
+    with gpu_ctx.gen_er(1 << 24, 2300000000, seed=1) as g:
+        i = g.info()
+        assert (i["m"], i["wplus"]) == (2299981280, 210131079941)
+        assert g.count("wedge").triangles == 3433745

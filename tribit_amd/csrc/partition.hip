@@ -385,10 +385,12 @@ bool distinct_keys(tribit_ctx* ctx, const uint64_t* d_keys, uint64_t nk, uint64_
 // beyond kDirectEdges keys the endpoints' low 16 bits are first grouped by
 // their high bits (2 bytes written per endpoint), and each group of 65,536 ids
 // is counted in LDS, half of its ids at a time. A pass covers up to
-// kEndMaxGroups groups (2^27 ids), so that a tile's runs stay long.
+// kEndMaxGroups groups (2^27 ids), so that a tile's runs stay long, and up to
+// kEndSpan keys, so that 32 bits hold a group's endpoints.
 constexpr uint64_t kDirectEdges = 1ull << 18;
 constexpr uint32_t kEndBits = 16;
 constexpr uint32_t kEndMaxGroups = 2048;
+constexpr uint64_t kEndSpan = 0x7FFFFFFF;
 constexpr uint32_t kEndKeys = 16;         // keys per thread and tile: 32 KiB of halves, as much of digits
 constexpr uint32_t kEndTile = kPartThreads * kEndKeys;
 constexpr uint32_t kEndCounters = 32768;  // 128 KiB of LDS
@@ -431,14 +433,6 @@ __global__ void __launch_bounds__(kEndThreads) k_deg_table(const uint64_t* __res
   __syncthreads();
   for (uint32_t i = threadIdx.x; i < kTableSlots; i += kEndThreads)
     if (s_n[i]) atomicAdd(&deg[s_id[i]], s_n[i]);
-}
-
-__global__ void k_deg_direct(const uint64_t* __restrict__ keys, uint64_t m, uint32_t kb, uint32_t* __restrict__ deg) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  const uint64_t k = keys[i];
-  atomicAdd(&deg[(uint32_t)(k >> kb)], 1u);
-  atomicAdd(&deg[(uint32_t)(k & ((1ull << kb) - 1))], 1u);
 }
 
 // Few edges over ids that fit LDS: every block counts its share there and adds
@@ -560,11 +554,12 @@ __global__ void __launch_bounds__(kPartThreads) k_ends_split(const uint64_t* __r
 }
 
 // Counting tasks: chunk c of group g, half h of its ids. A group of one chunk
-// stores its counts; several chunks add theirs (deg is zero before).
+// stores its counts, unless `more` spans of keys add to them; several chunks add
+// theirs (deg is zero before).
 __global__ void __launch_bounds__(kEndThreads) k_ends_count(const uint16_t* __restrict__ ends,
                                                             const uint64_t* __restrict__ base,
                                                             const uint32_t* __restrict__ task, uint32_t g0,
-                                                            uint32_t groups, uint32_t chunk, uint64_t n,
+                                                            uint32_t groups, uint32_t chunk, uint64_t n, bool more,
                                                             uint32_t* __restrict__ deg) {
   __shared__ uint32_t s_c[kEndCounters];
   const uint32_t tasks = task[groups];
@@ -578,7 +573,7 @@ __global__ void __launch_bounds__(kEndThreads) k_ends_count(const uint16_t* __re
         hi = mid;
     }
     const uint32_t g = lo, half = (t - task[g]) & 1u, c = (t - task[g]) >> 1;
-    const bool sole = task[g + 1] - task[g] == 2;
+    const bool sole = !more && task[g + 1] - task[g] == 2;
     for (uint32_t i = threadIdx.x; i < kEndCounters; i += kEndThreads) s_c[i] = 0u;
     __syncthreads();
     const uint64_t e0 = base[g] + (uint64_t)c * chunk, e1 = min(base[g + 1], e0 + chunk);
@@ -623,25 +618,25 @@ void count_degrees(tribit_ctx* ctx, const uint64_t* keys, uint64_t m, uint64_t n
     k_deg_table<<<grid_for(m, kTableKeys * kEndThreads), kEndThreads, 0, s>>>(keys, (uint32_t)m, kb, deg);
     return;
   }
-  if (m > 0x7FFFFFFFull) {  // 32-bit cursors over 2 m endpoints
-    k_deg_direct<<<grid_for(m, kBlock), kBlock, 0, s>>>(keys, m, kb, deg);
-    return;
-  }
   const uint32_t groups = (uint32_t)((n + (1ull << kEndBits) - 1) >> kEndBits);
   const uint32_t most = std::min(groups, kEndMaxGroups), cus = (uint32_t)(ctx->cus > 0 ? ctx->cus : 256);
-  DevBuf<uint16_t> ends(ctx, 2 * m + 8);
+  DevBuf<uint16_t> ends(ctx, 2 * std::min(m, kEndSpan) + 8);
   DevBuf<uint32_t> hist(ctx, 3 * most + 1);  // histogram, cursors, tasks
   DevBuf<uint64_t> base(ctx, most + 1);
   uint32_t *cursor = hist.p + most, *task = hist.p + 2 * most;
-  const uint32_t chunk = end_chunk(m, cus);
-  for (uint32_t g0 = 0; g0 < groups; g0 += kEndMaxGroups) {
-    const uint32_t ng = std::min(groups - g0, kEndMaxGroups);
-    k_part_zero<<<grid_for(2 * most, kBlock), kBlock, 0, s>>>(hist.p, 2 * most);
-    k_ends_hist<<<std::min<uint32_t>(4 * cus, grid_for(m, kPartThreads)), kPartThreads, 4 * ng, s>>>(keys, m, kb, g0,
-                                                                                                    ng, hist.p);
-    k_ends_base<<<1, kPartThreads, 0, s>>>(hist.p, ng, chunk, base.p, task);
-    k_ends_split<<<grid_for(m, kEndTile), kPartThreads, 8 * ng, s>>>(keys, m, kb, g0, ng, base.p, cursor, ends.p);
-    k_ends_count<<<cus, kEndThreads, 0, s>>>(ends.p, base.p, task, g0, ng, chunk, n, deg);
+  for (uint64_t k0 = 0; k0 < m; k0 += kEndSpan) {
+    const uint64_t* k = keys + k0;
+    const uint64_t mk = std::min(m - k0, kEndSpan);
+    const uint32_t chunk = end_chunk(mk, cus);
+    for (uint32_t g0 = 0; g0 < groups; g0 += kEndMaxGroups) {
+      const uint32_t ng = std::min(groups - g0, kEndMaxGroups);
+      k_part_zero<<<grid_for(2 * most, kBlock), kBlock, 0, s>>>(hist.p, 2 * most);
+      k_ends_hist<<<std::min<uint32_t>(4 * cus, grid_for(mk, kPartThreads)), kPartThreads, 4 * ng, s>>>(k, mk, kb, g0,
+                                                                                                       ng, hist.p);
+      k_ends_base<<<1, kPartThreads, 0, s>>>(hist.p, ng, chunk, base.p, task);
+      k_ends_split<<<grid_for(mk, kEndTile), kPartThreads, 8 * ng, s>>>(k, mk, kb, g0, ng, base.p, cursor, ends.p);
+      k_ends_count<<<cus, kEndThreads, 0, s>>>(ends.p, base.p, task, g0, ng, chunk, n, m > kEndSpan, deg);
+    }
   }
 }
 
