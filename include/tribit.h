@@ -162,8 +162,10 @@ typedef struct {
 /* Selects `device` and creates a stream and a device memory pool that keeps
  * freed memory for later calls, as init_gpu_kernel5 (main5_multi.cu:578-587) and
  * allocate_memory (tribit.cu:825-838) do. The pool is the context's own: at most
- * a quarter of the device's memory stays in it unused, and tribit_shutdown gives
- * all of it back, so free the context's graphs, batches and models first. */
+ * three quarters of the device's memory stay in it unused, an allocation for
+ * which the device has no room takes back what the context and the device's
+ * other contexts hold unused, and tribit_shutdown gives all of it back, so free
+ * the context's graphs, batches and models first. */
 int tribit_init(int device, tribit_ctx** out);
 int tribit_shutdown(tribit_ctx* ctx);
 /* Test hook: fail device allocations beyond `bytes` in total (0 = no cap). */

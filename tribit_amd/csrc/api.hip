@@ -86,7 +86,7 @@ int tribit_init(int device, tribit_ctx** out) {
       snprintf(dname, sizeof(dname), "%s", prop.name);
     snprintf(ctx->name, sizeof(ctx->name), "%s (%s, %d CUs)", dname, prop.gcnArchName, prop.multiProcessorCount);
     TB_HIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
-    ctx->pool.init(ctx->stream, prop.totalGlobalMem / 4);  // freed memory stays with the context (tribit.cu:829-830)
+    ctx->pool.init(device, ctx->stream, prop.totalGlobalMem);  // freed memory stays with the context (tribit.cu:829-830)
     for (auto& e : ctx->ev) TB_HIP(hipEventCreate(&e));
     TB_HIP(hipHostMalloc(&ctx->readback, tribit_ctx::kReadback, hipHostMallocDefault));
     tb::noalloc_init(ctx);  // the device is current: its copy of the scratch array

@@ -150,7 +150,7 @@ void build_part(tribit_ctx* ctx, tribit_batch* b, uint32_t first, uint32_t count
     // a part's replay never counts dense diagonal blocks, so the automatic id
     // order resolves to degree rank, which streams faster
     preprocess(ctx, keys.release(), nk, n, part.g, ctx->relabel == 3 ? 1 : ctx->relabel);
-    DevBuf<uint32_t> gid(ctx, n);
+    DevBuf<uint32_t> gid(ctx, n, kKept);
     k_vertex_gid<<<grid_for(n, 256), 256, 0, s>>>(part.g->labels, n, voff.p, count, first, gid.p);
     DevBuf<unsigned long long> m(ctx, b->ngraphs);
     k_zero_words<<<grid_for(b->ngraphs, 256), 256, 0, s>>>(m.p, b->ngraphs);
@@ -179,8 +179,9 @@ tribit_batch* new_batch(tribit_ctx* ctx, uint32_t ngraphs) {
 }
 
 void finish_batch(tribit_ctx* ctx, tribit_batch* b) {
-  b->gcount = ctx->alloc_n<unsigned long long>(b->ngraphs ? b->ngraphs : 1);
-  b->scratch = ctx->alloc_n<unsigned long long>(tb::kCountScratch * (b->parts.size() ? b->parts.size() : 1));
+  b->gcount = ctx->alloc_n<unsigned long long>(b->ngraphs ? b->ngraphs : 1, tb::kKept);
+  b->scratch =
+      ctx->alloc_n<unsigned long long>(tb::kCountScratch * (b->parts.size() ? b->parts.size() : 1), tb::kKept);
 }
 
 }  // namespace

@@ -86,11 +86,12 @@ struct tribit_ctx {
   static constexpr size_t kReadback = 4096;
   std::string last_error;
 
-  void* alloc(uint64_t bytes) {
+  // kept: the buffer outlives the call that takes it (a graph's, a batch's, a model's)
+  void* alloc(uint64_t bytes, bool kept = false) {
     if (bytes == 0) bytes = 8;
     bytes = (bytes + 255) & ~uint64_t(255);
     if (cap && held + bytes > cap) tb::fail(TRIBIT_ERR_NOMEM, "allocation exceeds the configured cap");
-    void* p = pool.alloc(bytes);
+    void* p = pool.alloc(bytes, kept);
     if (!p) tb::fail(TRIBIT_ERR_NOMEM, "no device memory for " + std::to_string(bytes) + " bytes");
     sizes[p] = bytes;
     held += bytes;
@@ -98,8 +99,8 @@ struct tribit_ctx {
     return p;
   }
   template <typename T>
-  T* alloc_n(uint64_t n) {
-    return static_cast<T*>(alloc(n * sizeof(T)));
+  T* alloc_n(uint64_t n, bool kept = false) {
+    return static_cast<T*>(alloc(n * sizeof(T), kept));
   }
   void free(void* p) {
     if (!p) return;
@@ -120,7 +121,7 @@ struct DevBuf {
   T* p = nullptr;
   uint64_t n = 0;
   DevBuf() = default;
-  DevBuf(tribit_ctx* c, uint64_t count) : ctx(c), p(c->alloc_n<T>(count)), n(count) {}
+  DevBuf(tribit_ctx* c, uint64_t count, bool kept = false) : ctx(c), p(c->alloc_n<T>(count, kept)), n(count) {}
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
   DevBuf(DevBuf&& o) noexcept : ctx(o.ctx), p(o.p), n(o.n) { o.p = nullptr; }
@@ -145,6 +146,8 @@ struct DevBuf {
 };
 
 namespace tb {
+constexpr bool kKept = true;  // of a DevBuf that an object takes over (release)
+
 struct BucketCache;
 
 // Device counters of one count, none of them sharing a 128-byte line with

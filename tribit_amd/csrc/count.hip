@@ -2138,6 +2138,7 @@ struct Schedule {
   const uint2* rng = nullptr;
   TileSrc ts{nullptr, nullptr, nullptr};
   DevBuf<uint4> tasks;
+  bool kept = false;       // held beyond the call (a batch's)
   Cnt8 tot{}, base{};
   uint64_t ntask = 0;
 };
@@ -2251,7 +2252,7 @@ void make_schedule(tribit_ctx* ctx, tribit_graph* g, int layout, int flags, bool
   if (arena)
     S.tasks.p = arena->take<uint4>(S.ntask);  // S.tasks.ctx stays null: the arena is never freed here
   else
-    S.tasks = DevBuf<uint4>(ctx, S.ntask ? S.ntask : 1);
+    S.tasks = DevBuf<uint4>(ctx, S.ntask ? S.ntask : 1, S.kept);
   if (nb) k_sched_fill<<<(unsigned)nb, kSchedBlock, 0, s>>>(sv, pd, n, off, S.base, S.tasks.p);
   TB_HIP(hipGetLastError());
   // bit tiles only for a launch that streams them: the menu always has a tile
@@ -2885,6 +2886,7 @@ static double batch_schedules(tribit_ctx* ctx, tribit_batch* b, int sched, int f
     if (layout == TRIBIT_SCHED_WEDGE && !p.g->rng_sfx) fail(TRIBIT_ERR_ARG, "the wedge schedule needs relabelled graphs");
     p.S = new Schedule;
     p.S->plan = plan;
+    p.S->kept = true;
     // per-graph attribution: no dense core and no dense blocks (their launches
     // add to the batch total, not to each graph's count)
     make_schedule(ctx, p.g, layout, flags & ~TRIBIT_COUNT_DENSE_BLOCKS, learned, *p.S, 0);
@@ -2934,6 +2936,7 @@ static double batch_capture(tribit_ctx* ctx, tribit_batch* b, int att, uint32_t*
   uint64_t blocks = 0;
   uint32_t nl = 2;
   uint64_t nt = 0;
+  const auto hold = ctx->pool.hold();
   TB_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
   try {
     k_zero_u64<<<grid_for(b->ngraphs ? b->ngraphs : 1, kBlock), kBlock, 0, s>>>(b->gcount, b->ngraphs);

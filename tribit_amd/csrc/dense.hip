@@ -325,7 +325,7 @@ void core_prepare(tribit_ctx* ctx, tribit_graph* g, uint64_t c) {
   if (c == 0) return;
   const uint64_t kp = (c + kCoreTile2 - 1) / kCoreTile2 * kCoreTile2;
   const uint64_t d0 = g->n - c;
-  DevBuf<uint32_t> bits(ctx, kp * kp / 32);
+  DevBuf<uint32_t> bits(ctx, kp * kp / 32, kKept);
   hipStream_t s = ctx->stream;
   k_core_bits<<<grid_for(kp, 4), 256, 0, s>>>(g->row_ptr, g->col, g->n, d0, (uint32_t)kp, bits.p);
   TB_HIP(hipGetLastError());
@@ -781,11 +781,11 @@ static bool blocks_build(tribit_ctx* ctx, tribit_graph* g) {
       for (uint32_t I = 0; I <= J; ++I)
         work.push_back(make_uint4((uint32_t)aoff[i], (uint32_t)(aoff[i] >> 32), kp, I | (J << 16)));
   }
-  DevBuf<int8_t> A(ctx, total);
-  DevBuf<uint4> dwork(ctx, work.size());
-  DevBuf<uint2> dblk(ctx, nb);
-  DevBuf<uint64_t> daoff(ctx, nb);
-  DevBuf<uint32_t> dkp(ctx, nb);
+  DevBuf<int8_t> A(ctx, total, kKept);
+  DevBuf<uint4> dwork(ctx, work.size(), kKept);
+  DevBuf<uint2> dblk(ctx, nb, kKept);
+  DevBuf<uint64_t> daoff(ctx, nb, kKept);
+  DevBuf<uint32_t> dkp(ctx, nb, kKept);
   TB_HIP(hipMemcpyAsync(dwork.p, work.data(), 16ull * work.size(), hipMemcpyHostToDevice, s));
   TB_HIP(hipMemcpyAsync(dblk.p, hb.data(), 8ull * nb, hipMemcpyHostToDevice, s));
   TB_HIP(hipMemcpyAsync(daoff.p, aoff.data(), 8ull * nb, hipMemcpyHostToDevice, s));
@@ -793,11 +793,11 @@ static bool blocks_build(tribit_ctx* ctx, tribit_graph* g) {
   k_core_zero<<<2048, 256, 0, s>>>(reinterpret_cast<uint4*>(A.p), total / 16);
   k_blk_fill<<<nb, 256, 0, s>>>(g->row_ptr, g->col, dblk.p, daoff.p, dkp.p, nb, A.p);
   // the streamed ranges: a copy of the wedge ranges with in-block arcs cut
-  DevBuf<int32_t> blk_of(ctx, n);
+  DevBuf<int32_t> blk_of(ctx, n, kKept);
   TB_HIP(hipMemsetAsync(blk_of.p, 0xFF, 4 * n, s));
   k_blk_mark<<<nb, 256, 0, s>>>(dblk.p, nb, blk_of.p);
   DevBuf<uint2> rng(ctx, m);
-  DevBuf<uint64_t> w(ctx, n);
+  DevBuf<uint64_t> w(ctx, n, kKept);
   DevBuf<unsigned long long> cut(ctx, 1);
   TB_HIP(hipMemcpyAsync(rng.p, g->rng_sfx, 8 * m, hipMemcpyDeviceToDevice, s));
   TB_HIP(hipMemcpyAsync(w.p, g->w_sfx, 8 * n, hipMemcpyDeviceToDevice, s));
@@ -808,7 +808,7 @@ static bool blocks_build(tribit_ctx* ctx, tribit_graph* g) {
   unsigned long long hcut = 0;
   TB_HIP(hipMemcpyAsync(&hcut, cut.p, 8, hipMemcpyDeviceToHost, s));
   // the owners' lists without the empty ranges of in-block arcs
-  DevBuf<uint32_t> bptr(ctx, n + 1);
+  DevBuf<uint32_t> bptr(ctx, n + 1, kKept);
   DevBuf<uint2> crng;
   crng.ctx = ctx;
   {
@@ -822,7 +822,7 @@ static bool blocks_build(tribit_ctx* ctx, tribit_graph* g) {
     uint32_t kept = 0;
     TB_HIP(hipMemcpyAsync(&kept, bptr.p + n, 4, hipMemcpyDeviceToHost, s));
     ctx->sync();
-    crng = DevBuf<uint2>(ctx, kept ? kept : 1);
+    crng = DevBuf<uint2>(ctx, kept ? kept : 1, kKept);
     k_blk_compact<<<grid_for(n, 256), 256, 0, s>>>(g->sfx_ptr, rng.p, n, range_end_mask(m), bptr.p, nullptr,
                                                    crng.p);
     TB_HIP(hipGetLastError());
@@ -853,7 +853,7 @@ static bool blocks_build(tribit_ctx* ctx, tribit_graph* g) {
     nkeys = last_off + last_cnt;
     if (nkeys) {
       DevBuf<uint64_t> raw(ctx, nkeys);
-      key = DevBuf<uint64_t>(ctx, nkeys);
+      key = DevBuf<uint64_t>(ctx, nkeys, kKept);
       k_blk_out_arcs<<<grid_for(n, 256), 256, 0, s>>>(g->row_ptr, g->col, dblk.p, blk_of.p, n, off.p, nullptr,
                                                       raw.p);
       size_t tb2 = 0;
@@ -884,11 +884,11 @@ static bool blocks_build(tribit_ctx* ctx, tribit_graph* g) {
         nruns = (uint32_t)hs.size();
         nruns_long = (uint32_t)hl.size();
         if (nruns) {
-          runs = DevBuf<uint2>(ctx, nruns);
+          runs = DevBuf<uint2>(ctx, nruns, kKept);
           TB_HIP(hipMemcpyAsync(runs.p, hs.data(), 8ull * nruns, hipMemcpyHostToDevice, s));
         }
         if (nruns_long) {
-          runs_long = DevBuf<uint2>(ctx, nruns_long);
+          runs_long = DevBuf<uint2>(ctx, nruns_long, kKept);
           TB_HIP(hipMemcpyAsync(runs_long.p, hl.data(), 8ull * nruns_long, hipMemcpyHostToDevice, s));
         }
       }

@@ -184,10 +184,10 @@ tribit_mlp* mlp_create(tribit_ctx* ctx, int nfeat, uint64_t seed) {
   m->shape = mlp_shape(nfeat);
   const size_t T = m->shape.total;
   try {
-    m->p = ctx->alloc_n<float>(T);
-    m->m1 = ctx->alloc_n<float>(T);
-    m->m2 = ctx->alloc_n<float>(T);
-    m->pb = ctx->alloc_n<uint16_t>(T);
+    m->p = ctx->alloc_n<float>(T, tb::kKept);
+    m->m1 = ctx->alloc_n<float>(T, tb::kKept);
+    m->m2 = ctx->alloc_n<float>(T, tb::kKept);
+    m->pb = ctx->alloc_n<uint16_t>(T, tb::kKept);
   } catch (...) {
     ctx->free(m->p);
     ctx->free(m->m1);

@@ -937,7 +937,7 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
   g->m = m;
 
   // 3. degrees
-  DevBuf<uint32_t> deg(ctx, n);
+  DevBuf<uint32_t> deg(ctx, n, kKept);
   count_degrees(ctx, uniq.p, m, n, kb, deg.p);
 
   // 3b. optional degree relabelling: internal id = rank of (deg, id) (mode 1)
@@ -960,7 +960,7 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
   ZeroSpans zero{};
   const auto take_zeroed = [&] {  // odeg, st and w_sfx, cleared by the next launch
     odeg = DevBuf<uint32_t>(ctx, n + 1);
-    if (relabel) w_sfx = DevBuf<uint64_t>(ctx, n);
+    if (relabel) w_sfx = DevBuf<uint64_t>(ctx, n, kKept);
     zero = {{odeg.p, reinterpret_cast<uint32_t*>(st.p), reinterpret_cast<uint32_t*>(w_sfx.p)},
             {n + 1, sizeof(RowStats) / 4, relabel ? 2 * n : 0}};
   };
@@ -969,15 +969,15 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
   DevBuf<uint32_t> col, col16;
   col.ctx = col16.ctx = ctx;
   const auto take_columns = [&] {
-    col = DevBuf<uint32_t>(ctx, m ? m : 1);
-    if (narrow) col16 = DevBuf<uint32_t>(ctx, col16_ids(m) / 2);
+    col = DevBuf<uint32_t>(ctx, m ? m : 1, kKept);
+    if (narrow) col16 = DevBuf<uint32_t>(ctx, col16_ids(m) / 2, kKept);
   };
   const auto ids16 = [&] { return reinterpret_cast<uint16_t*>(col16.p); };
   bool sorted = false;
   if (relabel) {
-    labels = DevBuf<uint32_t>(ctx, n);
+    labels = DevBuf<uint32_t>(ctx, n, kKept);
     {
-      DevBuf<uint32_t> deg_sorted(ctx, n);
+      DevBuf<uint32_t> deg_sorted(ctx, n, kKept);
       if (relabel == 2) {
         // octave classes: rank of (floor(log2(deg)), id); runs of consecutive
         // input ids with similar degrees (a block of a block model) stay runs
@@ -1021,10 +1021,10 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
     okeys.reset();
     k_csr_split<<<grid_for(m + 4, kBlock), kBlock, 0, s>>>(uniq.p, m, kb, col.p, ids16(), odeg.p);
   }
-  DevBuf<uint32_t> row_ptr(ctx, n + 1);
+  DevBuf<uint32_t> row_ptr(ctx, n + 1, kKept);
   DevBuf<uint32_t> sfx_ptr;
   sfx_ptr.ctx = ctx;
-  if (relabel) sfx_ptr = DevBuf<uint32_t>(ctx, n + 1);
+  if (relabel) sfx_ptr = DevBuf<uint32_t>(ctx, n + 1, kKept);
   scan_rows(ctx, odeg.p, deg.p, n, row_ptr.p, sfx_ptr.p);
   odeg.reset();
 
@@ -1042,10 +1042,10 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
   DevBuf<uint16_t> sfx_split;
   rng_sfx.ctx = ctx;
   if (relabel) {
-    rng_sfx = DevBuf<uint2>(ctx, m ? m : 1);
+    rng_sfx = DevBuf<uint2>(ctx, m ? m : 1, kKept);
     if (narrow) {
-      sfx_dh = DevBuf<uint8_t>(ctx, m);
-      sfx_split = DevBuf<uint16_t>(ctx, m);
+      sfx_dh = DevBuf<uint8_t>(ctx, m, kKept);
+      sfx_split = DevBuf<uint16_t>(ctx, m, kKept);
     }
     if (m) {
       // no outdegree passes 2 sqrt(m): its vertices' degrees (octave ids: half of
@@ -1127,8 +1127,8 @@ void build_layout(tribit_ctx* ctx, tribit_graph* g, int layout) {
   hipStream_t s = ctx->stream;
   const uint64_t n = g->n, m = g->m;
   if (layout == TRIBIT_SCHED_PLAIN) {
-    DevBuf<uint2> rng_all(ctx, m ? m : 1);
-    DevBuf<uint64_t> wrow(ctx, n ? n : 1);
+    DevBuf<uint2> rng_all(ctx, m ? m : 1, kKept);
+    DevBuf<uint64_t> wrow(ctx, n ? n : 1, kKept);
     if (m) k_ranges_all<<<grid_for(m, kBlock), kBlock, 0, s>>>(g->row_ptr, g->col, m, rng_all.p);
     if (n) k_row_wplus<<<grid_for(n, kBlock), kBlock, 0, s>>>(g->row_ptr, g->col, n, wrow.p);
     TB_HIP(hipGetLastError());
@@ -1139,10 +1139,10 @@ void build_layout(tribit_ctx* ctx, tribit_graph* g, int layout) {
   }
   if (layout != TRIBIT_SCHED_DIRECTED) fail(TRIBIT_ERR_ARG, "no such range layout");
   const uint32_t end_bit = 32 + bits_for(n);
-  DevBuf<uint2> rng_dir(ctx, m ? m : 1);
-  DevBuf<uint32_t> pid_dir(ctx, m ? m : 1);
-  DevBuf<uint32_t> fw_ptr(ctx, n + 1), rv_ptr(ctx, n + 1);
-  DevBuf<uint64_t> w_fw(ctx, n), w_rv(ctx, n);
+  DevBuf<uint2> rng_dir(ctx, m ? m : 1, kKept);
+  DevBuf<uint32_t> pid_dir(ctx, m ? m : 1, kKept);
+  DevBuf<uint32_t> fw_ptr(ctx, n + 1, kKept), rv_ptr(ctx, n + 1, kKept);
+  DevBuf<uint64_t> w_fw(ctx, n, kKept), w_rv(ctx, n, kKept);
   uint32_t m_fwd = 0;
   k_fill_u64<<<grid_for(n, kBlock), kBlock, 0, s>>>(reinterpret_cast<unsigned long long*>(w_rv.p), n);
   if (m) {
@@ -1293,7 +1293,7 @@ void build_offdiag(tribit_ctx* ctx, const uint64_t* d_cols, uint64_t ncols, cons
   DevBuf<uint64_t> hk(ctx, nidxs ? nidxs : 1);
   const uint64_t mh = sort_unique(ctx, d_idxs, nidxs, n, hk.p, &bad);
   if (mh > 0xFFFFFFFFull) fail(TRIBIT_ERR_TOO_LARGE, "more than 2^32-1 index edges in one task");
-  DevBuf<uint32_t> col(ctx, mh ? mh : 1), row_ptr(ctx, n + 1);
+  DevBuf<uint32_t> col(ctx, mh ? mh : 1, kKept), row_ptr(ctx, n + 1, kKept);
   {
     DevBuf<uint32_t> odeg(ctx, n + 1);
     k_fill_u32<<<grid_for(n + 1, kBlock), kBlock, 0, s>>>(odeg.p, n + 1, 0u);
@@ -1333,9 +1333,9 @@ void build_offdiag(tribit_ctx* ctx, const uint64_t* d_cols, uint64_t ncols, cons
     mc = cnt;
   }
   if (bad) fail(TRIBIT_ERR_RANGE, "edge key is not (min < max < n)");
-  DevBuf<uint2> rng(ctx, mc ? mc : 1);
-  DevBuf<uint32_t> pid(ctx, mc ? mc : 1), fw_ptr(ctx, n + 1), rv_ptr(ctx, n + 1);
-  DevBuf<uint64_t> w_fw(ctx, n), w_rv(ctx, n);
+  DevBuf<uint2> rng(ctx, mc ? mc : 1, kKept);
+  DevBuf<uint32_t> pid(ctx, mc ? mc : 1, kKept), fw_ptr(ctx, n + 1, kKept), rv_ptr(ctx, n + 1, kKept);
+  DevBuf<uint64_t> w_fw(ctx, n, kKept), w_rv(ctx, n, kKept);
   {
     DevBuf<uint32_t> rv_cnt(ctx, n + 1);
     k_fill_u32<<<grid_for(n + 1, kBlock), kBlock, 0, s>>>(rv_cnt.p, n + 1, 0u);

@@ -122,7 +122,7 @@ void build_tiles(tribit_ctx* ctx, tribit_graph* g, int layout, int width) {
   tribit_graph::TileSet& T = g->tiles[set_of(width)];
   const uint64_t n = g->n, m = g->m;
   if (!T.ptr) {
-    DevBuf<uint32_t> tile_ptr(ctx, n + 1);
+    DevBuf<uint32_t> tile_ptr(ctx, n + 1, kKept);
     {
       DevBuf<uint32_t> tcnt(ctx, n + 1);
       tile_counts(ctx, g, width, tcnt.p);
@@ -137,8 +137,8 @@ void build_tiles(tribit_ctx* ctx, tribit_graph* g, int layout, int width) {
     TB_HIP(hipMemcpyAsync(&W, tile_ptr.p + n, 4, hipMemcpyDeviceToHost, s));
     ctx->sync();
     const uint64_t mbytes = (uint64_t)(W ? W : 1) * (width / 8);
-    DevBuf<uint32_t> blk(ctx, W ? W : 1), tidx(ctx, m ? m : 1);
-    DevBuf<uint8_t> mask(ctx, mbytes);
+    DevBuf<uint32_t> blk(ctx, W ? W : 1, kKept), tidx(ctx, m ? m : 1, kKept);
+    DevBuf<uint8_t> mask(ctx, mbytes, kKept);
     if (width == 32)
       k_tile_fill<5, uint32_t><<<grid_for(n, kTBlock), kTBlock, 0, s>>>(
           g->row_ptr, g->col, n, tile_ptr.p, blk.p, reinterpret_cast<uint32_t*>(mask.p), tidx.p);
@@ -158,7 +158,7 @@ void build_tiles(tribit_ctx* ctx, tribit_graph* g, int layout, int width) {
                                                                                                : g->rng_dir;
   uint2** dst = &T.trng[layout & 3];
   if (*dst || !src) return;
-  DevBuf<uint2> tr(ctx, m ? m : 1);
+  DevBuf<uint2> tr(ctx, m ? m : 1, kKept);
   if (m) k_tile_ranges<<<grid_for(m, kTBlock), kTBlock, 0, s>>>(src, m, T.idx, tr.p);
   TB_HIP(hipGetLastError());
   ctx->sync();
