@@ -82,3 +82,18 @@ def test_batch_rejects_bad_keys(gpu_ctx):
     with pytest.raises(tribit_amd.TribitError) as ei:
         gpu_ctx.batch_from_keys(bad, [3])
     assert ei.value.status == 4
+
+
+# tasks of launches of fewer blocks than sub-queues, of about as many, and of several claims a wave
+@pytest.mark.parametrize("count,size", [(1, 12), (9, 40), (20, 24), (22, 24), (300, 30), (4000, 20), (60, 400)])
+def test_batch_task_feed(gpu_ctx, oracle_mod, count, size):
+    """Every task of a batch launch is taken once, whatever share of the sub-queues other waves pass by."""
+    note(f"task feed: {count} graphs of {size} vertices")
+    keys = [graphs.random_graph(size, 0.4, 1000 + j) for j in range(count)]
+    want = [oracle_mod.count_keys(k, size) for k in keys]
+    with gpu_ctx.batch_from_keys(keys, [size] * count) as b:
+        for sched in ("wedge", "plain"):
+            for fl in (0, tribit_amd.FORCE_MULTI):
+                c, ci = b.count(sched=sched, repeats=3, flags=fl)
+                assert [int(x) for x in c] == want, (sched, fl)
+                assert ci["repeats_agree"]

@@ -38,6 +38,9 @@ constexpr uint32_t kWaveBatch = 16;      // most wave tasks taken per queue atom
 // Tasks per wave of launches too small to fill the chip. A task is a serial chain
 // of dependent loads (about 3 us), so more waves shorten the launch: 80K-edge
 // R-MAT, 16 and 4 tasks a wave 51 + 21 us, two 28 + 17 (outdeg <= 32, <= 256).
+// Batches of one and four Chung-Lu graphs, us a replay with 2 / 4 / 8 / 16 tasks a
+// wave: 342 / 333 / 373 / 476 and 375 / 353 / 380 / 481; from 16 graphs on the
+// grid is full and all take the same.
 constexpr uint32_t kTasksPerWave = 2;
 constexpr uint32_t kClaimsPerWave = 8;   // queue claims per wave of a wave launch (when tasks allow)
 constexpr uint32_t kChunk = 2048;        // probe-set chunk of class-3 rows
@@ -630,7 +633,11 @@ __device__ __forceinline__ uint32_t stream_tiles(const TileSrc& ts, const uint2*
 // graphs: an eighth of the eighth for each sub-queue 22.6 ms, single units dealt
 // out 18.6, runs 17.8). Workgroup b runs on XCD b % 8 and starts on sub-queue
 // b % kQueues, so each XCD streams the rows of its own graphs and its L2 is not
-// filled with the rows the other seven stream.
+// filled with the rows the other seven stream. For the same reason a wave passes
+// by a sub-queue whose own waves take what
+// is left in two claims: all waves claiming the launch's last units queued up on
+// their counters (48 and 64 graphs: 1.84 and 1.95 ms a replay, now 1.76 and 1.86;
+// with one claim left out 1.80 and 1.90, with four 1.91 and 1.85).
 struct TaskFeed {
   static_assert(kQueues == 64, "one lane per sub-queue");
   uint32_t* queue;
@@ -639,10 +646,12 @@ struct TaskFeed {
   uint32_t home, q;   // the block's sub-queue, the current one
   uint32_t c, cend;   // claimed units: numbers in the launch (contiguous mode) or in sub-queue q
   uint64_t dry;       // sub-queues this wave's claims found empty: each is tried in vain once at most
+  uint32_t spare;     // what is left of a sub-queue to its own waves; each has some in a grid of kQueues blocks
 
   __device__ TaskFeed(uint32_t* qs, uint32_t nt, uint32_t unit_, uint32_t claim_, bool contig_ = false)
       : queue(qs), ntasks(nt), unit(unit_), claim(claim_), contig(contig_), open(true), home(blockIdx.x % kQueues),
-        q(home), c(0), cend(0), dry(0) {}
+        q(home), c(0), cend(0), dry(0),
+        spare(contig_ && gridDim.x >= kQueues ? 2 * (gridDim.x * (blockDim.x / 64) / kQueues) : 0u) {}
 
   __device__ uint32_t eighth(uint32_t x) const { return (uint32_t)((uint64_t)((ntasks + unit - 1) / unit) * x / 8); }
 
@@ -667,8 +676,8 @@ struct TaskFeed {
         // lane p: the p-th sub-queue to try, the eight of the block's XCD first
         const uint32_t sq = ((home + (lane >> 3)) & 7) + 8 * (((home >> 3) + lane) & 7);
         const uint32_t v = __hip_atomic_load(queue + sq * kQStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const uint64_t left = __ballot(v < size_of(sq) && !((dry >> sq) & 1ull));
-        if (!left) return false;  // counters only grow: an empty sub-queue stays empty
+        const uint64_t left = __ballot(v + spare < size_of(sq) && !((dry >> sq) & 1ull));
+        if (!left) return false;  // counters only grow: nothing is left later either
         q = __builtin_amdgcn_readlane(sq, __ffsll((long long)left) - 1);
       }
       const uint32_t nq = size_of(q), by = contig ? 1u : claim;
