@@ -22,7 +22,6 @@ constexpr unsigned kBlock = 256;
 constexpr uint32_t kPartThreads = 512;
 constexpr uint32_t kPartItems = 12;                          // items per thread and tile
 constexpr uint32_t kPartTile = kPartThreads * kPartItems;    // 48 KiB of 8-byte items: two blocks per CU
-constexpr uint32_t kPartMaxBits = 11;                        // widest digit of one pass
 
 // A bijection of the W = 2 kb bit integers and its inverse (two rounds of xor
 // shift and odd multiplier, as integer finalisers do; the multipliers are
@@ -86,10 +85,16 @@ __device__ __forceinline__ uint32_t block_scan(uint32_t* h, uint32_t nd, uint32_
   return total;
 }
 
+// Whether a bucket overflowed (bit 1 of *flags): what is left of the partition is
+// then work for nothing. Best effort, one relaxed read per block.
+__device__ __forceinline__ bool overflowed(const uint32_t* flags) {
+  return (__hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 2u) != 0;
+}
+
 // Keys (min << 32) | max: checked (min < max < n, else *flags |= 1), sentinels
 // dropped, packed to W = 2 kb bits, mixed and spread by the high `bits` bits
 // over buckets of `cap` items (cursor: items per bucket; *flags |= 2 when one
-// overflows, whose items past the end are dropped).
+// overflows, whose items past the end are dropped, and later tiles with them).
 //
 // Bound by memory (16 bytes a key). A tile is grouped by digit in LDS first, so
 // a bucket receives runs of tile / 2^bits items (96 bytes at 512 buckets) from
@@ -101,14 +106,17 @@ __global__ void __launch_bounds__(kPartThreads) k_split_keys(const uint64_t* __r
   __shared__ uint64_t s_item[kPartTile];
   __shared__ uint16_t s_dig[kPartTile];
   __shared__ uint32_t s_wsum[kPartThreads / 64];
+  __shared__ bool s_stop;
   extern __shared__ uint32_t s_dyn[];
   const uint32_t nd = 1u << bits;
   uint32_t *hist = s_dyn, *rel = s_dyn + nd;
+  if (threadIdx.x == 0) s_stop = overflowed(flags);
   const uint32_t W = 2 * kb;
   const uint64_t mask = W >= 64 ? ~0ull : (1ull << W) - 1;
   const uint32_t shift = W - bits;
   for (uint32_t i = threadIdx.x; i < nd; i += kPartThreads) hist[i] = 0u;
   __syncthreads();
+  if (s_stop) return;
   uint64_t h[kPartItems];
   uint32_t dr[kPartItems];  // digit << 16 | rank in the tile; all ones: no item
   bool bad = false;
@@ -171,14 +179,17 @@ __global__ void __launch_bounds__(kPartThreads) k_split_bucket(const uint64_t* _
   __shared__ P s_item[kPartTile];
   __shared__ uint16_t s_dig[kPartTile];
   __shared__ uint32_t s_wsum[kPartThreads / 64];
+  __shared__ bool s_stop;
   extern __shared__ uint32_t s_dyn[];
   const uint32_t nd = 1u << bits, b1 = blockIdx.y;
   const uint64_t cnt = min((uint64_t)cnt1[b1], cap1);
   const uint64_t t0 = (uint64_t)blockIdx.x * kPartTile;
   if (t0 >= cnt) return;
   uint32_t *hist = s_dyn, *rel = s_dyn + nd;
+  if (threadIdx.x == 0) s_stop = overflowed(flags);
   for (uint32_t i = threadIdx.x; i < nd; i += kPartThreads) hist[i] = 0u;
   __syncthreads();
+  if (s_stop) return;
   in += (uint64_t)b1 * cap1;
   cursor += (uint64_t)b1 * nd;
   out += (uint64_t)b1 * nd * cap;
@@ -245,8 +256,10 @@ template <typename P, uint32_t GROUP>
 __global__ void __launch_bounds__(kPartThreads) k_distinct(const P* __restrict__ in, uint64_t cap,
                                                            const uint32_t* __restrict__ cnt, uint32_t nb, uint32_t kb,
                                                            uint32_t rbits, uint64_t* __restrict__ out,
+                                                           const uint32_t* __restrict__ flags,
                                                            uint32_t* __restrict__ total, uint64_t band_ids,
                                                            unsigned long long* __restrict__ band) {
+  if (overflowed(flags)) return;  // set before this launch or not at all
   constexpr P kFree = (P)~(P)0;
   __shared__ P s_set[kSetSlots];
   __shared__ P s_list[GROUP * kBucketCap];
@@ -320,7 +333,8 @@ __global__ void k_part_zero(uint32_t* __restrict__ p, uint64_t n) {
 // Distinct keys of d_keys (as given, (min << 32) | max with sentinels), packed
 // (min << kb) | max, in any order, into out (room for nk). One device read-back.
 // Returns false when a bucket overflowed (keys repeated so often that hashing
-// cannot spread them): nothing is in `out` then, and the caller sorts.
+// cannot spread them): nothing is in `out` then, and the caller sorts. The passes
+// end early then: the 300M keys of 100K edges cost the time of the first one.
 bool distinct_keys(tribit_ctx* ctx, const uint64_t* d_keys, uint64_t nk, uint64_t n, uint32_t kb, uint64_t* out,
                    uint64_t* m, bool* bad, uint64_t band_ids, uint64_t* band) {
   hipStream_t s = ctx->stream;
@@ -330,7 +344,6 @@ bool distinct_keys(tribit_ctx* ctx, const uint64_t* d_keys, uint64_t nk, uint64_
   B = std::min(B, W);
   const bool two = B > 9;
   const uint32_t b1 = two ? (B + 1) / 2 : B, b2 = B - b1, r = W - B;
-  if (b1 > kPartMaxBits) return false;
   const uint32_t nd1 = 1u << b1;
   const uint64_t nb = 1ull << B;
   const uint64_t cap1 = two ? nk / nd1 + nk / nd1 / 8 + 4096 : kBucketCap;
@@ -355,19 +368,19 @@ bool distinct_keys(tribit_ctx* ctx, const uint64_t* d_keys, uint64_t nk, uint64_
                                                                  cur.p + nd1, tail);
       reg1.reset();
       k_distinct<uint32_t, 4><<<std::min<uint32_t>(grid_for(nb, 4), 8 * cus), kPartThreads, 0, s>>>(
-          reg4.p, kBucketCap, cur.p + nd1, (uint32_t)nb, kb, r, out, tail + 1, band_ids, band ? d_band : nullptr);
+          reg4.p, kBucketCap, cur.p + nd1, (uint32_t)nb, kb, r, out, tail, tail + 1, band_ids, band ? d_band : nullptr);
     } else {
       reg8 = DevBuf<uint64_t>(ctx, nb * kBucketCap);
       k_split_bucket<uint64_t><<<grid, kPartThreads, 8 * nd2, s>>>(reg1.p, cap1, cur.p, b2, r, kBucketCap, reg8.p,
                                                                  cur.p + nd1, tail);
       reg1.reset();
       k_distinct<uint64_t, 1><<<std::min<uint32_t>((uint32_t)nb, 8 * cus), kPartThreads, 0, s>>>(
-          reg8.p, kBucketCap, cur.p + nd1, (uint32_t)nb, kb, r, out, tail + 1, band_ids, band ? d_band : nullptr);
+          reg8.p, kBucketCap, cur.p + nd1, (uint32_t)nb, kb, r, out, tail, tail + 1, band_ids, band ? d_band : nullptr);
     }
   } else {
     // the first pass kept whole mixed keys: the bucket bits are already in them
     k_distinct<uint64_t, 1><<<std::min<uint32_t>((uint32_t)nb, 8 * cus), kPartThreads, 0, s>>>(
-        reg1.p, cap1, cur.p, (uint32_t)nb, kb, 64, out, tail + 1, band_ids, band ? d_band : nullptr);
+        reg1.p, cap1, cur.p, (uint32_t)nb, kb, 64, out, tail, tail + 1, band_ids, band ? d_band : nullptr);
   }
   uint32_t h[4] = {0, 0, 0, 0};
   TB_HIP(hipMemcpyAsync(h, tail, sizeof(h), hipMemcpyDeviceToHost, s));
