@@ -265,10 +265,10 @@ int tribit_count(tribit_ctx* ctx, tribit_graph* g, const tribit_count_opts* opts
  * (code under HIP graph capture, serving loops, harnesses that forbid
  * hipMalloc). tribit_count with no allocation and no free: the schedule's
  * task lists, its counters and the result live in one scratch array of
- * tribit_noalloc_scratch_bytes() (128 MiB) per GPU, file-scope device memory
- * held until the process ends. opts->sched must be PLAIN, DIRECTED or WEDGE
- * (LEARNED judges candidates and builds tables: TRIBIT_ERR_ARG), with no dense
- * core and no TRIBIT_COUNT_FORCE_TILES. A schedule needing more scratch than
+ * tribit_noalloc_scratch_bytes() (128 MiB; 49,920 bytes more for the counters)
+ * per GPU, file-scope device memory held until the process ends. opts->sched
+ * must be PLAIN, DIRECTED or WEDGE (LEARNED judges candidates and builds tables:
+ * TRIBIT_ERR_ARG), with no dense core and no TRIBIT_COUNT_FORCE_TILES. A schedule needing more scratch than
  * the array fails with TRIBIT_ERR_TOO_LARGE (R-MAT scale 25, 5.1M tasks, uses
  * about 90 MiB). Every call on one GPU shares that GPU's array and clears
  * what it needs at the start: calls that overlap on one GPU (two threads or

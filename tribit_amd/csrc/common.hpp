@@ -273,7 +273,7 @@ struct tribit_batch {
   std::vector<Part> parts;
   std::vector<uint64_t> n, m;             // per graph: vertices, simple undirected edges
   unsigned long long* gcount = nullptr;   // device: per-graph triangle counts
-  unsigned long long* scratch = nullptr;  // device: 8 words per part (count, fallbacks, queues)
+  unsigned long long* scratch = nullptr;  // device: kCountScratch words per part (results, queues)
   hipGraph_t graph = nullptr;             // captured counting launches of all parts
   hipGraphExec_t exec = nullptr;
   int sched = -1, flags = 0;              // what the schedules / capture were built for

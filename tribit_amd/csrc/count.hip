@@ -2521,10 +2521,12 @@ bool judged_known(const tribit_ctx* ctx, const tribit_graph* g, const tribit_cou
 // ends. Host code never passes the symbol itself (on the host it names a
 // stand-in, not device memory): noalloc_init looks its device address up once
 // per context, with the context's device current, and kernels get that.
+// The schedules that fit are those whose lists fit the documented size beside the
+// counters of eight sub-queues a slot and a plan's table, which it held once; the
+// counters of kQueues sub-queues take more and lie behind the lists.
 constexpr uint64_t kNoAllocScratchBytes = 128ull << 20;
-// The schedules that fit are those whose lists fit the documented size beside
-// 17,664 bytes; the counters' 64 sub-queues per slot take more, behind it.
-constexpr uint64_t kNoAllocSchedule = kNoAllocScratchBytes - 17664;
+constexpr uint64_t kEightQueueCounters = (32 + 8 * 8 * 32) * sizeof(unsigned long long), kTableSlice = 1024;
+constexpr uint64_t kNoAllocSchedule = kNoAllocScratchBytes - kEightQueueCounters - kTableSlice;
 constexpr uint64_t kNoAllocBytes = kNoAllocSchedule + kCountScratch * sizeof(unsigned long long);
 static __device__ __align__(256) unsigned char noalloc_scratch[kNoAllocBytes];
 

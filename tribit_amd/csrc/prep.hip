@@ -10,7 +10,8 @@
 //   --rows by partition, else a sort--> row_ptr[n+1] (u32), col[m] (u32, ascending
 //   within a row)
 //   W+ = sum over v of indeg(v) * outdeg(v); wedge ranges (relabelled graphs)
-// Every launch is a 1-D grid of 256-thread blocks (4 waves).
+// Launches are 1-D grids of 256-thread blocks (4 waves); sorts and scans by one
+// workgroup take 1024 threads.
 #include <cmath>
 #include <cstring>
 #include <rocprim/block/block_radix_sort.hpp>
@@ -237,7 +238,7 @@ inline unsigned totals_grid(uint64_t n) {
 // Edges {a, b}, a < b, of the deduplicated keys (a << kb) | b that join ids
 // less than kBandIds apart, summed into *out: two keys per 16-byte load over a
 // grid of at most kBandBlocks blocks, one atomic per block. keys is 256-byte
-// aligned (hipMallocAsync).
+// aligned, as every block of the context's pool.
 constexpr uint64_t kBandIds = 512;
 constexpr unsigned kBandBlocks = 4096;
 __global__ void __launch_bounds__(kBlock) k_band_edges(const uint64_t* __restrict__ keys, uint64_t m, uint32_t kb,
