@@ -317,3 +317,27 @@ def test_degrees_of_more_than_2_31_edges(gpu_ctx):
         i = g.info()
         assert (i["m"], i["wplus"]) == (2299981280, 210131079941)
         assert g.count("wedge").triangles == 3433745
+
+
+def test_records_that_need_the_largest_outdegree(gpu_ctx):
+    """More than 2^28 edges over 2^26 ids: an arc's packed record fits only with the real largest outdegree, read back
+    first. The wedge ranges unpacked from it against the direction-split ranges, which do not use them."""
+    note("er of 272M keys over 2^26 ids")
+    with gpu_ctx.gen_er(1 << 26, 272_000_000, seed=3) as g:
+        assert g.info()["m"] > 1 << 28
+        assert g.count("wedge").triangles == g.count("directed").triangles > 0
+
+
+def test_memory_kept_by_another_context(gpu_ctx):
+    """137 GB freed and kept by one context leave room for 206 GB in another."""
+    note("device keys of 137 and 206 GB")
+    import ctypes
+
+    def keys(ctx, ef):
+        d, n = ctypes.c_void_p(), ctypes.c_uint64()
+        assert ctx.lib.tribit_gen_rmat(ctx.h, 31, ef, 0.57, 0.19, 0.19, 1, ctypes.byref(d), ctypes.byref(n)) == 0
+        ctx.lib.tribit_free_device_keys(ctx.h, d)
+
+    with tribit_amd.Context(0) as a, tribit_amd.Context(0) as b:
+        keys(a, 8)
+        keys(b, 12)
