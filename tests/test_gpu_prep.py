@@ -341,3 +341,28 @@ def test_memory_kept_by_another_context(gpu_ctx):
     with tribit_amd.Context(0) as a, tribit_amd.Context(0) as b:
         keys(a, 8)
         keys(b, 12)
+
+
+# edges for a sort by one workgroup and for a partition of the rows, and few and many of them for the degrees
+@pytest.mark.parametrize("relabel,m,clique", [(0, 20000, 200), (1, 2000, 40), (1, 300000, 200), (2, 20000, 200)])
+def test_more_than_2_31_ids(gpu_ctx, oracle_mod, relabel, m, clique):
+    """Ids past 2^31, whose cleared spans have more words than a launch may have threads: counts equal those of the
+    same edges over their own ids."""
+    n = (1 << 31) + 1000
+    note(f"{m} edges over {n} ids, id order {relabel}")
+    rng = np.random.default_rng(m)
+    ids = np.unique(np.concatenate([rng.integers(0, n, clique), n - 1 - rng.integers(0, 1000, 60)]))
+    i, j = np.triu_indices(ids.size, 1)
+    a, b = np.concatenate([ids[i], rng.integers(0, n, m)]), np.concatenate([ids[j], rng.integers(0, n, m)])
+    small = np.unique(np.concatenate([a, b]), return_inverse=True)[1]
+    x, y = small[:a.size], small[a.size:]
+    pack = lambda u, v: ((np.minimum(u, v) << 32) | np.maximum(u, v))[u != v].astype(np.uint64)  # noqa: E731
+    want = oracle_mod.count_keys(pack(x, y), int(small.max()) + 1)
+    assert want >= ids.size * (ids.size - 1) * (ids.size - 2) // 6
+    gpu_ctx.set_relabel(relabel)
+    try:
+        with gpu_ctx.graph_from_keys(pack(a, b), n) as g:
+            scheds = ("plain", "directed") if relabel == 0 else ("wedge", "directed")
+            assert [g.count(s).triangles for s in scheds] == [want, want]
+    finally:
+        gpu_ctx.set_relabel("auto")

@@ -995,7 +995,7 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
     DevBuf<uint32_t> lab_buf(ctx, n + skew);
     uint32_t* lab = lab_buf.p + skew;
     take_zeroed();
-    k_scatter_labels<<<grid_for(std::max(n, zero.most()), kBlock), kBlock, 0, s>>>(labels.p, n, lab, zero);
+    k_scatter_labels<<<grid_for(zero.grid_items(n), kBlock), kBlock, 0, s>>>(labels.p, n, lab, zero);
     take_columns();
     // rows by partition, but a sort by one workgroup where that suffices (two
     // launches of 35 us against five of 31) and for more edges than the slots cover
@@ -1014,7 +1014,7 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
   } else {
     if (m) okeys = DevBuf<uint64_t>(ctx, m);
     take_zeroed();
-    k_orient<<<grid_for(std::max(m, zero.most()), kBlock), kBlock, 0, s>>>(uniq.p, m, deg.p, kb, okeys.p, zero);
+    k_orient<<<grid_for(zero.grid_items(m), kBlock), kBlock, 0, s>>>(uniq.p, m, deg.p, kb, okeys.p, zero);
     take_columns();
   }
   if (m && !sorted) {

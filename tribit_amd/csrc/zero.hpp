@@ -12,16 +12,21 @@ namespace tb {
 // Ids in col16: m rounded up to whole dwords, and one more dword.
 __host__ __device__ inline uint64_t col16_ids(uint64_t m) { return ((m + 1) / 2 + 1) * 2; }
 
-// Zeroed on the way by a kernel whose grid covers them: one launch fewer each.
+// Zeroed on the way by a kernel over `items` of its own: one launch fewer each.
+// A launch has fewer than 2^32 threads, so from 2^30 ids on a thread clears
+// several words of the longest span (8 bytes an id).
 struct ZeroSpans {
   uint32_t* p[3];
   uint64_t n[3];
   __device__ __forceinline__ void clear(uint64_t i) const {
+    const uint64_t threads = (uint64_t)gridDim.x * blockDim.x;
 #pragma unroll
     for (int k = 0; k < 3; ++k)
-      if (i < n[k]) p[k][i] = 0u;
+      for (uint64_t j = i; j < n[k]; j += threads) p[k][j] = 0u;
   }
-  uint64_t most() const { return std::max(n[0], std::max(n[1], n[2])); }
+  uint64_t grid_items(uint64_t items) const {
+    return std::max(items, std::min<uint64_t>(std::max(n[0], std::max(n[1], n[2])), 1ull << 31));
+  }
 };
 
 // out[0, n]: the exclusive scan of f(0), ..., f(n - 1), by one workgroup in one
