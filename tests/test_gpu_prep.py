@@ -366,3 +366,14 @@ def test_more_than_2_31_ids(gpu_ctx, oracle_mod, relabel, m, clique):
             assert [g.count(s).triangles for s in scheds] == [want, want]
     finally:
         gpu_ctx.set_relabel("auto")
+
+
+def test_degrees_of_one_full_id_group(gpu_ctx):
+    """The complete graph on 65,535 ids, whose 4,294,770,690 endpoints are one group's: W+, which every degree enters,
+    is its number of triangles."""
+    n = 65535
+    note("complete graph on 65535 ids")
+    with gpu_ctx.gen_sbm(1, n, 1.0, 0.0, 1) as g:
+        i = g.info()
+        assert (i["m"], i["max_outdeg"]) == (n * (n - 1) // 2, n - 1)
+        assert i["wplus"] == n * (n - 1) * (n - 2) // 6
