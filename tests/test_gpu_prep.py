@@ -377,3 +377,43 @@ def test_degrees_of_one_full_id_group(gpu_ctx):
         i = g.info()
         assert (i["m"], i["max_outdeg"]) == (n * (n - 1) // 2, n - 1)
         assert i["wplus"] == n * (n - 1) * (n - 2) // 6
+
+
+def test_keys_that_the_caller_allocated(gpu_ctx, oracle_mod):
+    """tribit_graph_from_device_keys frees the keys: those of the runtime's allocator too, and another context's."""
+    import ctypes
+
+    note("caller's device keys")
+    hip = ctypes.CDLL("libamdhip64.so")
+    keys = oracle_mod.gen_rmat(12, 8, seed=4)
+    want = oracle_mod.count_keys(keys, 1 << 12)
+
+    def build(d):
+        g = ctypes.c_void_p()
+        assert gpu_ctx.lib.tribit_graph_from_device_keys(gpu_ctx.h, d, keys.size, 1 << 12, ctypes.byref(g)) == 0
+        with tribit_amd.Graph(gpu_ctx, g.value) as graph:
+            assert graph.count("wedge").triangles == want
+
+    def free_bytes():
+        f, t = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipDeviceSynchronize() == 0 and hip.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value
+
+    left = []
+    for _ in range(3):  # the first pass takes the pool's own memory
+        d = ctypes.c_void_p()
+        assert hip.hipMalloc(ctypes.byref(d), ctypes.c_size_t(4 << 30)) == 0
+        assert hip.hipMemcpy(d, keys.ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(8 * keys.size), 1) == 0
+        build(d)
+        left.append(free_bytes())
+    assert left[2] > left[0] - (1 << 30)
+
+    with tribit_amd.Context(0) as other:
+        d, n = ctypes.c_void_p(), ctypes.c_uint64()
+        assert other.lib.tribit_gen_rmat(other.h, 12, 8, 0.57, 0.19, 0.19, 4, ctypes.byref(d), ctypes.byref(n)) == 0
+        assert n.value == keys.size and hip.hipDeviceSynchronize() == 0
+        build(d)
+        again = ctypes.c_void_p()
+        assert other.lib.tribit_gen_rmat(other.h, 12, 8, 0.57, 0.19, 0.19, 4, ctypes.byref(again), ctypes.byref(n)) == 0
+        assert again.value == d.value  # the block was free again
+        other.lib.tribit_free_device_keys(other.h, again)

@@ -120,6 +120,22 @@ int main() {
     b.release();
     CHECK(mapped().empty());
   }
+  {  // another context's block goes back to it, memory of no pool to the runtime; an inner address to nobody
+    tb::DevicePool a, b;
+    a.init(0, nullptr, kTotal);
+    b.init(0, nullptr, kTotal);
+    void* p = a.alloc(64 * MiB, false);
+    void* foreign = nullptr;
+    CHECK(hipMallocAsync(&foreign, MiB, nullptr) == hipSuccess);
+    const uint64_t was = mapped_bytes();
+    b.free((char*)p + 4096);
+    b.free(p);
+    CHECK(mapped_bytes() == was && a.alloc(64 * MiB, false) == p);
+    b.free(foreign);
+    CHECK(mapped_bytes() == was - MiB);
+    a.release();
+    b.release();
+  }
   {  // the last megabytes: a segment smaller than usual, then a free piece of any class
     tb::DevicePool p;
     p.init(0, nullptr, kTotal);

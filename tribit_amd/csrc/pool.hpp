@@ -71,23 +71,24 @@ class DevicePool {
     return nullptr;
   }
 
+  // Memory of another context's pool goes back there once this context's stream
+  // is done with it, memory of no pool (keys that the caller allocated) to the
+  // runtime.
   void free(void* ptr) {
-    std::lock_guard<std::mutex> lock(mu_);
-    auto it = blocks_.find(reinterpret_cast<uintptr_t>(ptr));
-    if (it == blocks_.end() || it->second.free) return;
-    it->second.free = true;
-    free_bytes_ += it->second.size;
-    auto next = std::next(it);
-    if (next != blocks_.end() && next->second.free && next->second.seg == it->second.seg) merge(it, next);
-    if (it != blocks_.begin()) {
-      auto prev = std::prev(it);
-      if (prev->second.free && prev->second.seg == it->second.seg) {
-        merge(prev, it);
-        it = prev;
-      }
+    const uintptr_t a = reinterpret_cast<uintptr_t>(ptr);
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      if (owns(a)) return put(a);
     }
-    free_[it->second.cls].insert({it->second.size, it->first});
-    if (free_bytes_ > keep_) give_back(keep_);
+    std::lock_guard<std::mutex> lock(all_mu());
+    for (DevicePool* p : all()) {
+      if (p == this) continue;
+      std::lock_guard<std::mutex> theirs(p->mu_);
+      if (!p->owns(a)) continue;
+      (void)hipStreamSynchronize(stream_);
+      return p->put(a);
+    }
+    if (hipFreeAsync(ptr, stream_) != hipSuccess) (void)hipGetLastError();
   }
 
   // No segment is given back while this lives: around a capture of the stream,
@@ -145,6 +146,30 @@ class DevicePool {
     }
     it = free_[cls].lower_bound({bytes, 0});
     return it == free_[cls].end() ? nullptr : take(it, cls, bytes, true);
+  }
+
+  bool owns(uintptr_t a) const {  // anywhere in a segment
+    auto s = segs_.upper_bound(a);
+    return s != segs_.begin() && a < std::prev(s)->first + std::prev(s)->second;
+  }
+
+  // The block at `a` is free from now on (no block, or a free one: nothing happens).
+  void put(uintptr_t a) {
+    auto it = blocks_.find(a);
+    if (it == blocks_.end() || it->second.free) return;
+    it->second.free = true;
+    free_bytes_ += it->second.size;
+    auto next = std::next(it);
+    if (next != blocks_.end() && next->second.free && next->second.seg == it->second.seg) merge(it, next);
+    if (it != blocks_.begin()) {
+      auto prev = std::prev(it);
+      if (prev->second.free && prev->second.seg == it->second.seg) {
+        merge(prev, it);
+        it = prev;
+      }
+    }
+    free_[it->second.cls].insert({it->second.size, it->first});
+    if (free_bytes_ > keep_) give_back(keep_);
   }
 
   bool whole_segment(const std::pair<uint64_t, uintptr_t>& f) const {
