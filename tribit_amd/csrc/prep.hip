@@ -830,10 +830,10 @@ static void sort_keys(tribit_ctx* ctx, const uint64_t* in, uint64_t* out, uint64
 // Where the labels of kSkewIds ids or more begin in their buffer (in ids): an
 // R-MAT graph's frequent endpoints are ids with few set bits, and the label
 // gathers of k_row_split met in few memory channels when the array began at a
-// multiple of 2 MiB (scale 25: 13.6 ms; 11.8 from 1 MiB past one; 11.0 from an
-// offset of many set bits). Smaller label arrays stay in L2.
+// multiple of 2 MiB (scale 25: 13.6 ms; 12.0 from 1 MiB past one; 11.0 to 11.4
+// from an offset of many set bits). Smaller label arrays stay in L2.
 constexpr uint64_t kSkewIds = 1ull << 20;
-constexpr uint64_t kLabelSkew = 0x16A200 / 4;
+constexpr uint64_t kLabelSkew = 0x1D9500 / 4;
 
 void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n, tribit_graph* g, int relabel_opt) {
   if (relabel_opt < 0) relabel_opt = ctx->relabel;

@@ -4,7 +4,7 @@
 // No counterpart in the reference. A radix sort of the arcs (50 bits at 2^25 ids)
 // streams them eight times through HBM after a pass that only turns edges into
 // arcs, and a pass that splits them follows: 34 ms for the 523M edges of R-MAT
-// scale 25, where the kernels here take 25.6; at 2^13 ids and 80K edges 13 launches
+// scale 25, where the kernels here take 25.9; at 2^13 ids and 80K edges 13 launches
 // of 60 us against five of 31. Rows have a known upper bound: in degree order no
 // outdegree passes deg(u) nor 2 sqrt(m) (the vertices above u have at least its
 // degree, octave ids half of it), so the scan P of min(deg(u), 2 sqrt(m)) gives
@@ -161,7 +161,7 @@ __device__ __forceinline__ void row_tile(RowLds<ITEMS>& s, const uint64_t (&h)[I
 
 // First pass: every distinct edge becomes its arc u -> v, u < v the new ids,
 // packed (u << kb) | v, in its slot. Bound by the two label gathers per edge (the
-// 134 MB of labels at 2^25 ids sit in the last-level cache): 10.7 ms for 523M
+// 134 MB of labels at 2^25 ids sit in the last-level cache): 11.0 to 11.4 ms for 523M
 // edges, where the gathers alone took 13.1 with one edge per thread.
 template <uint32_t ITEMS>
 __global__ void __launch_bounds__(kRowThreads) k_row_split(const uint64_t* __restrict__ keys, uint64_t m,
