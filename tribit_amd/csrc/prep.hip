@@ -962,8 +962,8 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
   const auto take_zeroed = [&] {  // odeg, st and w_sfx, cleared by the next launch
     odeg = DevBuf<uint32_t>(ctx, n + 1);
     if (relabel) w_sfx = DevBuf<uint64_t>(ctx, n, kKept);
-    zero = {{odeg.p, reinterpret_cast<uint32_t*>(st.p), reinterpret_cast<uint32_t*>(w_sfx.p)},
-            {n + 1, sizeof(RowStats) / 4, relabel ? 2 * n : 0}};
+    zero = ZeroSpans{{odeg.p, reinterpret_cast<uint32_t*>(st.p), reinterpret_cast<uint32_t*>(w_sfx.p)},
+                     {n + 1, sizeof(RowStats) / 4, relabel ? 2 * n : 0}};
   };
   // 4-6. the arcs sorted by (u, v) into the CSR
   const bool narrow = relabel && m && m < (1ull << 30);
@@ -995,7 +995,8 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
     DevBuf<uint32_t> lab_buf(ctx, n + skew);
     uint32_t* lab = lab_buf.p + skew;
     take_zeroed();
-    k_scatter_labels<<<grid_for(zero.grid_items(n), kBlock), kBlock, 0, s>>>(labels.p, n, lab, zero);
+    const unsigned grid = grid_for(zero.grid_items(n), kBlock);
+    k_scatter_labels<<<grid, kBlock, 0, s>>>(labels.p, n, lab, zero);
     take_columns();
     // rows by partition, but a sort by one workgroup where that suffices (two
     // launches of 35 us against five of 31) and for more edges than the slots cover
@@ -1014,7 +1015,8 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
   } else {
     if (m) okeys = DevBuf<uint64_t>(ctx, m);
     take_zeroed();
-    k_orient<<<grid_for(zero.grid_items(m), kBlock), kBlock, 0, s>>>(uniq.p, m, deg.p, kb, okeys.p, zero);
+    const unsigned grid = grid_for(zero.grid_items(m), kBlock);
+    k_orient<<<grid, kBlock, 0, s>>>(uniq.p, m, deg.p, kb, okeys.p, zero);
     take_columns();
   }
   if (m && !sorted) {

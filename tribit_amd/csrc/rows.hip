@@ -418,13 +418,13 @@ void build_rows(tribit_ctx* ctx, const uint64_t* edges, uint64_t m, const uint32
   if (two) {
     first1 = DevBuf<uint32_t>(ctx, nd1 + 1);
     cnt1 = DevBuf<uint32_t>(ctx, nd1);
-    const ZeroSpans z{{cnt1.p, nullptr, nullptr}, {nd1, 0, 0}};
-    k_row_slots<<<grid_for(z.grid_items(n + 1), kBlock), kBlock, 0, s>>>(P.p, n, limit, qb1, first1.p,
-                                                                                        z);
+    ZeroSpans z{{cnt1.p, nullptr, nullptr}, {nd1, 0, 0}};
+    const unsigned grid = grid_for(z.grid_items(n + 1), kBlock);
+    k_row_slots<<<grid, kBlock, 0, s>>>(P.p, n, limit, qb1, first1.p, z);
   }
-  const ZeroSpans z{{cnt.p, nullptr, nullptr}, {nslots, 0, 0}};
-  k_row_slots<<<grid_for(z.grid_items(n + 1), kBlock), kBlock, 0, s>>>(P.p, n, limit, qb,
-                                                                                      first.p, z);
+  ZeroSpans z{{cnt.p, nullptr, nullptr}, {nslots, 0, 0}};
+  const unsigned grid = grid_for(z.grid_items(n + 1), kBlock);
+  k_row_slots<<<grid, kBlock, 0, s>>>(P.p, n, limit, qb, first.p, z);
   DevBuf<uint64_t> b1(ctx, limit), b2;
   if (two) b2 = DevBuf<uint64_t>(ctx, limit);
   const auto split = [&](auto items) {

@@ -18,14 +18,21 @@ __host__ __device__ inline uint64_t col16_ids(uint64_t m) { return ((m + 1) / 2 
 struct ZeroSpans {
   uint32_t* p[3];
   uint64_t n[3];
+  bool more = false;  // a span has more words than the launch has threads
   __device__ __forceinline__ void clear(uint64_t i) const {
-    const uint64_t threads = (uint64_t)gridDim.x * blockDim.x;
 #pragma unroll
     for (int k = 0; k < 3; ++k)
-      for (uint64_t j = i; j < n[k]; j += threads) p[k][j] = 0u;
+      if (i < n[k]) p[k][i] = 0u;
+    if (!more) return;
+    const uint64_t threads = (uint64_t)gridDim.x * blockDim.x;
+    for (int k = 0; k < 3; ++k)
+      for (uint64_t j = i + threads; j < n[k]; j += threads) p[k][j] = 0u;
   }
-  uint64_t grid_items(uint64_t items) const {
-    return std::max(items, std::min<uint64_t>(std::max(n[0], std::max(n[1], n[2])), 1ull << 31));
+  uint64_t grid_items(uint64_t items) {
+    const uint64_t most = std::max(n[0], std::max(n[1], n[2]));
+    const uint64_t all = std::max(items, std::min<uint64_t>(most, 1ull << 31));
+    more = most > all;
+    return all;
   }
 };
 
