@@ -148,6 +148,15 @@ struct DevBuf {
 namespace tb {
 constexpr bool kKept = true;  // of a DevBuf that an object takes over (release)
 
+// f(temporary storage, its size): rocPRIM's two calls, with the storage between them.
+template <typename F>
+void with_temp(tribit_ctx* ctx, F&& f) {
+  size_t bytes = 0;
+  TB_HIP(f(nullptr, bytes));
+  DevBuf<uint8_t> tmp(ctx, bytes ? bytes : 8);
+  TB_HIP(f(tmp.p, bytes));
+}
+
 struct BucketCache;
 
 // Device counters of one count, none of them sharing a 128-byte line with
@@ -304,6 +313,14 @@ void gen_rmat(tribit_ctx* ctx, uint32_t scale, uint32_t ef, double a, double b, 
               uint64_t* d_keys);
 void gen_er(tribit_ctx* ctx, uint64_t n, uint64_t nsamples, uint64_t seed, uint64_t* d_keys);
 void rmat_thresholds(double a, double b, double c, uint32_t t[3]);
+// sort_ids.hip, sort_records.hip, sort_keys.hip: rocPRIM's device-wide sorts, in
+// files of their own because a file's device code is loaded when its first kernel
+// runs (a fresh process's first graph of 2^13 ids 16 ms, 48 with the sorts in prep.hip).
+void sort_ids_device(tribit_ctx* ctx, const uint32_t* in, uint32_t* out, uint32_t* order, uint64_t n, uint32_t bits);
+void sort_records_device(tribit_ctx* ctx, const uint32_t* in, uint32_t* out, const uint64_t* vin, uint64_t* vout,
+                         uint64_t n, uint32_t bits);
+void sort_keys_device(tribit_ctx* ctx, const uint64_t* in, uint64_t* out, uint64_t n, uint32_t end_bit);
+void unique_device(tribit_ctx* ctx, const uint64_t* in, uint64_t* out, uint64_t* count, uint64_t n);
 // partition.hip
 bool distinct_keys(tribit_ctx* ctx, const uint64_t* d_keys, uint64_t nk, uint64_t n, uint32_t kb, uint64_t* out,
                    uint64_t* m, bool* bad, uint64_t band_ids, uint64_t* band);

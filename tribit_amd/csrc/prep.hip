@@ -15,9 +15,7 @@
 #include <cmath>
 #include <cstring>
 #include <rocprim/block/block_radix_sort.hpp>
-#include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
-#include <rocprim/device/device_select.hpp>
 #include <rocprim/iterator/counting_iterator.hpp>
 #include <rocprim/iterator/transform_iterator.hpp>
 
@@ -669,37 +667,6 @@ __global__ void k_add_u32(uint32_t* __restrict__ p, uint64_t n, uint32_t v) {
   if (i < n) p[i] += v;
 }
 
-template <typename F>
-static void with_temp(tribit_ctx* ctx, F&& f) {
-  size_t bytes = 0;
-  TB_HIP(f(nullptr, bytes));
-  DevBuf<uint8_t> tmp(ctx, bytes ? bytes : 8);
-  TB_HIP(f(tmp.p, bytes));
-}
-
-// 9-bit digits for the sorts of 32-bit ids (three passes instead of four for
-// ids below 2^27). Measured on MI355X over 2^29 random 25-bit keys: pairs
-// with 32-bit values 14.7 -> 11.5 ms, keys alone 9.6 -> 8.0 ms. The 64-bit
-// key sorts keep rocPRIM's 8-bit digits (9 bits: 22.1 -> 23.4 ms; 10 bits
-// slower still).
-using IdSortConfig = rocprim::radix_sort_config<
-    rocprim::default_config, rocprim::default_config,
-    rocprim::radix_sort_onesweep_config<rocprim::kernel_config<1024, 16>, rocprim::kernel_config<1024, 16>, 9,
-                                        rocprim::block_radix_rank_algorithm::match>>;
-// rocPRIM merges blocks instead of sweeping digits up to 2^20 items: a launch per
-// doubling, each over all items. Digits of 8 bits in small tiles (two or three
-// passes of 7 to 14 us) are faster from kFewSort16 and kFewSort items on; whole builds with
-// digits / with merges, us: 40K ids 65K edges 222 / 226, 100K 228 / 241, 300K 326 /
-// 399, 1M 425 / 533; 1M ids 65K edges 291 / 344, 1M 546 / 703. Keys of more than 16
-// bits take a third pass: 250K ids 40K edges 282 / 268, 160K 327 / 329. Beyond 2^20
-// items the larger tiles of IdSortConfig win: 150K ids 4M edges 863 / 774.
-constexpr uint64_t kFewSort16 = 1ull << 16, kFewSort = 1ull << 18, kFewSortEnd = 1ull << 20;
-using FewSortConfig = rocprim::radix_sort_config<
-    rocprim::default_config, rocprim::default_config,
-    rocprim::radix_sort_onesweep_config<rocprim::kernel_config<512, 8>, rocprim::kernel_config<512, 8>, 8,
-                                        rocprim::block_radix_rank_algorithm::match>,
-    0>;
-
 // Sorts and scans of at most kSmallSort items: one workgroup, one launch. The
 // device-wide ones are seven or eight launches at these sizes (a block sort and
 // its merge steps), about 7 us each, and most of what a small graph's
@@ -754,26 +721,19 @@ __global__ void __launch_bounds__(kSmallThreads) k_sort_small_keys(const uint64_
   }
 }
 
-// values null: the items' numbers
-template <typename Config, typename V>
-static void sort_pairs(tribit_ctx* ctx, const uint32_t* in, uint32_t* out, const V* vin, V* vout, uint64_t n,
-                       uint32_t bits) {
-  if (n <= kSmallSort) {
-    k_sort_small<uint32_t, V><<<1, kSmallThreads, 0, ctx->stream>>>(in, out, vin, vout, (uint32_t)n, bits);
-    return;
-  }
-  const auto sort = [&](auto config) {
-    using C = decltype(config);
-    with_temp(ctx, [&](void* t, size_t& b) {
-      if (vin) return rocprim::radix_sort_pairs<C>(t, b, in, out, vin, vout, (size_t)n, 0u, bits, ctx->stream);
-      return rocprim::radix_sort_pairs<C>(t, b, in, out, rocprim::counting_iterator<V>(0), vout, (size_t)n, 0u, bits,
-                                          ctx->stream);
-    });
-  };
-  if (n <= kFewSortEnd && n >= (bits <= 16 ? kFewSort16 : kFewSort))
-    sort(FewSortConfig{});
+// The sorted keys' numbers, or the values vin, into vout.
+static void sort_pairs(tribit_ctx* ctx, const uint32_t* in, uint32_t* out, uint32_t* order, uint64_t n, uint32_t bits) {
+  if (n <= kSmallSort)
+    k_sort_small<uint32_t, uint32_t><<<1, kSmallThreads, 0, ctx->stream>>>(in, out, nullptr, order, (uint32_t)n, bits);
   else
-    sort(Config{});
+    sort_ids_device(ctx, in, out, order, n, bits);
+}
+static void sort_pairs(tribit_ctx* ctx, const uint32_t* in, uint32_t* out, const uint64_t* vin, uint64_t* vout,
+                       uint64_t n, uint32_t bits) {
+  if (n <= kSmallSort)
+    k_sort_small<uint32_t, uint64_t><<<1, kSmallThreads, 0, ctx->stream>>>(in, out, vin, vout, (uint32_t)n, bits);
+  else
+    sort_records_device(ctx, in, out, vin, vout, n, bits);
 }
 
 struct InDegree {
@@ -797,6 +757,13 @@ __global__ void __launch_bounds__(kScanBlockThreads) k_scan_small(OutDegree f, I
     scan_block(g, n, sfx_ptr);
 }
 
+// out[0, n): the exclusive scan of in (every caller through one instance of the device-wide scan).
+static void scan_u32(tribit_ctx* ctx, const uint32_t* in, uint32_t* out, uint64_t n) {
+  with_temp(ctx, [&](void* t, size_t& b) {
+    return rocprim::exclusive_scan(t, b, in, out, 0u, (size_t)n, rocprim::plus<uint32_t>(), ctx->stream);
+  });
+}
+
 // row_ptr[n + 1], the exclusive scan of odeg[0, n], and, with sfx_ptr, that of the
 // in-degrees deg - odeg.
 static void scan_rows(tribit_ctx* ctx, const uint32_t* odeg, const uint32_t* deg, uint64_t n, uint32_t* row_ptr,
@@ -807,9 +774,7 @@ static void scan_rows(tribit_ctx* ctx, const uint32_t* odeg, const uint32_t* deg
                                                               row_ptr, sfx_ptr);
     return;
   }
-  with_temp(ctx, [&](void* t, size_t& b) {
-    return rocprim::exclusive_scan(t, b, odeg, row_ptr, 0u, (size_t)(n + 1), rocprim::plus<uint32_t>(), s);
-  });
+  scan_u32(ctx, odeg, row_ptr, n + 1);
   if (!sfx_ptr) return;
   const auto indeg = rocprim::make_transform_iterator(rocprim::counting_iterator<uint64_t>(0), InDegree{deg, odeg, n});
   with_temp(ctx, [&](void* t, size_t& b) {
@@ -822,9 +787,7 @@ static void sort_keys(tribit_ctx* ctx, const uint64_t* in, uint64_t* out, uint64
     if (nk) k_sort_small_keys<<<1, kSmallThreads, 0, ctx->stream>>>(in, out, (uint32_t)nk, end_bit);
     return;
   }
-  with_temp(ctx, [&](void* t, size_t& b) {
-    return rocprim::radix_sort_keys(t, b, in, out, (size_t)nk, 0u, end_bit, ctx->stream);
-  });
+  sort_keys_device(ctx, in, out, nk, end_bit);
 }
 
 // Where the labels of kSkewIds ids or more begin in their buffer (in ids): an
@@ -897,9 +860,7 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
         k_head_flags<<<grid_for(nkeys, kBlock), kBlock, 0, s>>>(sorted.p, nkeys, head.p);
       }
       k_fill_u32<<<1, 64, 0, s>>>(head.p + nkeys, 1, 0u);
-      with_temp(ctx, [&](void* t, size_t& b) {
-        return rocprim::exclusive_scan(t, b, head.p, pos.p, 0u, (size_t)(nkeys + 1), rocprim::plus<uint32_t>(), s);
-      });
+      scan_u32(ctx, head.p, pos.p, nkeys + 1);
       k_scatter_heads<<<grid_for(nkeys, kBlock), kBlock, 0, s>>>(sorted.p, nkeys, pos.p, uniq.p);
       uint32_t cnt = 0;
       TB_HIP(hipMemcpyAsync(&cnt, pos.p + nkeys, 4, hipMemcpyDeviceToHost, s));
@@ -910,9 +871,7 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
       m = cnt;
     } else {
       DevBuf<uint64_t> ucount(ctx, 1);
-      with_temp(ctx, [&](void* t, size_t& b) {
-        return rocprim::unique(t, b, sorted.p, uniq.p, ucount.p, (size_t)nkeys, rocprim::equal_to<uint64_t>(), s);
-      });
+      unique_device(ctx, sorted.p, uniq.p, ucount.p, nkeys);
       uint64_t h[2] = {0, 0};
       TB_HIP(hipMemcpyAsync(&h[0], ucount.p, 8, hipMemcpyDeviceToHost, s));
       ctx->sync();
@@ -984,10 +943,10 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
         // input ids with similar degrees (a block of a block model) stay runs
         DevBuf<uint32_t> cls(ctx, n);
         k_octave<<<grid_for(n, kBlock), kBlock, 0, s>>>(deg.p, n, cls.p);
-        sort_pairs<rocprim::default_config, uint32_t>(ctx, cls.p, deg_sorted.p, nullptr, labels.p, n, 6u);
+        sort_pairs(ctx, cls.p, deg_sorted.p, labels.p, n, 6u);
         k_gather_u32<<<grid_for(n, kBlock), kBlock, 0, s>>>(deg.p, labels.p, n, deg_sorted.p);
       } else {
-        sort_pairs<IdSortConfig, uint32_t>(ctx, deg.p, deg_sorted.p, nullptr, labels.p, n, bits_for(n));
+        sort_pairs(ctx, deg.p, deg_sorted.p, labels.p, n, bits_for(n));
       }
       std::swap(deg.p, deg_sorted.p);  // deg now indexed by internal id
     }
@@ -1067,7 +1026,7 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
           DevBuf<uint32_t> key(ctx, m), key_sorted(ctx, m);
           DevBuf<uint64_t> val(ctx, m), val_sorted(ctx, m);
           k_arc_pack<<<grid_for(m, kBlock), kBlock, 0, s>>>(uniq.p, m, pack, row_ptr.p, col.p, rsplit.p, key.p, val.p);
-          sort_pairs<IdSortConfig, uint64_t>(ctx, key.p, key_sorted.p, val.p, val_sorted.p, m, kb);
+          sort_pairs(ctx, key.p, key_sorted.p, val.p, val_sorted.p, m, kb);
           k_sfx_unpack<<<grid_for(m, kBlock * kUnpackSteps), kBlock, 0, s>>>(
               key_sorted.p, val_sorted.p, m, pack, rng_sfx.p, sfx_dh.p, sfx_split.p, w);
           filled = true;
@@ -1081,7 +1040,7 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
         uniq.reset();
         rsplit.reset();
         DevBuf<uint32_t> head(ctx, m), arc_sorted(ctx, m);
-        sort_pairs<IdSortConfig, uint32_t>(ctx, col.p, head.p, nullptr, arc_sorted.p, m, kb);
+        sort_pairs(ctx, col.p, head.p, arc_sorted.p, m, kb);
         k_sfx_fill<<<grid_for(m, kBlock), kBlock, 0, s>>>(head.p, arc_sorted.p, m, arec.p, rng_sfx.p, sfx_dh.p,
                                                           sfx_split.p, w);
       }
@@ -1151,12 +1110,8 @@ void build_layout(tribit_ctx* ctx, tribit_graph* g, int layout) {
   if (m) {
     DevBuf<uint32_t> fw_cnt(ctx, n + 1), rv_cnt(ctx, n + 1), rv_off(ctx, n + 1);
     k_dir_count<<<grid_for(n + 1, kBlock), kBlock, 0, s>>>(g->row_ptr, g->col, n, fw_cnt.p, rv_cnt.p, w_fw.p);
-    with_temp(ctx, [&](void* t, size_t& b) {
-      return rocprim::exclusive_scan(t, b, fw_cnt.p, fw_ptr.p, 0u, (size_t)(n + 1), rocprim::plus<uint32_t>(), s);
-    });
-    with_temp(ctx, [&](void* t, size_t& b) {
-      return rocprim::exclusive_scan(t, b, rv_cnt.p, rv_off.p, 0u, (size_t)(n + 1), rocprim::plus<uint32_t>(), s);
-    });
+    scan_u32(ctx, fw_cnt.p, fw_ptr.p, n + 1);
+    scan_u32(ctx, rv_cnt.p, rv_off.p, n + 1);
     TB_HIP(hipMemcpyAsync(&m_fwd, fw_ptr.p + n, 4, hipMemcpyDeviceToHost, s));
     ctx->sync();
     const uint64_t m_rev = m - m_fwd;
@@ -1171,9 +1126,7 @@ void build_layout(tribit_ctx* ctx, tribit_graph* g, int layout) {
                                                            pid_dir.p + m_fwd, rv_cnt.p,
                                                            reinterpret_cast<unsigned long long*>(w_rv.p));
     }
-    with_temp(ctx, [&](void* t, size_t& b) {
-      return rocprim::exclusive_scan(t, b, rv_cnt.p, rv_ptr.p, 0u, (size_t)(n + 1), rocprim::plus<uint32_t>(), s);
-    });
+    scan_u32(ctx, rv_cnt.p, rv_ptr.p, n + 1);
     k_add_u32<<<grid_for(n + 1, kBlock), kBlock, 0, s>>>(rv_ptr.p, n + 1, m_fwd);
   } else {
     k_fill_u32<<<grid_for(n + 1, kBlock), kBlock, 0, s>>>(fw_ptr.p, n + 1, 0u);
@@ -1272,9 +1225,7 @@ static uint64_t sort_unique(tribit_ctx* ctx, const uint64_t* in, uint64_t nk, ui
   DevBuf<uint32_t> head(ctx, nk + 1), pos(ctx, nk + 1);
   k_head_flags<<<grid_for(nk, kBlock), kBlock, 0, s>>>(sorted.p, nk, head.p);
   k_fill_u32<<<1, 64, 0, s>>>(head.p + nk, 1, 0u);
-  with_temp(ctx, [&](void* t, size_t& b) {
-    return rocprim::exclusive_scan(t, b, head.p, pos.p, 0u, (size_t)(nk + 1), rocprim::plus<uint32_t>(), s);
-  });
+  scan_u32(ctx, head.p, pos.p, nk + 1);
   k_scatter_heads<<<grid_for(nk, kBlock), kBlock, 0, s>>>(sorted.p, nk, pos.p, out);
   uint32_t cnt = 0, f = 0;
   TB_HIP(hipMemcpyAsync(&cnt, pos.p + nk, 4, hipMemcpyDeviceToHost, s));
@@ -1301,9 +1252,7 @@ void build_offdiag(tribit_ctx* ctx, const uint64_t* d_cols, uint64_t ncols, cons
     DevBuf<uint32_t> odeg(ctx, n + 1);
     k_fill_u32<<<grid_for(n + 1, kBlock), kBlock, 0, s>>>(odeg.p, n + 1, 0u);
     if (mh) k_csr_split<<<grid_for(mh, kBlock), kBlock, 0, s>>>(hk.p, mh, 32, col.p, nullptr, odeg.p);
-    with_temp(ctx, [&](void* t, size_t& b) {
-      return rocprim::exclusive_scan(t, b, odeg.p, row_ptr.p, 0u, (size_t)(n + 1), rocprim::plus<uint32_t>(), s);
-    });
+    scan_u32(ctx, odeg.p, row_ptr.p, n + 1);
   }
   hk.reset();
   // the cols edges, owner first, distinct, as streamed ranges of H rows grouped by owner
@@ -1326,9 +1275,7 @@ void build_offdiag(tribit_ctx* ctx, const uint64_t* d_cols, uint64_t ncols, cons
     DevBuf<uint32_t> head(ctx, ncols + 1), pos(ctx, ncols + 1);
     k_head_flags<<<grid_for(ncols, kBlock), kBlock, 0, s>>>(sorted.p, ncols, head.p);
     k_fill_u32<<<1, 64, 0, s>>>(head.p + ncols, 1, 0u);
-    with_temp(ctx, [&](void* t, size_t& b) {
-      return rocprim::exclusive_scan(t, b, head.p, pos.p, 0u, (size_t)(ncols + 1), rocprim::plus<uint32_t>(), s);
-    });
+    scan_u32(ctx, head.p, pos.p, ncols + 1);
     k_scatter_heads<<<grid_for(ncols, kBlock), kBlock, 0, s>>>(sorted.p, ncols, pos.p, ck.p);
     uint32_t cnt = 0;
     TB_HIP(hipMemcpyAsync(&cnt, pos.p + ncols, 4, hipMemcpyDeviceToHost, s));
@@ -1348,9 +1295,7 @@ void build_offdiag(tribit_ctx* ctx, const uint64_t* d_cols, uint64_t ncols, cons
     if (mc)
       k_rv_fill<<<grid_for(mc, kBlock), kBlock, 0, s>>>(ck.p, mc, row_ptr.p, rng.p, pid.p, rv_cnt.p,
                                                         reinterpret_cast<unsigned long long*>(w_rv.p));
-    with_temp(ctx, [&](void* t, size_t& b) {
-      return rocprim::exclusive_scan(t, b, rv_cnt.p, rv_ptr.p, 0u, (size_t)(n + 1), rocprim::plus<uint32_t>(), s);
-    });
+    scan_u32(ctx, rv_cnt.p, rv_ptr.p, n + 1);
   }
   ck.reset();
   // totals: streamed elements, owner rows
