@@ -271,6 +271,24 @@ def test_narrow_ranges(gpu_ctx):
                     assert g.count(sched="wedge", flags=fl, group_width=gw).triangles == want, (n, fl, gw)
 
 
+# single tasks of one launch: fewer than sub-queues, one over, about the first claims of
+# several units, and sub-queues that run dry amid one
+@pytest.mark.parametrize("hubs,each", [(1, 40), (65, 12), (64 * 33, 6), (64 * 66 + 1, 5), (64 * 150 - 1, 4), (120000, 3)])
+def test_task_feed(gpu_ctx, oracle_mod, hubs, each):
+    """Every task of a wave launch is taken once, however claims grow: `hubs` cliques of `each` ids, and a sparse rest."""
+    note(f"task feed: {hubs} cliques of {each} ids")
+    n = hubs * each + 1000
+    pairs = [(a, b) for a in range(each) for b in range(a + 1, each)]
+    base = np.arange(hubs, dtype=np.uint64) * each
+    keys = np.concatenate([graphs.pack(base + a, base + b) for a, b in pairs] + [graphs.random_graph(1000, 0.01, 5)])
+    want = oracle_mod.count_keys(keys, n)
+    with gpu_ctx.graph_from_keys(keys, n) as g:
+        for sched in scheds_of(g):
+            for fl in (0, tribit_amd.FORCE_MULTI):
+                res = g.count(sched, repeats=3, flags=fl)
+                assert res.triangles == want and res.repeats_agree, (sched, fl)
+
+
 def test_forced_multi_task_waves(gpu_ctx, oracle_mod):
     """Every launch of the 64-slot wave kernel as multi-task waves (the kernel large launches switch to),
     under every schedule, with cuckoo and with fallback sets."""

@@ -43,6 +43,12 @@ constexpr uint32_t kWaveBatch = 16;      // most wave tasks taken per queue atom
 // grid is full and all take the same.
 constexpr uint32_t kTasksPerWave = 2;
 constexpr uint32_t kClaimsPerWave = 8;   // queue claims per wave of a wave launch (when tasks allow)
+// A claim is at most the sub-queue's counter >> kClaimRamp: about 110 claims more a
+// sub-queue than whole ones from the start. Counts in ms with 2, 3, 5 and without:
+// R-MAT scale 22 4.23, 4.24, 4.08, 4.53, Chung-Lu of 5M ids 2.91, 2.74, 2.61, 3.30
+// (4, 6 and 7 as 5); uniform graphs the same with all (Erdos-Renyi 4M ids 2.72),
+// only 512,000 ids in blocks of 512 lose: 2.62, 2.62, 2.70, 2.60.
+constexpr uint32_t kClaimRamp = 5;
 constexpr uint32_t kChunk = 2048;        // probe-set chunk of class-3 rows
 constexpr uint64_t kWaveCap = 1u << 15;  // target streamed elements per wave task
 constexpr uint64_t kBlockCap = 1u << 18; // target streamed elements per block task
@@ -616,7 +622,12 @@ __device__ __forceinline__ uint32_t stream_tiles(const TileSrc& ts, const uint2*
 // Hands out the tasks of a wave launch to its waves in units of `unit`
 // consecutive tasks. The units are split over kQueues sub-queues (unit k goes
 // to sub-queue k % kQueues, in order: each sub-queue also starts with its
-// heaviest) and claimed `claim` units at a time; a block starts on sub-queue
+// heaviest) and claimed up to `claim` units at a time: one at first, more as the
+// sub-queue's counter rises (kClaimRamp), since the heaviest come first. Claims of
+// sixteen from the start kept waves on sixteen of the heaviest to the end of the
+// launch, all of one kind where hubs have about 64 tasks each, of rising weight
+// (R-MAT scale 24, outdeg <= 256: 3.4 ms with them, 2.3 with the ramp; every eighth
+// unit of a window to each of eight sub-queues 2.5). A block starts on sub-queue
 // blockIdx.x % kQueues. Claims on one address serialise (about 13 ns each on
 // MI355X): a full grid of 8,192 waves makes about 64K claims, 106 us of them on
 // each of eight sub-queues, 13 us on each of 64. When a wave's sub-queue runs
@@ -634,9 +645,8 @@ __device__ __forceinline__ uint32_t stream_tiles(const TileSrc& ts, const uint2*
 // out 18.6, runs 17.8). Workgroup b runs on XCD b % 8 and starts on sub-queue
 // b % kQueues, so each XCD streams the rows of its own graphs and its L2 is not
 // filled with the rows the other seven stream. For the same reason a wave passes
-// by a sub-queue whose own waves take what
-// is left in two claims: all waves claiming the launch's last units queued up on
-// their counters (48 and 64 graphs: 1.84 and 1.95 ms a replay, now 1.76 and 1.86;
+// by a sub-queue whose own waves take what is left in two claims: all waves
+// claiming the launch's last units queued up on their counters (48 and 64 graphs: 1.84 and 1.95 ms a replay, now 1.76 and 1.86;
 // with one claim left out 1.80 and 1.90, with four 1.91 and 1.85).
 struct TaskFeed {
   static_assert(kQueues == 64, "one lane per sub-queue");
@@ -646,12 +656,11 @@ struct TaskFeed {
   uint32_t home, q;   // the block's sub-queue, the current one
   uint32_t c, cend;   // claimed units: numbers in the launch (contiguous mode) or in sub-queue q
   uint64_t dry;       // sub-queues this wave's claims found empty: each is tried in vain once at most
-  uint32_t spare;     // what is left of a sub-queue to its own waves; each has some in a grid of kQueues blocks
+  uint32_t seen;      // where this wave last found sub-queue q
 
   __device__ TaskFeed(uint32_t* qs, uint32_t nt, uint32_t unit_, uint32_t claim_, bool contig_ = false)
       : queue(qs), ntasks(nt), unit(unit_), claim(claim_), contig(contig_), open(true), home(blockIdx.x % kQueues),
-        q(home), c(0), cend(0), dry(0),
-        spare(contig_ && gridDim.x >= kQueues ? 2 * (gridDim.x * (blockDim.x / 64) / kQueues) : 0u) {}
+        q(home), c(0), cend(0), dry(0), seen(0) {}
 
   __device__ uint32_t eighth(uint32_t x) const { return (uint32_t)((uint64_t)((ntasks + unit - 1) / unit) * x / 8); }
 
@@ -676,15 +685,19 @@ struct TaskFeed {
         // lane p: the p-th sub-queue to try, the eight of the block's XCD first
         const uint32_t sq = ((home + (lane >> 3)) & 7) + 8 * (((home >> 3) + lane) & 7);
         const uint32_t v = __hip_atomic_load(queue + sq * kQStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // what is left of a sub-queue to its own waves (in a grid of kQueues blocks each has some)
+        const uint32_t spare = contig && gridDim.x >= kQueues ? 2 * (gridDim.x * (blockDim.x / 64) / kQueues) : 0u;
         const uint64_t left = __ballot(v + spare < size_of(sq) && !((dry >> sq) & 1ull));
         if (!left) return false;  // counters only grow: nothing is left later either
         q = __builtin_amdgcn_readlane(sq, __ffsll((long long)left) - 1);
+        seen = __builtin_amdgcn_readlane(v, __ffsll((long long)left) - 1);
       }
-      const uint32_t nq = size_of(q), by = contig ? 1u : claim;
+      const uint32_t nq = size_of(q), by = contig ? 1u : min(claim, max(1u, seen >> kClaimRamp));
       uint32_t v = 0;
       if (lane == 0) v = atomicAdd(queue + q * kQStride, by);
       v = __builtin_amdgcn_readfirstlane(v);  // every member stays in scalar registers
       open = v < nq;
+      seen = v + by;
       if (!open) {
         dry |= 1ull << q;
       } else if (contig) {
@@ -693,7 +706,7 @@ struct TaskFeed {
         cend = min(c + claim, eighth((q & 7) + 1));
       } else {
         c = v;
-        cend = min(v + claim, nq);
+        cend = min(v + by, nq);
       }
     }
   }
