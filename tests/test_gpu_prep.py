@@ -1,4 +1,8 @@
 """GPU parity of the generator, preprocessing and core-matrix kernels at the sizes where they change path."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -417,3 +421,20 @@ def test_keys_that_the_caller_allocated(gpu_ctx, oracle_mod):
         assert other.lib.tribit_gen_rmat(other.h, 12, 8, 0.57, 0.19, 0.19, 4, ctypes.byref(again), ctypes.byref(n)) == 0
         assert again.value == d.value  # the block was free again
         other.lib.tribit_free_device_keys(other.h, again)
+
+
+def test_preprocessing_time_without_code_loading():
+    """A process's first graph reports the time of its preprocessing, not of the sorts' code being loaded (5 ms a file)."""
+    note("times of a process's first graph")
+    code = ("import tribit_amd as tb\n"
+            "ctx = tb.Context(0)\n"
+            "for seed in (1, 2):\n"
+            "    with ctx.gen_rmat(16, 16, seed=seed) as g:\n"
+            "        g.count('directed')\n"
+            "        i = g.info()\n"
+            "        print(i['ms_preprocess'], i['ms_layout'][2], flush=True)\n")
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100,
+                         cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert out.returncode == 0, out.stderr
+    first, second = (np.array(line.split(), float) for line in out.stdout.splitlines())
+    assert (first < second + 4.0).all(), (first, second)

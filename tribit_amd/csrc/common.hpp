@@ -84,6 +84,7 @@ struct tribit_ctx {
   // copies into pageable memory go through a staging buffer and wait
   void* readback = nullptr;
   static constexpr size_t kReadback = 4096;
+  uint32_t loaded = 0;  // the files whose device code load_code has loaded
   std::string last_error;
 
   // kept: the buffer outlives the call that takes it (a graph's, a batch's, a model's)
@@ -321,6 +322,18 @@ void sort_records_device(tribit_ctx* ctx, const uint32_t* in, uint32_t* out, con
                          uint64_t n, uint32_t bits);
 void sort_keys_device(tribit_ctx* ctx, const uint64_t* in, uint64_t* out, uint64_t n, uint32_t end_bit);
 void unique_device(tribit_ctx* ctx, const uint64_t* in, uint64_t* out, uint64_t* count, uint64_t n);
+// Loads a file's device code (5 ms, once a process), for callers about to time what
+// it does: the events around a kernel span its loading too. Asked once a context.
+inline void load_code(tribit_ctx* ctx, uint32_t file, const void* kernel) {
+  if (ctx->loaded & file) return;
+  hipFuncAttributes a;
+  TB_HIP(hipFuncGetAttributes(&a, kernel));
+  ctx->loaded |= file;
+}
+enum : uint32_t { kSortIdsFile = 1, kSortRecordsFile = 2, kSortKeysFile = 4, kRowsFile = 8 };
+void load_sort_ids(tribit_ctx* ctx);
+void load_sort_records(tribit_ctx* ctx);
+void load_sort_keys(tribit_ctx* ctx);
 // partition.hip
 bool distinct_keys(tribit_ctx* ctx, const uint64_t* d_keys, uint64_t nk, uint64_t n, uint32_t kb, uint64_t* out,
                    uint64_t* m, bool* bad, uint64_t band_ids, uint64_t* band);
@@ -329,6 +342,7 @@ void count_degrees(tribit_ctx* ctx, const uint64_t* keys, uint64_t m, uint64_t n
 constexpr uint64_t kRowsMaxEdges = 1ull << 29;  // build_rows takes fewer edges than this
 void build_rows(tribit_ctx* ctx, const uint64_t* edges, uint64_t m, const uint32_t* lab, const uint32_t* deg, uint64_t n,
                 uint32_t kb, uint64_t* arcs, uint32_t* col, uint16_t* col16, uint32_t* odeg, uint32_t* flag);
+void load_rows(tribit_ctx* ctx);
 // gen.hip
 uint64_t chung_lu_samples(uint64_t n, double avg_deg);
 void chung_lu_cdf(uint64_t n, double gamma, uint64_t* cdf);

@@ -809,6 +809,16 @@ void preprocess(tribit_ctx* ctx, uint64_t* d_keys_in, uint64_t nkeys, uint64_t n
   g->ctx = ctx;
   g->n = n;
   g->entries = nkeys;
+  // the code that a graph of this size comes to, unless a partition overflows
+  if (relabel_opt && n > kSmallSort) load_sort_ids(ctx);
+  if (nkeys > kSmallSort) {
+    if (relabel_opt) {
+      load_rows(ctx);
+      load_sort_records(ctx);
+    } else {
+      load_sort_keys(ctx);
+    }
+  }
   TB_HIP(hipEventRecord(ctx->ev[0], s));
 
   // keys checked and packed to (min << kb) | max for the sort
@@ -1158,6 +1168,7 @@ void ensure_layout(tribit_ctx* ctx, tribit_graph* g, int layout) {
   hipEvent_t a = nullptr, b = nullptr;
   TB_HIP(hipEventCreate(&a));
   TB_HIP(hipEventCreate(&b));
+  if (layout == TRIBIT_SCHED_DIRECTED && g->m > kSmallSort) load_sort_keys(ctx);
   TB_HIP(hipEventRecord(a, s));
   build_layout(ctx, g, layout);
   TB_HIP(hipEventRecord(b, s));

@@ -395,6 +395,8 @@ static void scan_to(tribit_ctx* ctx, F f, uint64_t n, uint32_t* out) {
   TB_HIP(rocprim::exclusive_scan(tmp.p, bytes, it, out, 0u, (size_t)(n + 1), rocprim::plus<uint32_t>(), s));
 }
 
+void load_rows(tribit_ctx* ctx) { load_code(ctx, kRowsFile, reinterpret_cast<const void*>(k_row_sort)); }
+
 // The arcs of a relabelled graph sorted by (u, v): packed into arcs[m] (whose
 // memory may hold the edges: they are read before), col, col16 (or null) and the
 // rows' lengths odeg (zeroed before). Every allocation comes before the first write

@@ -5,6 +5,9 @@
 
 namespace tb {
 
+static __global__ void k_ids_loaded() {}
+void load_sort_ids(tribit_ctx* ctx) { load_code(ctx, kSortIdsFile, reinterpret_cast<const void*>(k_ids_loaded)); }
+
 // order: the numbers of the items in the stable order of their keys' low `bits`
 // bits. Keys of one 8-bit digit (octave classes) keep rocPRIM's own digits.
 void sort_ids_device(tribit_ctx* ctx, const uint32_t* in, uint32_t* out, uint32_t* order, uint64_t n, uint32_t bits) {

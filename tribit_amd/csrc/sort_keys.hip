@@ -6,6 +6,9 @@
 
 namespace tb {
 
+static __global__ void k_keys_loaded() {}
+void load_sort_keys(tribit_ctx* ctx) { load_code(ctx, kSortKeysFile, reinterpret_cast<const void*>(k_keys_loaded)); }
+
 void sort_keys_device(tribit_ctx* ctx, const uint64_t* in, uint64_t* out, uint64_t n, uint32_t end_bit) {
   with_temp(ctx, [&](void* t, size_t& b) {
     return rocprim::radix_sort_keys(t, b, in, out, (size_t)n, 0u, end_bit, ctx->stream);

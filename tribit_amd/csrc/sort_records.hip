@@ -3,6 +3,11 @@
 
 namespace tb {
 
+static __global__ void k_records_loaded() {}
+void load_sort_records(tribit_ctx* ctx) {
+  load_code(ctx, kSortRecordsFile, reinterpret_cast<const void*>(k_records_loaded));
+}
+
 void sort_records_device(tribit_ctx* ctx, const uint32_t* in, uint32_t* out, const uint64_t* vin, uint64_t* vout,
                          uint64_t n, uint32_t bits) {
   with_sort_config<IdSortConfig>(n, bits, [&](auto config) {
