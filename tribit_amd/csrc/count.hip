@@ -46,8 +46,8 @@ constexpr uint32_t kClaimsPerWave = 8;   // queue claims per wave of a wave laun
 // A claim is at most the sub-queue's counter >> kClaimRamp: about 110 claims more a
 // sub-queue than whole ones from the start. Counts in ms with 2, 3, 5 and without:
 // R-MAT scale 22 4.23, 4.24, 4.08, 4.53, Chung-Lu of 5M ids 2.91, 2.74, 2.61, 3.30
-// (4, 6 and 7 as 5); uniform graphs the same with all (Erdos-Renyi 4M ids 2.72),
-// only 512,000 ids in blocks of 512 lose: 2.62, 2.62, 2.70, 2.60.
+// (4, 6 and 7 as 5); Erdos-Renyi graphs the same with all (4M ids 2.72),
+// equal blocks lose: 512,000 ids in blocks of 512 2.62, 2.62, 2.70, 2.60.
 constexpr uint32_t kClaimRamp = 5;
 constexpr uint32_t kChunk = 2048;        // probe-set chunk of class-3 rows
 constexpr uint64_t kWaveCap = 1u << 15;  // target streamed elements per wave task
